@@ -329,6 +329,16 @@ int tt_gmm_fp8_dgrad(const void* dy, const uint8_t* qw, const void* scale, int s
                      int64_t m, int64_t k, int64_t n, int32_t num_experts,
                      const int64_t* counts, void* dx, void* stream);
 
+/* Blockwise FP8 quantisation: bf16 weights w [num_experts, rows, cols] (rows
+ * and cols multiples of 128) to e4m3 codes q of the same shape and one scale
+ * per 128 x 128 block, scale [num_experts, rows/128, cols/128] (bf16 or f32):
+ * scale = amax / 448 (1 where amax is 0 or NaN) rounded to its dtype,
+ * q = e4m3(clamp(f32(w) / f32(scale), -448, 448)), NaN staying NaN. The
+ * inverse of the rule of scripts/dequant/bailing.py:57-102. */
+int tt_fp8_quantize_blocks(const void* w, int dtype, int64_t num_experts, int64_t rows,
+                           int64_t cols, uint8_t* q, void* scale, int scale_dtype,
+                           void* stream);
+
 #ifdef __cplusplus
 }
 #endif

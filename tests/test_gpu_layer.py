@@ -286,3 +286,49 @@ def test_full_layer_forward_with_fused_router_matches_cpu(process_ops, monkeypat
         assert_bf16_close(a, b, what=name)
     for key in ("aux_loss", "z_loss"):
         torch.testing.assert_close(got[6][key], ref[6][key], rtol=1e-4, atol=0)
+
+
+@pytest.mark.parametrize("scale_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hidden,ffn", [(128, 128), (384, 256)])
+def test_fp8_requantize_equals_torch_composition(process_ops, scale_dtype, hidden, ffn):
+    """The one-pass kernel gives the codes and scales of the torch composition it
+    replaces, byte for byte: ordinary blocks, exact ties, blocks of zeros, tiny
+    and huge scales (the dividing path), signed zeros, infinities and NaN."""
+    process_ops(CudaRuntime(), OpPolicy.CUSTOM)
+    E = 5
+    cfg = MoEConfig(hidden_size=hidden, num_moe_experts=E, moe_ffn_hidden_size=ffn,
+                    gated_linear_unit=True, activation_func=F.silu, params_dtype=torch.bfloat16)
+    mlp = Fp8GroupedMLP(E, False, cfg).to(DEV)
+    mlp.s1, mlp.s2 = mlp.s1.to(scale_dtype), mlp.s2.to(scale_dtype)
+    g = torch.Generator().manual_seed(hidden)
+    for m in (mlp.master1, mlp.master2):
+        w = torch.randn(m.shape, generator=g) * 0.02
+        w[1, :128, :128] = torch.randint(-1792, 1793, (128, 128), generator=g) / 4.0
+        w[1, 0, 0] = 448.0  # scale 1: quarter steps tie between codes
+        w[2, :128, :128] = 0.0
+        w[2, :4, :7] = -0.0
+        w[2, -1, :5] = -0.0
+        w[3, :128, :128] *= 1e-37
+        w[3, -128:, -128:] *= 1e38
+        w[4, 3, 5] = float("inf")
+        w[4, 9, 2] = float("-inf")
+        w[4, -3, -5] = float("nan")
+        with torch.no_grad():
+            m.copy_(w.bfloat16())
+    want = []
+    for master, s in ((mlp.master1, mlp.s1), (mlp.master2, mlp.s2)):
+        n, R, C = master.shape
+        w = master.detach().float()
+        blocks = w.view(n, R // 128, 128, C // 128, 128).abs().amax(dim=(2, 4))
+        scale = torch.where(blocks > 0, blocks / 448.0, torch.ones_like(blocks)).to(s.dtype)
+        full = scale.float().repeat_interleave(128, 1).repeat_interleave(128, 2)
+        want += [(w / full).clamp(-448.0, 448.0).to(torch.float8_e4m3fn), scale]
+    versions = [b._version for b in (mlp.q1, mlp.s1, mlp.q2, mlp.s2)]
+    mlp.requantize()
+    for got, ref, v in zip((mlp.q1, mlp.s1, mlp.q2, mlp.s2), want, versions):
+        nan = ref.float().isnan()
+        assert torch.equal(got.float().isnan(), nan)
+        bits = torch.uint8 if ref.dtype == torch.float8_e4m3fn else (
+            torch.int16 if ref.dtype == torch.bfloat16 else torch.int32)
+        assert torch.equal(got.view(bits)[~nan], ref.view(bits)[~nan])
+        assert got._version > v  # a backward that saved the old values is refused

@@ -3,7 +3,7 @@
 from .base import OpImpl, OpImplKind, OpPolicy, OpSpec
 from .dispatcher import OpDispatcher
 from .moe import MoEPermutation, get_expert_indices
-from .ops import get_ops, get_or_create_ops, ops, reset_ops
+from .ops import get_ops, get_or_create_ops, op_resolves, ops, reset_ops
 from .providers import add_provider_package, iter_provider_modules, remove_provider_package
 from .registry import OpRegistry, register_op, registry
 
@@ -20,6 +20,7 @@ __all__ = [
     "get_ops",
     "get_or_create_ops",
     "iter_provider_modules",
+    "op_resolves",
     "ops",
     "register_op",
     "registry",

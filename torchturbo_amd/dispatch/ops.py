@@ -60,6 +60,15 @@ def get_ops() -> OpDispatcher:
     return _OPS
 
 
+def op_resolves(name: str) -> bool:
+    """Whether the process dispatcher has an implementation of ``name`` for its device."""
+    try:
+        d = get_ops()
+    except RuntimeError:
+        return False
+    return bool(d.registry.list(lambda s: s.op_name == name)) and name not in d.unresolved_ops
+
+
 def reset_ops() -> None:
     """Forget the process dispatcher (tests and benchmarks switch devices)."""
     global _OPS
@@ -78,4 +87,4 @@ class _OpsProxy:
 
 ops = _OpsProxy()
 
-__all__ = ["get_or_create_ops", "get_ops", "ops", "reset_ops"]
+__all__ = ["get_or_create_ops", "get_ops", "op_resolves", "ops", "reset_ops"]

@@ -27,7 +27,7 @@ import torch
 import torch.nn.functional as F
 from torch.nn.parameter import Parameter
 
-from ..dispatch import ops
+from ..dispatch import op_resolves, ops
 from .moe_config import MoEConfig
 
 
@@ -142,6 +142,9 @@ class Fp8GroupedMLP(torch.nn.Module):
             raise RuntimeError("no master weights to quantize")
         with torch.no_grad():
             for master, q, s in ((self.master1, self.q1, self.s1), (self.master2, self.q2, self.s2)):
+                if (master.is_cuda and op_resolves("quantize_fp8_blocks")
+                        and ops.quantize_fp8_blocks(master, q, s)):
+                    continue
                 E, R, C = master.shape
                 blocks = master.float().view(E, R // 128, 128, C // 128, 128).abs().amax(dim=(2, 4))
                 scale = torch.where(blocks > 0, blocks / 448.0, torch.ones_like(blocks)).to(s.dtype)

@@ -29,24 +29,13 @@ from typing import Optional
 import torch
 import torch.distributed as dist
 
-from ..dispatch import ops
+from ..dispatch import op_resolves, ops
 from .moe_config import MoEConfig
 
 # Sizes the HIP router kernels cover (tt_router_topk_fwd / _bwd,
 # tt_router_loss_fwd: E <= 1024, k <= 64).
 MAX_EXPERTS = 1024
 MAX_TOPK = 64
-
-
-def _op_resolves(name: str) -> bool:
-    """Whether the process dispatcher has an implementation of ``name`` for its device."""
-    from ..dispatch.ops import get_ops
-
-    try:
-        d = get_ops()
-    except RuntimeError:
-        return False
-    return bool(d.registry.list(lambda s: s.op_name == name)) and name not in d.unresolved_ops
 
 
 def _group_size(group) -> int:
@@ -313,7 +302,7 @@ class TopKRouter(Router):
                 and self.weight.dtype == input.dtype
                 and self.router_dtype(input.dtype) in (input.dtype, torch.float32)
                 and E % 32 == 0 and 32 <= E <= 256 and input.shape[-1] % 64 == 0
-                and _op_resolves("router_gate_topk"))
+                and op_resolves("router_gate_topk"))
 
     def forward(self, input, input_ids=None, padding_mask=None,
                 accumulate_tokens_per_expert: bool = True):
