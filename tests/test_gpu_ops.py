@@ -1060,6 +1060,50 @@ def test_grouped_matmul_thin_experts_exact(trans_b, E, K, N):
             s0 += c
 
 
+# Launches of at most 96 rows per expert on average: 64-row tiles up to 40 rows, 128-row
+# tiles above. Row counts on both sides of a 32-row block and of a tile, one expert far above
+# the average (several row tiles over the same weights), widths on both sides of a 128-column
+# tile, reductions of one k-tile, of the stage ring's depth and with tails.
+FEW_ROWS = [
+    ([0, 1, 31, 32, 33, 63, 64, 65, 0, 2], 64, 128),
+    ([1], 8, 8),
+    ([200, 0, 0, 3, 0, 0, 1, 0], 200, 136),
+    ([0] * 130 + [5] + [0] * 169 + [1, 2], 128, 1000),  # more experts than threads
+    ([96, 127, 128, 129, 0, 1, 64], 192, 264),
+    ([300, 30, 0, 33, 65, 97], 72, 120),
+    ([96] * 5, 2048, 24),
+]
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,K,N", FEW_ROWS, ids=[f"E{len(c)}K{k}N{n}" for c, k, n in FEW_ROWS])
+def test_grouped_matmul_few_rows_exact(counts, K, N, dtype, trans_b):
+    """Small-integer operands (exact sums) into NaN-filled outputs with a guard row."""
+    from torchturbo_amd import _lib
+
+    g = torch.Generator().manual_seed(K + N)
+    E, M = len(counts), sum(counts)
+    x = torch.randint(-2, 3, (M, K), generator=g).to(dtype).to(DEV)
+    dy = torch.randint(-2, 3, (M, N), generator=g).to(dtype).to(DEV)
+    w = torch.randint(-2, 3, (E, N, K) if trans_b else (E, K, N), generator=g).to(dtype).to(DEV)
+    cnt = torch.tensor(counts, dtype=torch.int64, device=DEV)
+    args = (_lib.dtype_code(dtype), M, K, N, E, int(trans_b), _lib.ptr(cnt))
+    y = torch.full((M + 1, N), float("nan"), dtype=dtype, device=DEV)
+    dx = torch.full((M + 1, K), float("nan"), dtype=dtype, device=DEV)
+    _lib.call("tt_gmm_fwd", _lib.ptr(x), _lib.ptr(w), *args, _lib.ptr(y), _lib.stream())
+    _lib.call("tt_gmm_dgrad", _lib.ptr(dy), _lib.ptr(w), *args, _lib.ptr(dx), _lib.stream())
+    torch.cuda.synchronize()
+    assert y[M].isnan().all() and dx[M].isnan().all()
+    s0 = 0
+    for e, c in enumerate(counts):
+        we = (w[e].t() if trans_b else w[e]).double().cpu()  # [K, N]
+        xe, de = x[s0:s0 + c].double().cpu(), dy[s0:s0 + c].double().cpu()
+        assert torch.equal(y[s0:s0 + c].cpu(), (xe @ we).to(dtype)), (e, c)
+        assert torch.equal(dx[s0:s0 + c].cpu(), (de @ we.t()).to(dtype)), (e, c)
+        s0 += c
+
+
 # more 256x256 output tiles than the GPU has compute units, so every persistent block
 # walks many tiles (tile switch, cross-tile prefetch, XCD remap); mean expert loads above
 # 512 rows take the four-stage weight-gradient kernel, at most 512 the persistent

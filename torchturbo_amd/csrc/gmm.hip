@@ -45,7 +45,8 @@
 //   row. fwd/dgrad tiles of at most 64 rows leave that stream for a
 //   weight-streaming pipeline of their own (two weight k-tiles in flight
 //   while a third is multiplied), and an expert of at most 64 rows takes its
-//   tiles two per schedule slot.
+//   tiles two per schedule slot. Launches of few rows per expert on average
+//   (thin_rows) run on gmm_thin.hip instead.
 // * gmm_q8_kernel (fwd/dgrad with e4m3 weights and 128x128 block scales,
 //   every launch whose reduction is longer than one 64-deep k-tile):
 //   persistent like gmm_p64_kernel, 128x512x64 tiles (the four waves share
@@ -75,44 +76,12 @@
 // (one-tile-per-block kernel, whose blocks read the launch's ranking from
 // wgrad_rank_kernel) or to every XCD as rectangles (persistent kernel), so
 // that the XCDs share its activation panels in L2.
-#include "common.h"
+#include "gemm.h"
 
 #include <atomic>
 #include <type_traits>
 
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) short i16x4;
-typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-typedef __attribute__((address_space(3))) char lds_char;
-
-enum { MODE_FWD = 0, MODE_DGRAD = 1, MODE_WGRAD = 2 };
-
-template <int ET>
-struct Mma;
-template <>
-struct Mma<TT_BF16> {
-  static __device__ __forceinline__ f32x16 run(const uint4& a, const uint4& b, const f32x16& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <>
-struct Mma<TT_F16> {
-  static __device__ __forceinline__ f32x16 run(const uint4& a, const uint4& b, const f32x16& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
-
-__device__ __forceinline__ int xcd_remap(int b, int nb) {
-  const int q = nb / 8, r = nb % 8;
-  const int xcd = b % 8, pos = b / 8;
-  return xcd < r ? xcd * (q + 1) + pos : r * (q + 1) + (xcd - r) * q + pos;
-}
 
 // Block-wide exclusive scans over the E expert counts: row starts and
 // m-tile starts. Writes E + 1 entries of each into LDS.
@@ -197,13 +166,6 @@ struct TileDesc {
   int e;
   int nsub;  // persistent fwd / dgrad: thin tiles in this slot (0: one ordinary tile)
 };
-
-// A block-uniform 64-bit value (read from LDS) into scalar registers.
-__device__ __forceinline__ int64_t rfl64(int64_t v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
 
 // Weight-gradient tiles of one block per tile (gmm_mfma_kernel): each
 // expert's output tiles go to one pair of XCDs, half of its tile grid to
@@ -412,91 +374,12 @@ __device__ bool describe_tile(const char* p0, const char* p1, char* out, int64_t
   return true;
 }
 
-// Operand layouts per mode: A is K-major except in wgrad; B is K-major for
-// fwd with trans_b and dgrad without.
-template <int MODE, bool TRANS_B>
-struct Layout {
-  static constexpr bool A_K = MODE != MODE_WGRAD;
-  static constexpr bool B_K = (MODE == MODE_FWD) ? TRANS_B : (MODE == MODE_DGRAD ? !TRANS_B : false);
-};
-
 // ===========================================================================
 // MFMA kernel (bf16 / f16): 256x256x32 block tiles, 4 waves of 128x128.
 // ===========================================================================
 constexpr int DM_BM = 256, DM_BN = 256, DM_BK = 32, DM_ST = 4, DM_NT = 256;
 constexpr int DM_TILE = DM_BM * DM_BK * 2;  // bytes of one operand tile (16 KiB)
 constexpr int DM_STAGE = 2 * DM_TILE;       // A tile then B tile
-constexpr uint32_t DM_OOB = 0xFFFFFFF0u;    // buffer offset past any resource
-// Gathered A rows: the offset of a row past an expert's end, past any gathered
-// source (sources are smaller than 2 GiB) with room for the chunk and k-tile
-// offsets added to it.
-constexpr uint32_t GA_NOROW = 0x80000000u;
-
-typedef __attribute__((ext_vector_type(4))) int i32x4;
-typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
-typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
-
-// Buffer resource over [base, base + bytes): offsets at or past `bytes` read
-// as zeros. Word 3 is the raw 32-bit data format of the gfx9 family.
-__device__ __forceinline__ i32x4 make_rsrc(const void* base, int64_t bytes) {
-  const uint64_t b = reinterpret_cast<uint64_t>(base);
-  const uint32_t n = bytes <= 0 ? 0u : (bytes < (int64_t)DM_OOB ? (uint32_t)bytes : DM_OOB);
-  i32x4 r;
-  r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  r.y = __builtin_amdgcn_readfirstlane((int)((uint32_t)(b >> 32) & 0xFFFFu));
-  r.z = __builtin_amdgcn_readfirstlane((int)n);
-  r.w = 0x00020000;
-  return r;
-}
-
-// One 16-byte buffer load per lane straight into LDS at lds_addr + 16 * lane
-// (lds_addr is wave-uniform and goes to M0). Inline assembly, so that the
-// compiler does not drain outstanding loads before every LDS read:
-// completion of a stage is awaited explicitly (TT_WAIT_VMCNT) before the
-// barrier that publishes it. Nothing else in these kernels uses M0.
-// The resource moved `adv` bytes along (scalar arithmetic): an offset from
-// the new base is in range exactly when the same offset plus adv was before,
-// and nothing is once adv passes the end.
-__device__ __forceinline__ i32x4 advance_rsrc(i32x4 r, uint32_t adv) {
-  const uint64_t b = (((uint64_t)(uint32_t)r.y << 32) | (uint32_t)r.x) + adv;  // stride 0
-  i32x4 o;
-  o.x = (int)(uint32_t)b;
-  o.y = (int)(uint32_t)(b >> 32);
-  // records - adv, or 0 on a borrow (SCC), in scalar instructions: the
-  // compiler's saturating subtract is a vector one.
-  uint32_t n;
-  asm("s_sub_u32 %0, %1, %2\n\ts_cselect_b32 %0, 0, %0" : "=s"(n) : "s"(r.z), "s"(adv) : "scc");
-  o.z = (int)n;
-  o.w = r.w;
-  return o;
-}
-
-__device__ __forceinline__ void dma16(uint32_t voff, i32x4 rsrc, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :
-               : "s"(lds_addr), "v"(voff), "s"(rsrc)
-               : "memory");
-}
-
-// One dword per lane into LDS at m0 + 4 lane (row indices of a gathered operand).
-__device__ __forceinline__ void dma4(uint32_t voff, i32x4 rsrc, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-               :
-               : "s"(lds_addr), "v"(voff), "s"(rsrc)
-               : "memory");
-}
-
-__device__ __forceinline__ uint32_t lds_addr_of(lds_char* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p));
-}
-
-// s_waitcnt with only vmcnt = n (gfx9 encoding: vmcnt[3:0] | vmcnt[5:4] << 14,
-// expcnt and lgkmcnt left at their maxima).
-#define TT_WAIT_VMCNT(n) \
-  __builtin_amdgcn_s_waitcnt(((n) & 0xF) | ((((n) >> 4) & 3) << 14) | (0x7 << 4) | (0xF << 8))
-
 // LDS operand tiles.
 // * K-major (k contiguous in memory): LDS row r (64 bytes = 32 k) holds tile
 //   row r, its 16-byte chunk c in slot c ^ ((r >> 2) & 3). An MFMA operand
@@ -527,28 +410,11 @@ __device__ __forceinline__ uint32_t fragmn_base(int c0, int lane) {
   return (uint32_t)(kr * 512 + (((col >> 3) ^ (4 * (kr & 3))) << 4) + (col & 7) * 2);
 }
 
-__device__ __forceinline__ uint4 read_k(lds_char* tile, uint32_t off) {
-  return __builtin_bit_cast(uint4, *reinterpret_cast<const lds_u32x4*>(tile + off));
-}
 __device__ __forceinline__ uint4 read_mn(lds_char* tile, uint32_t off) {
   const i16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(tile + off));
   const i16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(tile + off + 2048));
   const uint2 w0 = __builtin_bit_cast(uint2, v0), w1 = __builtin_bit_cast(uint2, v1);
   return uint4{w0.x, w0.y, w1.x, w1.y};
-}
-
-// Four fp32 values -> four 16-bit values (hardware round to nearest even).
-template <int ET>
-__device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
-  if constexpr (ET == TT_BF16) {
-    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-    const bf16x2 lo = {(__bf16)a, (__bf16)b}, hi = {(__bf16)c, (__bf16)d};
-    return uint2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
-  } else {
-    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-    const f16x2 lo = {(_Float16)a, (_Float16)b}, hi = {(_Float16)c, (_Float16)d};
-    return uint2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
-  }
 }
 
 // Epilogue through LDS. The accumulators hold C^T blocks (the MFMA operands
@@ -920,12 +786,6 @@ __global__ __launch_bounds__(DM_NT) void gmm_mfma_kernel(const char* __restrict_
   store_wave_tile<ET>(acc, t, t.i0 + wm * WT, t.j0 + wn * WT, lane, region);
 }
 
-// Barrier that also publishes this wave's LDS stores and retires its LDS
-// reads: wait for them, then s_barrier; the memory clobber keeps the
-// compiler from moving LDS accesses across it. Loads in flight (vmcnt) are
-// not waited for.
-#define TT_LDS_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
-
 // Output tile L (fwd / dgrad) from the schedule in LDS.
 template <int MODE, bool TRANS_B, int ESZ>
 __device__ __forceinline__ void tile_at(int L, const char* p0, const char* p1, char* out,
@@ -997,18 +857,6 @@ constexpr int P_EPI = 4096;             // epilogue staging per wave
 constexpr int64_t P_WGRAD_ROWS = 512;
 // ... or experts of at least this many 256x256 output tiles.
 constexpr int P_WGRAD_TILES = 512;
-
-// K-major 64-deep tile: LDS row r (128 bytes) holds tile row r, its 16-byte
-// chunk c in slot c ^ ((r >> 1) & 7): any 16 consecutive rows then cover the
-// 16 distinct 16-byte bank groups of a 256-byte bank line, so a fragment
-// read (one chunk of 32 rows per half-wave) is free of bank conflicts.
-// Fragment for k-step s (0..3): rows r0 + lane % 32, chunk 2 s + lane / 32;
-// further 32-row blocks add 4096.
-__device__ __forceinline__ uint32_t fragk64(int r0, int s, int lane) {
-  const int r = r0 + (lane & 31);
-  const int c = 2 * s + (lane >> 5);
-  return (uint32_t)(r * 128 + ((c ^ ((r >> 1) & 7)) << 4));
-}
 
 // Epilogue of the 64-deep kernel: the wave's 128x128 tile in 8 rounds of
 // 32 rows x 64 columns through its private 4 KiB of LDS (row r at 128 r,
@@ -2751,6 +2599,17 @@ int launch_p64_k(const void* p0, const void* p1, void* out, int64_t M, int64_t K
   return tt_check_launch("gmm");
 }
 
+// fwd / dgrad with at most this many rows per expert on average run on the
+// kernel of gmm_thin.hip (its loads run up to a k-tile past the reduction end,
+// in 32-bit offsets). Measured, persistent / thin: Qwen3-30B-A3B's fc1 fwd,
+// fc2 fwd, fc1 dgrad, fc2 dgrad at 62 rows per expert 188 + 97 + 181 + 135 /
+// 164 + 90 + 171 + 107 us, at 80 179 + 101 + 193 + 129 / 165 + 94 + 177 + 108,
+// at 96 176 + 97 + 184 + 127 / 168 + 96 + 181 + 110, at 128 188 + 112 + 197 +
+// 140 / 218 + 118 + 224 + 129; 64 experts of 1024 x 1408 at 94 rows 60 + 29 +
+// 54 + 37 / 50 + 24 + 39 + 26 us, at 144 66 + 31 + 52 + 35 / 63 + 35 + 60 + 41.
+constexpr int64_t THIN_ROWS = 96;
+bool thin_rows(int64_t M, int E) { return M <= (int64_t)E * THIN_ROWS; }
+
 template <int MODE, bool TB, int ET>
 int launch_mfma(const void* p0, const void* p1, void* out, int64_t M, int64_t K, int64_t N,
                 int E, const int64_t* counts, hipStream_t s) {
@@ -2770,6 +2629,8 @@ int launch_mfma(const void* p0, const void* p1, void* out, int64_t M, int64_t K,
   const int64_t R = MODE == MODE_FWD ? K : N;  // reduction length of fwd / dgrad
   const bool p64_lds = p64_lds_bytes(E) <= 160 * 1024;
   if constexpr (MODE != MODE_WGRAD) {
+    if (thin_rows(M, E) && (R + 2 * P_BK) * ld * 2 < (int64_t)DM_OOB)
+      return tt_gmm_thin(MODE, TB, ET, p0, p1, out, M, K, N, E, counts, s);
     // The persistent kernel needs two k-tiles per output tile, its LDS
     // (stages, epilogue staging, schedule) and 32-bit offsets for loads that
     // run up to two k-tiles past the reduction end.

@@ -1,0 +1,338 @@
+// Grouped GEMM, forward and data gradient, for experts of few rows (gfx950).
+//
+// With a few rows per expert the launch streams every used expert's weights
+// once and is bound by that stream. The persistent 256x256 kernel of gmm.hip
+// holds one block per CU: a tile's prologue and epilogue leave the CU's
+// memory path idle, and its few tiles (48 for one token of Qwen3-30B-A3B's
+// fc1) leave most CUs idle. Here a block computes BM x 128 outputs over the
+// whole reduction, small enough that two blocks share a CU and one streams
+// while the other starts or ends.
+#include "gemm.h"
+
+#include <type_traits>
+
+namespace {
+
+constexpr int T_BN = 128, T_BK = 64, T_NT = 256;
+// Up to this many bytes of weights (half the memory-side cache) a launch
+// reads with the default policy: they may still be cached from the last call.
+// Larger streams only push each other out, and the streaming policy reads
+// them faster: 119 experts of 2048 x 1536 (751 MB) 120 us, 6.3 TB/s, against
+// 135 us with the default policy; 8 of them (50 MB, cached) 20 against 15 us.
+constexpr int64_t T_CACHED = 128 << 20;
+// Rows per expert on average up to which tiles have 64 rows: Qwen3-30B-A3B's
+// four products with 64- / 128-row tiles at 32 rows per expert 148 + 78 + 143
+// + 84 / 148 + 80 + 152 + 102 us, at 48 166 + 87 + 161 + 96 / 159 + 87 + 163
+// + 106, at 62 177 + 90 + 179 + 95 / 164 + 90 + 171 + 107; 16 experts of
+// 4096 x 3072 at 50 rows 85 + 48 + 87 + 45 / 80 + 37 + 71 + 67 us.
+constexpr int64_t T_ROWS64 = 40;
+constexpr int T_B = T_BN * T_BK * 2;  // weight tile (16 KiB)
+
+// What one block computes.
+struct ThinTile {
+  int e, mt, nt;
+  int64_t seg0, nrows;
+};
+
+// The block's (expert, row tile, column tile) from the per-expert counts:
+// consecutive slots, an expert's row tiles of one column tile first (they
+// share its weights), on one XCD. Returns false past the last slot.
+template <int BM>
+__device__ __forceinline__ bool thin_tile(const int64_t* __restrict__ counts, int E, int tiles_j,
+                                          char* scratch, ThinTile& t) {
+  int64_t* const wrow = reinterpret_cast<int64_t*>(scratch);
+  int64_t* const found_seg = wrow + T_NT / 64;
+  int* const wtile = reinterpret_cast<int*>(found_seg + 2);
+  int* const found = wtile + T_NT / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int per = (E + T_NT - 1) / T_NT;
+  int64_t r = 0;
+  int tl = 0;
+  for (int i = 0; i < per; ++i) {
+    const int e = tid * per + i;
+    const int64_t c = e < E ? counts[e] : 0;
+    r += c;
+    tl += (int)((c + BM - 1) / BM);
+  }
+  int64_t ri = r;
+  int ti = tl;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int64_t o = __shfl_up(ri, off, 64);
+    const int ot = __shfl_up(ti, off, 64);
+    if (lane >= off) {
+      ri += o;
+      ti += ot;
+    }
+  }
+  if (lane == 63) {
+    wrow[wave] = ri;
+    wtile[wave] = ti;
+  }
+  __syncthreads();
+  int64_t rb = 0;
+  int tb = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < T_NT / 64; ++w) {
+    if (w < wave) {
+      rb += wrow[w];
+      tb += wtile[w];
+    }
+    total += wtile[w];
+  }
+  rb += ri - r;
+  tb += ti - tl;
+  total *= tiles_j;
+  if ((int)blockIdx.x >= total) return false;
+  const int slot = xcd_remap(blockIdx.x, total);
+  if (slot >= tb * tiles_j && slot < (tb + tl) * tiles_j) {
+    for (int i = 0;; ++i) {
+      const int e = tid * per + i;
+      const int64_t c = counts[e];
+      const int m = (int)((c + BM - 1) / BM);
+      if (slot < (tb + m) * tiles_j) {
+        const int local = slot - tb * tiles_j;
+        found[0] = e;
+        found[1] = local % m;
+        found[2] = local / m;
+        found_seg[0] = rb;
+        found_seg[1] = c;
+        break;
+      }
+      rb += c;
+      tb += m;
+    }
+  }
+  __syncthreads();
+  t.e = __builtin_amdgcn_readfirstlane(found[0]);
+  t.mt = __builtin_amdgcn_readfirstlane(found[1]);
+  t.nt = __builtin_amdgcn_readfirstlane(found[2]);
+  t.seg0 = rfl64(found_seg[0]);
+  t.nrows = rfl64(found_seg[1]);
+  __syncthreads();  // the scratch is the first stage's memory
+  return true;
+}
+
+// One block computes BM x 128 outputs of one expert; wave w owns columns
+// 32 w .. 32 w + 31 of every row, so each weight fragment is read from LDS
+// once. The 64-deep k-tiles stream into a ring of S LDS stages (weights
+// 16 KiB, activations 128 bytes per row), S - 1 of them in flight or being
+// waited for, with one barrier per k-tile: it publishes k-tile kt and frees
+// the stage of kt - 1, into which kt + S - 1 is then loaded. Resources end at
+// the expert's rows and weights, so rows past them read as zeros without
+// memory traffic; a K-major reduction tail (KMASK) is masked per chunk.
+template <int MODE, bool TRANS_B, int ET, bool KMASK, int BM, int S, int OCC>
+__global__ __launch_bounds__(T_NT, OCC) void gmm_thin_kernel(
+    const char* __restrict__ p0, const char* __restrict__ p1, char* __restrict__ out, int64_t K,
+    int64_t N, int E, const int64_t* __restrict__ counts, int tiles_j, int stream) {
+  constexpr bool B_K = Layout<MODE, TRANS_B>::B_K;
+  constexpr int T_A = BM * T_BK * 2, STAGE = T_A + T_B;
+  constexpr int FM = BM / 32;           // 32-row blocks
+  constexpr int LA = BM / 32, LD = 4 + LA;  // loads per wave and k-tile
+  __shared__ __align__(16) char lds_raw[S * STAGE];
+  ThinTile t;
+  if (!thin_tile<BM>(counts, E, tiles_j, lds_raw, t)) return;
+  const int64_t R = MODE == MODE_FWD ? K : N, J = MODE == MODE_FWD ? N : K;
+  const int64_t ldb = TRANS_B ? K : N;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nkt = (int)((R + T_BK - 1) / T_BK);
+  const int64_t i0 = (int64_t)t.mt * BM, j0 = (int64_t)t.nt * T_BN;
+  const int64_t rows = t.nrows - i0;  // valid rows of the tile, at least one
+
+  // Weights that only this block reads go past the caches.
+  const bool once = stream && t.nrows <= BM;
+
+  // Resources at the tile origin, advanced by a k-tile at a time.
+  const i32x4 ra = make_rsrc(p0 + (t.seg0 + i0) * R * 2, (rows < BM ? rows : BM) * R * 2);
+  const char* wb = p1 + (int64_t)t.e * K * N * 2;
+  const int64_t boff = B_K ? j0 * ldb * 2 : j0 * 2;
+  const i32x4 rb = make_rsrc(wb + boff, K * N * 2 - boff);
+  const uint32_t ks_a = T_BK * 2, ks_b = B_K ? T_BK * 2 : (uint32_t)(T_BK * ldb * 2);
+
+  // Loads, 1 KiB per instruction. A: rows (BM / 4) w + 8 q + lane / 8, chunk
+  // slot lane % 8 holding chunk slot ^ ((row >> 1) & 7); K-major weights the
+  // same with rows 32 w + 8 q. MN-major weights: k-rows 16 w + 4 q + lane / 16
+  // of 256 bytes, slot lane % 16 holding chunk slot ^ (4 (k-row % 4)).
+  uint32_t aoff[LA], boffs[4];
+  int akof[LA], bkof[4];
+#pragma unroll
+  for (int q = 0; q < LA; ++q) {
+    const int r = 8 * LA * wave + 8 * q + (lane >> 3);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    akof[q] = 8 * c;
+    aoff[q] = (uint32_t)((r * R + 8 * c) * 2);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (B_K) {
+      const int r = 32 * wave + 8 * q + (lane >> 3);
+      const int c = (lane & 7) ^ ((r >> 1) & 7);
+      bkof[q] = 8 * c;
+      boffs[q] = (uint32_t)((r * ldb + 8 * c) * 2);
+    } else {
+      const int kr = 16 * wave + 4 * q + (lane >> 4);
+      const int c = (lane & 15) ^ (4 * (kr & 3));
+      bkof[q] = 0;
+      boffs[q] = (uint32_t)((kr * ldb + 8 * c) * 2);
+    }
+  }
+  lds_char* const lds = (lds_char*)lds_raw;
+  auto issue = [&](int kt, int slot) {
+    const uint32_t base = lds_addr_of(lds) + (uint32_t)slot * STAGE;
+    const i32x4 rbk = advance_rsrc(rb, (uint32_t)kt * ks_b);
+    const i32x4 rak = advance_rsrc(ra, (uint32_t)kt * ks_a);
+    uint32_t off[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      off[q] = KMASK && B_K && kt * T_BK + bkof[q] >= (int)R ? DM_OOB : boffs[q];
+    const uint32_t wbase = base + T_A + (uint32_t)(4 * wave) * 1024u;
+    if (once) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) dma16_stream(off[q], rbk, wbase + q * 1024u);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) dma16(off[q], rbk, wbase + q * 1024u);
+    }
+#pragma unroll
+    for (int q = 0; q < LA; ++q) {
+      dma16(KMASK && kt * T_BK + akof[q] >= (int)R ? DM_OOB : aoff[q], rak, base + (uint32_t)(LA * wave + q) * 1024u);
+    }
+  };
+
+  // Fragment offsets within a stage.
+  uint32_t fa[4], fb[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    fa[s] = fragk64(0, s, lane);
+    if constexpr (B_K) {
+      fb[s] = T_A + fragk64(32 * wave, s, lane);
+    } else {
+      const int g = lane >> 4, i = lane & 15;
+      const int col = 32 * wave + 16 * (g & 1) + 4 * (i & 3);
+      const int kr = 16 * s + 8 * (g >> 1) + (i >> 2);
+      fb[s] = T_A + (uint32_t)(kr * 256 + (((col >> 3) ^ (4 * (kr & 3))) << 4) + (col & 7) * 2);
+    }
+  }
+  f32x16 acc[FM] = {};
+  const int nmi = __builtin_amdgcn_readfirstlane((int)((rows + 31) / 32));  // blocks with rows
+
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < nkt) issue(s, s);
+  // The k-loop for the NM 32-row blocks that hold rows.
+  auto loop = [&](auto nm_c) {
+    constexpr int NM = decltype(nm_c)::value;
+    int slot = 0;
+    for (int kt = 0; kt < nkt; ++kt) {
+      // k-tile kt has landed once at most the later ones are outstanding.
+      const int later = nkt - 1 - kt;
+      if (S >= 4 && later >= 2) TT_WAIT_VMCNT(2 * LD);
+      else if (S >= 3 && later >= 1) TT_WAIT_VMCNT(LD);
+      else TT_WAIT_VMCNT(0);
+      TT_LDS_BARRIER();
+      const int nslot = slot == 0 ? S - 1 : slot - 1;  // the stage of kt - 1
+      if (kt + S - 1 < nkt) issue(kt + S - 1, nslot);
+      lds_char* const stg = lds + slot * STAGE;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        uint4 b;
+        if constexpr (B_K) {
+          b = read_k(stg, fb[s]);
+        } else {
+          const i16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(stg + fb[s]));
+          const i16x4 v1 =
+              __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(stg + fb[s] + 1024));
+          const uint2 w0 = __builtin_bit_cast(uint2, v0), w1 = __builtin_bit_cast(uint2, v1);
+          b = uint4{w0.x, w0.y, w1.x, w1.y};
+        }
+#pragma unroll
+        for (int mi = 0; mi < NM; ++mi)
+          acc[mi] = Mma<ET>::run(b, read_k(stg, fa[s] + mi * 4096), acc[mi]);
+      }
+      slot = slot == S - 1 ? 0 : slot + 1;
+    }
+  };
+  if (FM == 1 || nmi == 1) loop(std::integral_constant<int, 1>{});
+  else if (FM == 2 || nmi == 2) loop(std::integral_constant<int, (FM < 2 ? FM : 2)>{});
+  else if (nmi == 3) loop(std::integral_constant<int, (FM < 3 ? FM : 3)>{});
+  else loop(std::integral_constant<int, FM>{});
+
+  // Epilogue: the BM x 128 tile row-major through LDS (256-byte rows, 16-byte
+  // chunk c of row r in slot c ^ (r % 16)), stored as whole row segments.
+  // Block mi, register 4g + e of lane l is row 32 mi + l % 32, column
+  // 32 wave + 8 g + 4 (l / 32) + e.
+  TT_LDS_BARRIER();  // every wave is past its fragment reads
+#pragma unroll
+  for (int mi = 0; mi < FM; ++mi)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int r = 32 * mi + (lane & 31), c = 4 * wave + g;
+      const uint2 v = pack4<ET>(acc[mi][4 * g], acc[mi][4 * g + 1], acc[mi][4 * g + 2],
+                                acc[mi][4 * g + 3]);
+      *reinterpret_cast<lds_u32x2*>(lds + r * 256 + ((c ^ (r & 15)) << 4) + 8 * (lane >> 5)) =
+          u32x2{v.x, v.y};
+    }
+  __syncthreads();
+  const int c = threadIdx.x & 15;
+  if (j0 + 8 * c >= J) return;
+#pragma unroll
+  for (int p = 0; p < BM / 16; ++p) {
+    const int r = 16 * p + (threadIdx.x >> 4);
+    if (r < rows)
+      *reinterpret_cast<uint4*>(out + ((t.seg0 + i0 + r) * J + j0 + 8 * c) * 2) =
+          read_k(lds, (uint32_t)(r * 256 + ((c ^ (r & 15)) << 4)));
+  }
+}
+
+template <int MODE, bool TB, int ET, bool KMASK, int BM, int S, int OCC>
+int launch_thin_k(const void* p0, const void* p1, void* out, int64_t M, int64_t K, int64_t N,
+                  int E, const int64_t* counts, hipStream_t s) {
+  const int64_t J = MODE == MODE_FWD ? N : K;
+  const int tj = (int)((J + T_BN - 1) / T_BN);
+  // Each used expert adds at most one partial row tile.
+  const int64_t nblk = (M / BM + (M < E ? M : E)) * tj;
+  if (nblk == 0) return TT_OK;
+  TT_REQUIRE(nblk < 0x7fffffff, "gmm: grid too large");
+  const int stream = (M < E ? M : E) * K * N * 2 > T_CACHED ? 1 : 0;
+  hipLaunchKernelGGL((gmm_thin_kernel<MODE, TB, ET, KMASK, BM, S, OCC>), dim3((unsigned)nblk),
+                     dim3(T_NT), 0, s, static_cast<const char*>(p0),
+                     static_cast<const char*>(p1), static_cast<char*>(out), K, N, E, counts, tj,
+                     stream);
+  return tt_check_launch("gmm");
+}
+
+// 64-row tiles (72 KiB of LDS, three stages) up to an average of T_ROWS64
+// rows per expert, 128-row tiles (64 KiB, two stages) above.
+template <int MODE, bool TB, int ET>
+int launch_thin(const void* p0, const void* p1, void* out, int64_t M, int64_t K, int64_t N,
+                int E, const int64_t* counts, hipStream_t s) {
+  const int64_t R = MODE == MODE_FWD ? K : N;
+  if (M <= (int64_t)E * T_ROWS64) {
+    if (R % T_BK)
+      return launch_thin_k<MODE, TB, ET, true, 64, 3, 2>(p0, p1, out, M, K, N, E, counts, s);
+    return launch_thin_k<MODE, TB, ET, false, 64, 3, 2>(p0, p1, out, M, K, N, E, counts, s);
+  }
+  if (R % T_BK)
+    return launch_thin_k<MODE, TB, ET, true, 128, 2, 2>(p0, p1, out, M, K, N, E, counts, s);
+  return launch_thin_k<MODE, TB, ET, false, 128, 2, 2>(p0, p1, out, M, K, N, E, counts, s);
+}
+
+}  // namespace
+
+int tt_gmm_thin(int mode, bool tb, int dtype, const void* p0, const void* p1, void* out,
+                int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s) {
+  auto go = [&](auto mode_c, auto tb_c, auto et_c) {
+    return launch_thin<decltype(mode_c)::value, decltype(tb_c)::value, decltype(et_c)::value>(
+        p0, p1, out, M, K, N, E, counts, s);
+  };
+  using FW = std::integral_constant<int, MODE_FWD>;
+  using DG = std::integral_constant<int, MODE_DGRAD>;
+  using BF = std::integral_constant<int, TT_BF16>;
+  using HF = std::integral_constant<int, TT_F16>;
+  auto typed = [&](auto mode_c, auto et_c) {
+    return tb ? go(mode_c, std::true_type{}, et_c) : go(mode_c, std::false_type{}, et_c);
+  };
+  if (mode == MODE_FWD) return dtype == TT_BF16 ? typed(FW{}, BF{}) : typed(FW{}, HF{});
+  return dtype == TT_BF16 ? typed(DG{}, BF{}) : typed(DG{}, HF{});
+}
