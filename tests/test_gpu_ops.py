@@ -1104,6 +1104,50 @@ def test_grouped_matmul_few_rows_exact(counts, K, N, dtype, trans_b):
         s0 += c
 
 
+# FP8 launches of at most 40 rows per expert on average: 32-row tiles up to 20 rows, 64-row
+# tiles above; reductions with partial scale blocks and tails, both scale dtypes.
+FEW_ROWS_FP8 = [
+    ([0, 1, 31, 32, 33, 0, 2], 256, 384, torch.bfloat16),
+    ([1], 16, 16, torch.float32),
+    ([63, 64, 65, 0, 0, 0, 1, 39], 400, 144, torch.float32),
+    ([0] * 260 + [5, 3], 128, 272, torch.bfloat16),
+    ([40, 70, 10], 1024, 656, torch.bfloat16),
+    ([3, 20], 128 * 70, 48, torch.float32),  # scales of two registers
+]
+
+
+@pytest.mark.parametrize("counts,K,N,sdt", FEW_ROWS_FP8, ids=[f"E{len(c[0])}K{c[1]}N{c[2]}" for c in FEW_ROWS_FP8])
+def test_grouped_matmul_fp8_few_rows_exact(counts, K, N, sdt):
+    """Small-integer codes, power-of-two scales (exact sums), NaN-filled outputs with a guard
+    row; codes include every sign and zero."""
+    from torchturbo_amd import _lib
+
+    g = torch.Generator().manual_seed(K * 3 + N)
+    E, M = len(counts), sum(counts)
+    x = torch.randint(-2, 3, (M, K), generator=g).to(torch.bfloat16).to(DEV)
+    dy = torch.randint(-2, 3, (M, N), generator=g).to(torch.bfloat16).to(DEV)
+    q = torch.randint(-2, 3, (E, N, K), generator=g).float().to(torch.float8_e4m3fn).to(DEV)
+    sc = (2.0 ** torch.randint(-1, 2, (E, -(-N // 128), -(-K // 128)), generator=g)).to(sdt).to(DEV)
+    cnt = torch.tensor(counts, dtype=torch.int64, device=DEV)
+    y = torch.full((M + 1, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    dx = torch.full((M + 1, K), float("nan"), dtype=torch.bfloat16, device=DEV)
+    args = (_lib.ptr(q.view(torch.uint8)), _lib.ptr(sc), _lib.dtype_code(sdt), M, K, N, E, _lib.ptr(cnt))
+    _lib.call("tt_gmm_fp8_fwd", _lib.ptr(x), *args, _lib.ptr(y), _lib.stream())
+    _lib.call("tt_gmm_fp8_dgrad", _lib.ptr(dy), *args, _lib.ptr(dx), _lib.stream())
+    torch.cuda.synchronize()
+    assert y[M].isnan().all() and dx[M].isnan().all()
+    s0 = 0
+    for e, c in enumerate(counts):
+        if not c:
+            continue
+        full = sc[e].double().cpu().repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)[:, :K]
+        we = q[e].float().cpu().double() * full  # [N, K]
+        xe, de = x[s0:s0 + c].double().cpu(), dy[s0:s0 + c].double().cpu()
+        assert torch.equal(y[s0:s0 + c].cpu(), (xe @ we.t()).to(torch.bfloat16)), (e, c)
+        assert torch.equal(dx[s0:s0 + c].cpu(), (de @ we).to(torch.bfloat16)), (e, c)
+        s0 += c
+
+
 # more 256x256 output tiles than the GPU has compute units, so every persistent block
 # walks many tiles (tile switch, cross-tile prefetch, XCD remap); mean expert loads above
 # 512 rows take the four-stage weight-gradient kernel, at most 512 the persistent

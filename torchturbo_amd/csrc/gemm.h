@@ -149,6 +149,17 @@ __device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
   }
 }
 
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+// Four e4m3 bytes -> four bf16 (two dwords), each bf16(f32(q) * s).
+__device__ __forceinline__ uint2 deq4(uint32_t q, float s) {
+  const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)q, false);
+  const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)q, true);
+  const bf16x2_t a = {(__bf16)(lo.x * s), (__bf16)(lo.y * s)};
+  const bf16x2_t b = {(__bf16)(hi.x * s), (__bf16)(hi.y * s)};
+  return uint2{__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b)};
+}
+
 // K-major 64-deep tile: LDS row r (128 bytes) holds tile row r, its 16-byte
 // chunk c in slot c ^ ((r >> 1) & 7): any 16 consecutive rows then cover the
 // 16 distinct 16-byte bank groups of a 256-byte bank line, so a fragment
@@ -173,3 +184,10 @@ __device__ __forceinline__ uint32_t fragk64(int r0, int s, int lane) {
 // tt_gmm_fwd / tt_gmm_dgrad, already checked; see thin_rows in gmm.hip.
 int tt_gmm_thin(int mode, bool tb, int dtype, const void* p0, const void* p1, void* out,
                 int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s);
+// The same with e4m3 weights and block scales, as tt_gmm_fp8_fwd / _dgrad, at
+// most TT_THIN8_SCALES scale blocks along the reduction; see thin8_rows in
+// gmm.hip.
+#define TT_THIN8_SCALES 128
+int tt_gmm_thin8(int mode, const void* p0, const uint8_t* qw, const void* scale, int sdt,
+                 void* out, int64_t M, int64_t K, int64_t N, int E, const int64_t* counts,
+                 hipStream_t s);

@@ -48,7 +48,8 @@
 //   tiles two per schedule slot. Launches of few rows per expert on average
 //   (thin_rows) run on gmm_thin.hip instead.
 // * gmm_q8_kernel (fwd/dgrad with e4m3 weights and 128x128 block scales,
-//   every launch whose reduction is longer than one 64-deep k-tile):
+//   launches of more than a few rows per expert (thin8_rows; the others run on
+//   gmm_thin.hip) whose reduction is longer than one 64-deep k-tile):
 //   persistent like gmm_p64_kernel, 128x512x64 tiles (the four waves share
 //   the tile's 128 rows and take 128 columns each, so an expert's rows are
 //   padded to 128 only). The weight tile stays e4m3 in LDS; each wave reads
@@ -1721,18 +1722,7 @@ constexpr int F8_STAGE = DM_TILE + DM_TILE / 2;  // A (bf16) + B (e4m3) of one k
 constexpr int F8_BUF = DM_TILE;                  // one dequantised B tile
 constexpr int F8_LDS = 4 * F8_STAGE + 3 * F8_BUF;
 
-typedef __attribute__((ext_vector_type(2))) float f32x2;
 
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-
-// Four e4m3 bytes -> four bf16 (two dwords), each bf16(f32(q) * s).
-__device__ __forceinline__ uint2 deq4(uint32_t q, float s) {
-  const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)q, false);
-  const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)q, true);
-  const bf16x2_t a = {(__bf16)(lo.x * s), (__bf16)(lo.y * s)};
-  const bf16x2_t b = {(__bf16)(hi.x * s), (__bf16)(hi.y * s)};
-  return uint2{__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b)};
-}
 
 template <int MODE, bool KMASK>
 __global__ __launch_bounds__(DM_NT) void gmm_fp8_kernel(const char* __restrict__ p0,
@@ -2754,6 +2744,14 @@ int launch_q8_k(const void* p0, const uint8_t* qw, const void* scale, int sdt, v
   return tt_check_launch("gmm_fp8");
 }
 
+// FP8 fwd / dgrad with at most this many rows per expert on average run on
+// gmm_thin8_kernel (gmm_thin.hip). DeepSeek-V3's fc1 + fc2 (256 experts),
+// gmm_q8_kernel / thin: at 32 rows per expert forward 1718 + 879 / 1418 + 802
+// us, data gradient 1586 + 793 / 1575 + 718; at 64 rows 1806 + 934 / 2001 +
+// 1081 and 1693 + 863 / 2100 + 1047.
+constexpr int64_t THIN8_ROWS = 40;
+bool thin8_rows(int64_t M, int E) { return M <= (int64_t)E * THIN8_ROWS; }
+
 template <int MODE>
 int launch_fp8(const void* p0, const uint8_t* qw, const void* scale, int sdt, void* out, int64_t M,
                int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s) {
@@ -2767,6 +2765,9 @@ int launch_fp8(const void* p0, const uint8_t* qw, const void* scale, int sdt, vo
     const int tjq = (int)((J + Q_BN - 1) / Q_BN);
     const int64_t nq = ((M + Q_BM - 1) / Q_BM + E) * (int64_t)tjq;
     if (nq == 0) return TT_OK;
+    if (thin8_rows(M, E) && (R + 127) / 128 <= TT_THIN8_SCALES &&
+        (M + DM_BM) * lda * 2 < (int64_t)DM_OOB && (N + 2 * Q_BK + Q_BN) * K < (int64_t)DM_OOB)
+      return tt_gmm_thin8(MODE, p0, qw, scale, sdt, out, M, K, N, E, counts, s);
     if (R > Q_BK && (R + 127) / 128 <= Q_SMAX &&
         schedule_bytes(E) + 2 * Q_STAGE + 4 * P_EPI + 4 * Q_SMAX * sizeof(float) + 64 <=
             160 * 1024 &&
