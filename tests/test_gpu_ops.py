@@ -257,6 +257,76 @@ def test_router_gate_topk_hash_routing(hip_ops):
     assert rel_errors(p.cpu(), pr)[0] <= 2e-6
 
 
+@pytest.mark.parametrize("H,E", [(64, 32), (192, 96), (320, 256)])
+@pytest.mark.parametrize("dtype,rdt", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+def test_router_gate_small_batches_equal_the_one_kernel_gate(H, E, dtype, rdt):
+    """Batches whose logits are formed with the experts spread over blocks (one 32x32 tile per
+    block, and 64x64 tiles at 4200 tokens) against the same rows of a 16384-token batch, which
+    takes the one-kernel gate: logits, probabilities, map and ids bit for bit."""
+    from torchturbo_amd import _lib
+
+    g = torch.Generator().manual_seed(H)
+    x = torch.randn(16384, H, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(E, H, generator=g) * H ** -0.5).to(dtype).to(DEV)
+
+    def run(T):
+        out = (torch.full((T, E), float("nan"), dtype=rdt, device=DEV),
+               torch.full((T, E), float("nan"), dtype=rdt, device=DEV),
+               torch.full((T, E), 7, dtype=torch.uint8, device=DEV),
+               torch.full((T, 4), -1, dtype=torch.int64, device=DEV))
+        _lib.call("tt_router_gate_fwd", _lib.ptr(x), _lib.ptr(w), _lib.dtype_code(dtype), T, H, E,
+                  _lib.dtype_code(rdt), 4, 1, 0, None, 0, 0, 2.5, None, *map(_lib.ptr, out),
+                  _lib.stream())
+        return out
+
+    full = run(16384)
+    for T in (1, 31, 33, 64, 1000, 4200):
+        for got, ref in zip(run(T), full):
+            assert torch.equal(got, ref[:T]), T
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 8, 2), (63, 64, 8), (64, 128, 8), (65, 1000, 16), (256, 33, 1),
+                                   (257, 128, 8), (1000, 300, 6), (1024, 256, 16), (1536, 320, 8),
+                                   (1537, 64, 4), (513, 1097, 2), (700, 2048, 3)])
+def test_route_index_small_batches(T, E, k):
+    """The one-launch routing index (up to 1536 tokens) and sizes just past its limits: rows,
+    tokens, counts, packed probabilities and rejected slots (ids out of range, repeats),
+    against a stable sort."""
+    from torchturbo_amd import _lib
+
+    g = torch.Generator().manual_seed(T + E)
+    ids = torch.rand(T, E, generator=g).topk(k, dim=1).indices
+    bad = torch.rand(T, k, generator=g)
+    ids[bad < 0.05] = E
+    ids[bad > 0.97] = -3
+    if k > 1:
+        ids[::7, 1] = ids[::7, 0]
+    ok = (ids >= 0) & (ids < E)
+    for j in range(1, k):
+        ok[:, j] &= ~((ids[:, :j] == ids[:, j:j + 1]) & ok[:, :j]).any(1)
+    probs = torch.rand(T, E, generator=g)
+    flat = ok.reshape(-1).nonzero().squeeze(1)
+    order = flat[torch.argsort(ids.reshape(-1)[flat], stable=True)]
+    rows_r = torch.full((T * k,), -1, dtype=torch.int32)
+    rows_r[order] = torch.arange(len(order), dtype=torch.int32)
+    idd, pd = ids.to(DEV), probs.to(DEV)
+    rows = torch.full((T, k), -9, dtype=torch.int32, device=DEV)
+    tok = torch.full((T * k,), -9, dtype=torch.int32, device=DEV)
+    packed = torch.full((T * k,), -9.0, device=DEV)
+    counts = torch.full((E,), -9, dtype=torch.int64, device=DEV)
+    nbytes = _lib.route_index_workspace(T, E)
+    ws = torch.full((nbytes,), 255, dtype=torch.uint8, device=DEV)
+    _lib.call("tt_route_index", _lib.ptr(idd), T, k, E, _lib.ptr(pd), 0, _lib.ptr(rows), _lib.ptr(tok),
+              _lib.ptr(packed), _lib.ptr(counts), _lib.ptr(ws), nbytes, _lib.stream())
+    n = len(order)
+    assert torch.equal(rows.cpu().reshape(-1), rows_r)
+    assert torch.equal(tok.cpu()[:n].long(), order // k) and (tok.cpu()[n:] == -9).all()
+    assert torch.equal(packed.cpu()[:n], probs.reshape(-1)[order // k * E + ids.reshape(-1)[order]])
+    assert torch.equal(counts.cpu(), torch.bincount(ids.reshape(-1)[order], minlength=E))
+    off = _lib.route_index_rejected_offset(T, E)
+    assert int(ws[off:off + 4].view(torch.int32).item()) == T * k - n
+
+
 def test_router_gate_rejects_unsupported_shapes(hip_ops):
     x = torch.randn(8, 96, device=DEV).bfloat16()
     w = torch.randn(64, 96, device=DEV).bfloat16()

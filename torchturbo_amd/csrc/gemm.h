@@ -191,3 +191,8 @@ int tt_gmm_thin(int mode, bool tb, int dtype, const void* p0, const void* p1, vo
 int tt_gmm_thin8(int mode, const void* p0, const uint8_t* qw, const void* scale, int sdt,
                  void* out, int64_t M, int64_t K, int64_t N, int E, const int64_t* counts,
                  hipStream_t s);
+
+// Router logits of few tokens (gate.hip): logits [T, E] = x [T, H] w [E, H]^T
+// in 16 bits (dtype), E a multiple of 32, H of 64; ldt is TT_F32 or dtype.
+int tt_gate_logits(const void* x, const void* w, int dtype, int64_t T, int H, int E, int ldt,
+                   void* logits, hipStream_t s);

@@ -6,7 +6,9 @@
 // lanes' best remaining keys and a ballot for the lowest lane holding it.
 // Group-limited selection uses segmented shuffles over the lanes of a group.
 //
-// Routing index: packed rows are ordered by expert, then token. Three kernels:
+// Routing index: packed rows are ordered by expert, then token. One block
+// per 256 tokens in one launch for small batches (route_small_kernel), above
+// kSmallTokens three kernels:
 //   hist  : per 256-token block, per-expert counts  -> bc[E][nb]
 //   scan  : per expert, exclusive scan over blocks   -> bc (in place), totals
 //   rank  : per block, expert base + wave prefix + in-wave ballot rank
@@ -17,7 +19,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "common.h"
+#include "gemm.h"
 
 namespace {
 
@@ -958,6 +960,138 @@ __global__ __launch_bounds__(kIdxBlock) void route_rank_kernel(
   }
 }
 
+// The routing index of a small batch in one launch. Every block counts the
+// whole batch's assignments per expert itself (LDS atomics, order-free), and
+// apart those of the tokens before its own 256, so no block waits for another;
+// then each lane's rank among its wave comes from a 64-bit lane mask per
+// (wave, expert), as in route_rank_kernel. Latency-bound: E 128, k 8, three
+// kernels / this one: 1 token 15.4 / 8.1 us, 256 18.4 / 10.4, 1000 19.2 / 15.1,
+// 1531 19.8 / 18.0, 2048 19.8 / 20.5; E 64, k 16: 48 31.9 / 14.2, 1531 45.2 /
+// 40.1. (One block of 1024 threads for the whole batch took 31 us at 1000
+// tokens: one CU's scattered accesses.)
+template <int KMAX>
+__global__ __launch_bounds__(kIdxBlock) void route_small_kernel(
+    const int64_t* __restrict__ ids, int T, int K, int E, const void* __restrict__ probs,
+    int pbytes, int32_t* __restrict__ rows_out, int32_t* __restrict__ token_of_row,
+    void* __restrict__ packed_probs, int64_t* __restrict__ counts, int* __restrict__ bad_total) {
+  constexpr int NT = kIdxBlock, W = NT / TT_WAVE;
+  extern __shared__ __align__(16) uint64_t small_smem[];
+  uint64_t* const wmask = small_smem;                        // [W][E] lanes holding the expert
+  int* const wbase = reinterpret_cast<int*>(wmask + W * E);  // [W][E] first row of the wave
+  int* const total = wbase + W * E;                          // [E]
+  int* const before = total + E;                             // [E] of the blocks before
+  __shared__ int wsum[W];
+  __shared__ int nbad;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int t0 = blockIdx.x * NT, mine = t0 + tid;
+  for (int i = tid; i < W * E; i += NT) wmask[i] = 0ull;
+  for (int i = tid; i < 2 * E; i += NT) total[i] = 0;
+  if (tid == 0) nbad = 0;
+  __syncthreads();
+  int my[KMAX];  // the thread's own token
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) my[j] = -1;
+  int rejected = 0;
+  for (int t = tid; t < T; t += NT) {
+    int id[KMAX];
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+      const int64_t e = j < K ? ids[(int64_t)t * K + j] : -1;
+      id[j] = (e >= 0 && e < E) ? (int)e : -1;
+    }
+    // A repeated id keeps its first slot only.
+#pragma unroll
+    for (int j = 1; j < KMAX; ++j)
+#pragma unroll
+      for (int i = 0; i < j; ++i)
+        if (id[j] >= 0 && id[i] == id[j]) id[j] = -1;
+    rejected += K;
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j)
+      if (id[j] >= 0) {
+        --rejected;
+        atomicAdd(&total[id[j]], 1);
+        if (t < t0) atomicAdd(&before[id[j]], 1);
+        if (t == mine) {
+          my[j] = id[j];
+          atomicOr(reinterpret_cast<unsigned long long*>(&wmask[wave * E + id[j]]), 1ull << lane);
+        }
+      }
+  }
+  if (rejected) atomicAdd(&nbad, rejected);
+  __syncthreads();
+  // Exclusive scan of the totals (a run of experts per thread), then the first
+  // row of every (wave, expert) of this block.
+  const int per = (E + NT - 1) / NT;
+  int local = 0;
+  for (int i = 0; i < per; ++i) {
+    const int e = tid * per + i;
+    if (e < E) local += total[e];
+  }
+  int incl = local;
+#pragma unroll
+  for (int off = 1; off < TT_WAVE; off <<= 1) {
+    const int o = __shfl_up(incl, off, TT_WAVE);
+    if (lane >= off) incl += o;
+  }
+  if (lane == TT_WAVE - 1) wsum[wave] = incl;
+  __syncthreads();
+  int run = incl - local;
+  for (int w = 0; w < wave; ++w) run += wsum[w];
+  for (int i = 0; i < per; ++i) {
+    const int e = tid * per + i;
+    if (e < E) {
+      int base = run + before[e];
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        wbase[w * E + e] = base;
+        base += __popcll(wmask[w * E + e]);
+      }
+      if (blockIdx.x == 0) counts[e] = total[e];
+      run += total[e];
+    }
+  }
+  if (blockIdx.x == 0 && tid == 0) *bad_total = nbad;
+  __syncthreads();
+  if (mine >= T) return;
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (TT_WAVE - lane));
+  const bool weigh = probs != nullptr && packed_probs != nullptr;
+  int row[KMAX];
+  uint32_t p[KMAX];
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) {
+    row[j] = -1;
+    p[j] = 0;
+    if (my[j] >= 0) {
+      const int at = wave * E + my[j];
+      row[j] = wbase[at] + __popcll(wmask[at] & below);
+      const int64_t src = (int64_t)mine * E + my[j];
+      if (weigh)
+        p[j] = pbytes == 4 ? static_cast<const uint32_t*>(probs)[src]
+                           : static_cast<const uint16_t*>(probs)[src];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) {
+    if (j < K) rows_out[(int64_t)mine * K + j] = row[j];
+    if (row[j] >= 0) {
+      token_of_row[row[j]] = mine;
+      if (weigh) {
+        if (pbytes == 4) static_cast<uint32_t*>(packed_probs)[row[j]] = p[j];
+        else static_cast<uint16_t*>(packed_probs)[row[j]] = (uint16_t)p[j];
+      }
+    }
+  }
+}
+
+// Batches route_small_kernel takes: at most kSmallTokens tokens of at most 16
+// experts each, its tables within 60 KiB of LDS.
+constexpr int64_t kSmallTokens = 1536;
+size_t route_small_lds(int E) { return (size_t)E * (4 * 12 + 8); }
+bool route_small_takes(int64_t T, int K, int E) {
+  return T > 0 && T <= kSmallTokens && K <= 16 && route_small_lds(E) <= 60 * 1024;
+}
+
 inline hipStream_t S(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 template <int EPL>
@@ -1043,8 +1177,7 @@ __device__ __forceinline__ gf32x16 rg_mma<TT_F16>(const uint4& a, const uint4& b
                                                  __builtin_bit_cast(gf16x8, b), c, 0, 0, 0);
 }
 
-// N 32-expert tiles (E = 32 N), TOK tokens per block (64, or 32 when 64-token
-// blocks would leave compute units idle).
+// N 32-expert tiles (E = 32 N), TOK tokens per block.
 template <int N, int TOK>
 struct GateShape {
   static constexpr int E = 32 * N;                              // experts
@@ -1222,18 +1355,6 @@ int gate_cu_count() {
   return cached[dev];
 }
 
-// 64 tokens per block, or 32 when 64-token blocks would not cover the device.
-template <int ET, int N>
-int launch_gate(const void* x, const void* w, int64_t T, int H, int ldt, int K, int sf, int pre,
-                const float* bias, int G, int GK, float scale, const int64_t* fixed, void* logits,
-                void* probs, uint8_t* rmap, int64_t* top, hipStream_t s) {
-  if ((T + 63) / 64 < gate_cu_count())
-    return launch_gate_t<ET, N, 32>(x, w, T, H, ldt, K, sf, pre, bias, G, GK, scale, fixed,
-                                    logits, probs, rmap, top, s);
-  return launch_gate_t<ET, N, 64>(x, w, T, H, ldt, K, sf, pre, bias, G, GK, scale, fixed, logits,
-                                  probs, rmap, top, s);
-}
-
 int epl_for(int E) {
   const int need = (E + TT_WAVE - 1) / TT_WAVE;
   int epl = 1;
@@ -1357,6 +1478,19 @@ int route_index_run(const int64_t* expert_indices, int64_t num_tokens, int32_t t
     hipLaunchKernelGGL(route_scan_kernel, dim3(num_experts), dim3(64), 0, s, bc, 0, num_experts,
                        totals, tokens_per_expert, bad, bad_total);
     return tt_check_launch("route_scan");
+  }
+  if (route_small_takes(num_tokens, topk, num_experts)) {
+    const void* pp = (packed_probs != nullptr) ? probs_dense : nullptr;
+#define TT_SMALL(KM)                                                                             \
+  hipLaunchKernelGGL(route_small_kernel<KM>, dim3(nb), dim3(kIdxBlock),                         \
+                     route_small_lds(num_experts), s, expert_indices, (int)num_tokens, topk,    \
+                     num_experts, pp, tt_elem_size(probs_dtype), row_indices, token_of_row,     \
+                     packed_probs, tokens_per_expert, bad_total)
+    if (topk <= 2) TT_SMALL(2);
+    else if (topk <= 8) TT_SMALL(8);
+    else TT_SMALL(16);
+#undef TT_SMALL
+    return tt_check_launch("route_small");
   }
   hipLaunchKernelGGL(route_hist_kernel, dim3(nb), dim3(kIdxBlock), num_experts * sizeof(int), s,
                      expert_indices, num_tokens, topk, num_experts, nb, bc, bad);
@@ -1526,12 +1660,32 @@ extern "C" int tt_router_gate_fwd(const void* x, const void* weight, int in_dtyp
   const int gk = fixed_indices ? 0 : group_topk;
   const int H = (int)hidden;
   const int NE = num_experts / 32;
+  if ((num_tokens + 63) / 64 < gate_cu_count()) {
+    // 64-token blocks would leave compute units idle: the logits with the
+    // experts spread over blocks too (gate.hip), then the top-k on its own;
+    // the same bits. H 2048, E 128: 26.0 -> 17.0 us at 1000 tokens, 28.4 ->
+    // 27.2 at 8192; with 16384 tokens (256 blocks) 41.2 here, 37.8 split; H
+    // 7168, E 256: 135 here, 162 split.
+    const int rc = tt_gate_logits(x, weight, in_dtype, num_tokens, H, num_experts, logits_dtype,
+                                  logits, S(stream));
+    if (rc != TT_OK) return rc;
+    const dim3 grid((unsigned)((num_tokens + kRouterWaves - 1) / kRouterWaves));
+#define TT_GATE_TOPK(EPL)                                                                       \
+  launch_router_fwd<EPL>(grid, S(stream), logits, logits_dtype, num_tokens, num_experts, topk,  \
+                         score_function, pre_softmax, expert_bias, num_groups, gk,              \
+                         scaling_factor, fixed_indices, probs, routing_map, top_indices)
+    if (epl == 1) TT_GATE_TOPK(1);
+    else if (epl == 2) TT_GATE_TOPK(2);
+    else TT_GATE_TOPK(4);
+#undef TT_GATE_TOPK
+    return tt_check_launch("router_gate_topk");
+  }
 #define TT_GATE_N(ET, NN)                                                                       \
   case NN:                                                                                     \
-    return launch_gate<ET, NN>(x, weight, num_tokens, H, logits_dtype, topk, score_function,   \
-                               pre_softmax, expert_bias, num_groups, gk, scaling_factor,       \
-                               fixed_indices, logits, probs, routing_map, top_indices,         \
-                               S(stream));
+    return launch_gate_t<ET, NN, 64>(x, weight, num_tokens, H, logits_dtype, topk,             \
+                                     score_function, pre_softmax, expert_bias, num_groups, gk, \
+                                     scaling_factor, fixed_indices, logits, probs,             \
+                                     routing_map, top_indices, S(stream));
 #define TT_GATE(ET)                                                                            \
   switch (NE) {                                                                                \
     TT_GATE_N(ET, 1) TT_GATE_N(ET, 2) TT_GATE_N(ET, 3) TT_GATE_N(ET, 4)                        \
