@@ -339,6 +339,27 @@ int tt_fp8_quantize_blocks(const void* w, int dtype, int64_t num_experts, int64_
                            int64_t cols, uint8_t* q, void* scale, int scale_dtype,
                            void* stream);
 
+/* Per-expert LoRA residual of a grouped linear layer (engine/peft/lora.py:54-125,
+ * 640-725): y = base + round(round(h B_e) * scale), h = x A_e, for
+ * expert-major rows in bf16 / f16, A [E, k, r] and B [E, r, n] in fp32 (r <=
+ * 64, k and n multiples of 8), fp32 products and sums.
+ * down: out [m, r] fp32 = in [m, c] w, w = A (transposed 0); or, transposed,
+ *   out = round(in * scale) w^T with w = B [E, r, c] (the backward of up).
+ * up: out [m, c] = base + round(round(h w) * scale), w = B [E, r, c]; or,
+ *   transposed, out = round(h w^T) with w = A [E, c, r] and no base.
+ * wgrad: out [E, c, r] = in_e^T v_e (A's gradient); or, transposed, out
+ *   [E, r, c] = v_e^T round(in_e * scale) (B's); in [m, c], v [m, r] fp32.
+ *   Zeros for experts without rows. */
+int tt_lora_down(const void* in, const float* w, int dtype, int64_t m, int64_t c, int32_t r,
+                 int32_t transposed, float scale, int32_t num_experts, const int64_t* counts,
+                 float* out, void* stream);
+int tt_lora_up(const float* h, const float* w, const void* base, int dtype, int64_t m, int64_t c,
+               int32_t r, int32_t transposed, float scale, int32_t num_experts,
+               const int64_t* counts, void* out, void* stream);
+int tt_lora_wgrad(const void* in, const float* v, int dtype, int64_t m, int64_t c, int32_t r,
+                  int32_t transposed, float scale, int32_t num_experts, const int64_t* counts,
+                  float* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1421,3 +1421,54 @@ def test_grouped_matmul_fp8_many_tiles(hip_ops):
         assert mx <= 1e-2 and mean <= 2e-3, f"{name}: {mx:.3e} {mean:.3e}"
     for e in (3, 17):
         assert torch.count_nonzero(mw.grad[e]) == 0, e
+
+
+LORA_CASES = [
+    ([1], 8, 8, 1, torch.bfloat16),
+    ([0, 3, 64, 65, 0, 130], 264, 520, 16, torch.bfloat16),
+    ([17, 0, 63, 1], 72, 136, 17, torch.float16),
+    ([200, 5], 40, 248, 33, torch.bfloat16),
+    ([0] * 258 + [2, 0, 70], 512, 1000, 8, torch.float16),  # more experts than threads
+    ([96, 0, 33], 1032, 24, 64, torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("counts,K,N,r,dtype", LORA_CASES, ids=[f"E{len(c[0])}K{c[1]}N{c[2]}r{c[3]}" for c in LORA_CASES])
+def test_lora_residual_matches_fp64(hip_ops, counts, K, N, r, dtype):
+    """Output and every gradient of the fused residual against fp64. Bounds: u = half a unit of
+    the 16-bit type's relative spacing; the output rounds the product, its scaling and the sum
+    (u each, of |s d|, |s d| and |y|), dx once; the fp32 sums add 2^-24 per addition of |terms|
+    (K, N, r or the rows of them; twice over where two products chain)."""
+    g = torch.Generator().manual_seed(K + N + r)
+    E, M, s = len(counts), sum(counts), 0.37
+    x = torch.randn(M, K, generator=g).to(dtype)
+    base, dy = torch.randn(M, N, generator=g).to(dtype), torch.randn(M, N, generator=g).to(dtype)
+    a = torch.randn(E, K, r, generator=g) * K ** -0.5
+    b = torch.randn(E, r, N, generator=g)
+    leaves = [t.to(DEV).requires_grad_() for t in (base, x, a, b)]
+    y = hip_ops.lora_residual(*leaves, torch.tensor(counts, device=DEV), s)
+    y.backward(dy.to(DEV))
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    sp = 2.0 ** -23 * (K + N + r + max(counts))  # fp32 sums, two in a chain
+    got_dx, got_da, got_db = (t.grad.double().cpu() for t in leaves[1:])
+    assert torch.equal(leaves[0].grad.cpu(), dy)
+    gs = (dy * s).double()  # the scaled gradient, rounded as the module's composition does
+    r0 = 0
+    for e, c in enumerate(counts):
+        xe, ae, be, ge = x[r0:r0 + c].double(), a[e].double(), b[e].double(), gs[r0:r0 + c]
+        h, dh = xe @ ae, ge @ be.t()
+        habs = xe.abs() @ ae.abs()
+        d = h @ be
+        dabs = habs @ be.abs()
+        ref = base[r0:r0 + c].double() + s * d
+        err = (y[r0:r0 + c].double().cpu() - ref).abs()
+        assert torch.all(err <= u * (2 * s * d.abs() + ref.abs()) * 1.01 + sp * dabs + 1e-6), e
+        dhabs = ge.abs() @ be.abs().t()
+        dx = dh @ ae.t()
+        err = (got_dx[r0:r0 + c] - dx).abs()
+        assert torch.all(err <= u * dx.abs() * 1.01 + sp * (dhabs @ ae.abs().t()) + 1e-6), e
+        assert torch.all((got_da[e] - xe.t() @ dh).abs() <= sp * (xe.abs().t() @ dhabs) + 1e-9), e
+        assert torch.all((got_db[e] - h.t() @ ge).abs() <= sp * (habs.t() @ ge.abs()) + 1e-9), e
+        if not c:
+            assert not got_da[e].any() and not got_db[e].any()
+        r0 += c

@@ -178,6 +178,92 @@ __device__ __forceinline__ uint32_t fragk64(int r0, int s, int lane) {
 // not waited for.
 #define TT_LDS_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
+// Tile of a grid with one block per (expert, row tile, column tile).
+struct RowTile {
+  int e, mt, nt;
+  int64_t seg0, nrows;
+};
+
+// The block's (expert, row tile, column tile) from the per-expert counts:
+// consecutive slots, an expert's row tiles of one column tile first (they
+// share its weights), on one XCD. Returns false past the last slot. `scratch`:
+// at least 256 bytes of LDS, free again afterwards; NT threads.
+template <int BM, int NT>
+__device__ __forceinline__ bool row_tile(const int64_t* __restrict__ counts, int E, int tiles_j,
+                                          char* scratch, RowTile& t) {
+  int64_t* const wrow = reinterpret_cast<int64_t*>(scratch);
+  int64_t* const found_seg = wrow + NT / 64;
+  int* const wtile = reinterpret_cast<int*>(found_seg + 2);
+  int* const found = wtile + NT / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int per = (E + NT - 1) / NT;
+  int64_t r = 0;
+  int tl = 0;
+  for (int i = 0; i < per; ++i) {
+    const int e = tid * per + i;
+    const int64_t c = e < E ? counts[e] : 0;
+    r += c;
+    tl += (int)((c + BM - 1) / BM);
+  }
+  int64_t ri = r;
+  int ti = tl;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int64_t o = __shfl_up(ri, off, 64);
+    const int ot = __shfl_up(ti, off, 64);
+    if (lane >= off) {
+      ri += o;
+      ti += ot;
+    }
+  }
+  if (lane == 63) {
+    wrow[wave] = ri;
+    wtile[wave] = ti;
+  }
+  __syncthreads();
+  int64_t rb = 0;
+  int tb = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) {
+    if (w < wave) {
+      rb += wrow[w];
+      tb += wtile[w];
+    }
+    total += wtile[w];
+  }
+  rb += ri - r;
+  tb += ti - tl;
+  total *= tiles_j;
+  if ((int)blockIdx.x >= total) return false;
+  const int slot = xcd_remap(blockIdx.x, total);
+  if (slot >= tb * tiles_j && slot < (tb + tl) * tiles_j) {
+    for (int i = 0;; ++i) {
+      const int e = tid * per + i;
+      const int64_t c = counts[e];
+      const int m = (int)((c + BM - 1) / BM);
+      if (slot < (tb + m) * tiles_j) {
+        const int local = slot - tb * tiles_j;
+        found[0] = e;
+        found[1] = local % m;
+        found[2] = local / m;
+        found_seg[0] = rb;
+        found_seg[1] = c;
+        break;
+      }
+      rb += c;
+      tb += m;
+    }
+  }
+  __syncthreads();
+  t.e = __builtin_amdgcn_readfirstlane(found[0]);
+  t.mt = __builtin_amdgcn_readfirstlane(found[1]);
+  t.nt = __builtin_amdgcn_readfirstlane(found[2]);
+  t.seg0 = rfl64(found_seg[0]);
+  t.nrows = rfl64(found_seg[1]);
+  __syncthreads();  // the scratch is the first stage's memory
+  return true;
+}
+
 }  // namespace
 
 // fwd / dgrad for experts of few rows (gmm_thin.hip): operands as

@@ -28,91 +28,6 @@ constexpr int64_t T_CACHED = 128 << 20;
 constexpr int64_t T_ROWS64 = 40;
 constexpr int T_B = T_BN * T_BK * 2;  // weight tile (16 KiB)
 
-// What one block computes.
-struct ThinTile {
-  int e, mt, nt;
-  int64_t seg0, nrows;
-};
-
-// The block's (expert, row tile, column tile) from the per-expert counts:
-// consecutive slots, an expert's row tiles of one column tile first (they
-// share its weights), on one XCD. Returns false past the last slot.
-template <int BM>
-__device__ __forceinline__ bool thin_tile(const int64_t* __restrict__ counts, int E, int tiles_j,
-                                          char* scratch, ThinTile& t) {
-  int64_t* const wrow = reinterpret_cast<int64_t*>(scratch);
-  int64_t* const found_seg = wrow + T_NT / 64;
-  int* const wtile = reinterpret_cast<int*>(found_seg + 2);
-  int* const found = wtile + T_NT / 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int per = (E + T_NT - 1) / T_NT;
-  int64_t r = 0;
-  int tl = 0;
-  for (int i = 0; i < per; ++i) {
-    const int e = tid * per + i;
-    const int64_t c = e < E ? counts[e] : 0;
-    r += c;
-    tl += (int)((c + BM - 1) / BM);
-  }
-  int64_t ri = r;
-  int ti = tl;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int64_t o = __shfl_up(ri, off, 64);
-    const int ot = __shfl_up(ti, off, 64);
-    if (lane >= off) {
-      ri += o;
-      ti += ot;
-    }
-  }
-  if (lane == 63) {
-    wrow[wave] = ri;
-    wtile[wave] = ti;
-  }
-  __syncthreads();
-  int64_t rb = 0;
-  int tb = 0, total = 0;
-#pragma unroll
-  for (int w = 0; w < T_NT / 64; ++w) {
-    if (w < wave) {
-      rb += wrow[w];
-      tb += wtile[w];
-    }
-    total += wtile[w];
-  }
-  rb += ri - r;
-  tb += ti - tl;
-  total *= tiles_j;
-  if ((int)blockIdx.x >= total) return false;
-  const int slot = xcd_remap(blockIdx.x, total);
-  if (slot >= tb * tiles_j && slot < (tb + tl) * tiles_j) {
-    for (int i = 0;; ++i) {
-      const int e = tid * per + i;
-      const int64_t c = counts[e];
-      const int m = (int)((c + BM - 1) / BM);
-      if (slot < (tb + m) * tiles_j) {
-        const int local = slot - tb * tiles_j;
-        found[0] = e;
-        found[1] = local % m;
-        found[2] = local / m;
-        found_seg[0] = rb;
-        found_seg[1] = c;
-        break;
-      }
-      rb += c;
-      tb += m;
-    }
-  }
-  __syncthreads();
-  t.e = __builtin_amdgcn_readfirstlane(found[0]);
-  t.mt = __builtin_amdgcn_readfirstlane(found[1]);
-  t.nt = __builtin_amdgcn_readfirstlane(found[2]);
-  t.seg0 = rfl64(found_seg[0]);
-  t.nrows = rfl64(found_seg[1]);
-  __syncthreads();  // the scratch is the first stage's memory
-  return true;
-}
-
 // Epilogue: the BM x 128 tile row-major through LDS (256-byte rows, 16-byte
 // chunk c of row r in slot c ^ (r % 16)), stored as whole row segments.
 // Block mi, register 4g + e of lane l is row 32 mi + l % 32, column
@@ -162,8 +77,8 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin_kernel(
   constexpr int FM = BM / 32;           // 32-row blocks
   constexpr int LA = BM / 32, LD = 4 + LA;  // loads per wave and k-tile
   __shared__ __align__(16) char lds_raw[S * STAGE];
-  ThinTile t;
-  if (!thin_tile<BM>(counts, E, tiles_j, lds_raw, t)) return;
+  RowTile t;
+  if (!row_tile<BM, T_NT>(counts, E, tiles_j, lds_raw, t)) return;
   const int64_t R = MODE == MODE_FWD ? K : N, J = MODE == MODE_FWD ? N : K;
   const int64_t ldb = TRANS_B ? K : N;
   const int lane = threadIdx.x & 63;
@@ -326,8 +241,8 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin8_kernel(
   constexpr int FM = BM / 32;
   constexpr int LA = BM / 16, LD = 4 + LA;  // loads per wave and k-tile
   __shared__ __align__(16) char lds_raw[S * STAGE];
-  ThinTile t;
-  if (!thin_tile<BM>(counts, E, tiles_j, lds_raw, t)) return;
+  RowTile t;
+  if (!row_tile<BM, T_NT>(counts, E, tiles_j, lds_raw, t)) return;
   const int64_t R = FW ? K : N, J = FW ? N : K;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

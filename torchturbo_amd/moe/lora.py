@@ -26,7 +26,7 @@ from typing import Any, Optional, Union
 import torch
 import torch.nn as nn
 
-from ..dispatch import ops
+from ..dispatch import op_resolves, ops
 from .experts import GroupedMLP
 
 try:  # PEFT integration is optional (the reference requires it)
@@ -262,16 +262,18 @@ class GroupedMLPLoRA(nn.Module, _TunerBase):
             base.weight2.data -= d2.view_as(base.weight2)
 
     # -- forward --------------------------------------------------------------
-    def _residual(self, x, counts, names, a_group, b_group, out_dtype):
-        total = None
-        for name in names:
-            a, b = a_group[name], b_group[name]
-            xd = self.lora_dropout[name](x).to(a.weight.dtype)
-            delta = ops.grouped_matmul(ops.grouped_matmul(xd, a.weight, counts, trans_b=False),
-                                       b.weight, counts, trans_b=False)
-            term = delta.to(out_dtype) * self.scaling[name]
-            total = term if total is None else total + term
-        return total
+    def _add_residual(self, base, x, counts, name, a_group, b_group):
+        """``base`` plus adapter ``name``'s residual of ``x``."""
+        a, b = a_group[name], b_group[name]
+        xd, scale = self.lora_dropout[name](x), self.scaling[name]
+        if x.is_cuda and op_resolves("lora_residual"):
+            y = ops.lora_residual(base, xd, a.weight, b.weight, counts, scale)
+            if y is not None:
+                return y
+        xd = xd.to(a.weight.dtype)
+        delta = ops.grouped_matmul(ops.grouped_matmul(xd, a.weight, counts, trans_b=False),
+                                   b.weight, counts, trans_b=False)
+        return base + delta.to(base.dtype) * scale
 
     def forward(self, permuted_local_hidden_states: torch.Tensor,
                 tokens_per_expert: torch.Tensor, permuted_probs: torch.Tensor, **kwargs):
@@ -305,11 +307,11 @@ class GroupedMLPLoRA(nn.Module, _TunerBase):
         fc1 = ops.grouped_matmul(x, w1, counts, trans_b=False)
         # Each adapter's residual is added in turn, as the reference does.
         for name in active:
-            fc1 = fc1 + self._residual(x, counts, [name], self.lora_A, self.lora_B, fc1.dtype)
+            fc1 = self._add_residual(fc1, x, counts, name, self.lora_A, self.lora_B)
         act = base.activation_func_with_probs(fc1, probs.unsqueeze(-1))
         fc2 = ops.grouped_matmul(act, w2, counts, trans_b=False)
         for name in active:
-            fc2 = fc2 + self._residual(act, counts, [name], self.lora_A2, self.lora_B2, fc2.dtype)
+            fc2 = self._add_residual(fc2, act, counts, name, self.lora_A2, self.lora_B2)
         return fc2, None
 
     def __repr__(self) -> str:
