@@ -155,11 +155,22 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else c_void_p(t.data_ptr())
+    """Device address of ``t`` (NULL for None), as the ``c_void_p`` parameters take it."""
+    return None if t is None else t.data_ptr()
+
+
+# The current stream's handle without building a ``torch.cuda.Stream`` per
+# launch (about 5 us each): ``torch.cuda.current_stream`` where this build of
+# PyTorch does not have it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream(device: torch.device | None = None):
-    return c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """Handle of PyTorch's current HIP stream on ``device`` (default: the current device)."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if device is not None else None
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def route_index_workspace(num_tokens: int, num_experts: int) -> int:

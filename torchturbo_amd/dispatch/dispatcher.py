@@ -104,6 +104,9 @@ class OpDispatcher:
     def unresolved_ops(self) -> dict[str, str]:
         return dict(self._unresolved_ops)
 
+    def is_unresolved(self, op_name: str) -> bool:
+        return op_name in self._unresolved_ops
+
     # -- resolution --------------------------------------------------------
     def _resolve_all(self) -> None:
         """Resolve every op the device has providers for. Overrides are checked
@@ -296,12 +299,13 @@ class OpDispatcher:
     def __getattr__(self, name: str):
         if name.startswith("_"):
             raise AttributeError(name)
-        if not self.registry.list(lambda s: s.op_name == name):
+        if not self.registry.serves(name):
             raise AttributeError(name)
 
         def facade(*args: Any, impl: str | None = None, **kwargs: Any):
             return self._dispatch(name, *args, impl=impl, **kwargs)
 
+        self.__dict__[name] = facade  # it resolves per call; only the lookup is kept
         return facade
 
 

@@ -66,7 +66,7 @@ def op_resolves(name: str) -> bool:
         d = get_ops()
     except RuntimeError:
         return False
-    return bool(d.registry.list(lambda s: s.op_name == name)) and name not in d.unresolved_ops
+    return d.registry.serves(name) and not d.is_unresolved(name)
 
 
 def reset_ops() -> None:

@@ -47,6 +47,10 @@ class OpRegistry:
         # sorted() is stable, also with reverse=True: ties stay in table order
         return sorted((s for s in self._table.values() if keep(s)), key=_rank, reverse=True)
 
+    def serves(self, op_name: str) -> bool:
+        """Whether any registered spec implements ``op_name``."""
+        return any(s.op_name == op_name for s in self._table.values())
+
     def get_by_impl_name(self, impl_name: str) -> OpSpec:
         try:
             return self._table[impl_name]

@@ -221,11 +221,13 @@ class TopKRouter(Router):
             local = (~padding_mask.reshape(-1).bool()).sum()
             local_z = z_sum.to(logits.dtype) / torch.clamp(local, min=1)
         else:
-            local = torch.tensor(logits.shape[0], device=logits.device, dtype=torch.long)
+            # filled on the device: a tensor made from the host's number waits for the copy
+            local = torch.full((), logits.shape[0], device=logits.device, dtype=torch.long)
             local_z = (z_sum / max(logits.shape[0], 1)).to(logits.dtype)
-        total = local.clone()
+        total = local
         sp_size = _group_size(self.sp_group)
         if sp_size > 1:
+            total = local.clone()
             dist.all_reduce(total, op=dist.ReduceOp.SUM, group=self.sp_group)
         z = local_z * coeff * (sp_size * local / torch.clamp(total, min=1))
         self._metrics = {**(self._metrics or {}), "z_loss": (z / coeff).detach(),
