@@ -360,6 +360,22 @@ int tt_lora_wgrad(const void* in, const float* v, int dtype, int64_t m, int64_t 
                   int32_t transposed, float scale, int32_t num_experts, const int64_t* counts,
                   float* out, void* stream);
 
+/* The experts' forward without gradients in one call (moe_layer.py:149-183 from
+ * the routing on): routing index, fc1 over the tokens' rows, gate with the
+ * probabilities (act -1: SwiGLU as tt_swiglu_fwd, else as tt_gated_act_fwd),
+ * fc2 and the sum of each token's rows. 16-bit weights w1 [E, H, 2F], w2
+ * [E, F, H], or e4m3 [E, 2F, H], [E, H, F] with block scales (scale1, scale2).
+ * Equal to the separate entry points bit for bit. tokens_per_expert [E] is
+ * written; workspace: tt_moe_experts_workspace bytes, 16-byte aligned. */
+size_t tt_moe_experts_workspace(int64_t num_tokens, int32_t topk, int32_t num_experts,
+                                int64_t hidden, int64_t ffn);
+int tt_moe_experts_fwd(const void* x, int dtype, int64_t num_tokens, int64_t hidden,
+                       const int64_t* expert_indices, const void* probs, int probs_dtype,
+                       int32_t topk, int32_t num_experts, const void* w1, const void* w2,
+                       const void* scale1, const void* scale2, int scale_dtype, int64_t ffn,
+                       int act, float limit, int clamp_after, int64_t* tokens_per_expert,
+                       void* out, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

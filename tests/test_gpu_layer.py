@@ -332,3 +332,66 @@ def test_fp8_requantize_equals_torch_composition(process_ops, scale_dtype, hidde
             torch.int16 if ref.dtype == torch.bfloat16 else torch.int32)
         assert torch.equal(got.view(bits)[~nan], ref.view(bits)[~nan])
         assert got._version > v  # a backward that saved the old values is refused
+
+
+@pytest.mark.parametrize("tokens", [1, 33, 200, 1500])
+@pytest.mark.parametrize("kind", ["silu", "gelu", "capped", "f16", "fp8"])
+def test_inference_forward_equals_the_separate_ops(process_ops, kind, tokens):
+    """The experts' forward in one call (no gradients) against the separate ops, which a forward
+    hook on the experts keeps: output, logits and counts bit for bit, over row counts that take
+    the gathering few-row kernels (both tile heights) and the permuted path."""
+    process_ops(CudaRuntime(), OpPolicy.CUSTOM)
+    fp8 = kind == "fp8"
+    dtype = torch.float16 if kind == "f16" else torch.bfloat16
+    E, H, Fd = 32, 256, 128
+    cfg = MoEConfig(hidden_size=H, num_moe_experts=E, moe_ffn_hidden_size=Fd, gated_linear_unit=True,
+                    activation_func=F.gelu if kind == "gelu" else F.silu, moe_router_topk=4,
+                    moe_router_dtype="fp32", params_dtype=dtype,
+                    moe_swiglu_limit=[0.3] if kind == "capped" else None)
+    experts = Fp8GroupedMLP if fp8 else GroupedMLP
+    layer = MoELayer(cfg, None, layer_number=0,
+                     submodules=MoESubmodules(experts=ModuleSpec(module=experts))).to(DEV)
+    g = torch.Generator().manual_seed(tokens)
+    with torch.no_grad():
+        layer.router.weight.copy_(torch.randn(E, H, generator=g) * 0.05)
+        if fp8:
+            for m in (layer.experts.master1, layer.experts.master2):
+                m.copy_(torch.randn(m.shape, generator=g) * 0.05)
+            layer.experts.requantize()
+        else:
+            for p in (layer.experts.weight1, layer.experts.weight2):
+                p.copy_(torch.randn(p.shape, generator=g) * 0.05)
+    x = torch.randn(tokens, H, generator=g).to(dtype).to(DEV)
+    from torchturbo_amd import _lib
+    calls = []
+    real = _lib.call
+
+    def spy(name, *args):
+        calls.append(name)
+        return real(name, *args)
+
+    _lib.call = spy
+    try:
+        with torch.no_grad():
+            out, logits = layer(x)
+            counts = layer.token_dispatcher.tokens_per_expert
+        assert "tt_moe_experts_fwd" in calls and "tt_permute_scatter" not in calls
+        calls.clear()
+        hook = layer.experts.register_forward_hook(lambda *a: None)
+        with torch.no_grad():
+            ref, ref_logits = layer(x)
+        hook.remove()
+        assert "tt_moe_experts_fwd" not in calls and "tt_permute_scatter" in calls
+        calls.clear()
+        layer(x)  # gradients are on
+        assert "tt_moe_experts_fwd" not in calls
+    finally:
+        _lib.call = real
+    assert torch.equal(out, ref) and torch.equal(logits, ref_logits)
+    assert torch.equal(counts, layer.token_dispatcher.tokens_per_expert)
+    # an unaligned source is permuted into aligned rows first, as before
+    flat = torch.zeros(tokens * H + 1, dtype=dtype, device=DEV)[1:]
+    flat.copy_(x.view(-1))
+    with torch.no_grad():
+        assert torch.equal(layer.forward_with_logits(flat.view(tokens, H), logits),
+                           layer.forward_with_logits(x, logits))

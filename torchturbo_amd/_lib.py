@@ -63,13 +63,17 @@ _PROTOS: dict[str, list] = {
     "tt_gmm_wgrad_persistent": [c_int, I64, I64, I64, I32, I32],
     "tt_gmm_fp8_fwd": [P, P, P, c_int, I64, I64, I64, I32, P, P, P],
     "tt_gmm_fp8_dgrad": [P, P, P, c_int, I64, I64, I64, I32, P, P, P],
+    "tt_moe_experts_workspace": [I64, I32, I32, I64, I64],
+    "tt_moe_experts_fwd": [P, c_int, I64, I64, P, P, c_int, I32, I32, P, P, P, P, c_int, I64, c_int,
+                           c_float, c_int, P, P, P, c_size_t, P],
     "tt_lora_down": [P, P, c_int, I64, I64, I32, I32, c_float, I32, P, P, P],
     "tt_lora_up": [P, P, P, c_int, I64, I64, I32, I32, c_float, I32, P, P, P],
     "tt_lora_wgrad": [P, P, c_int, I64, I64, I32, I32, c_float, I32, P, P, P],
     "tt_fp8_quantize_blocks": [P, c_int, I64, I64, I64, P, P, c_int, P],
 }
 _RESTYPES = {"tt_last_error": ctypes.c_char_p, "tt_route_index_workspace": c_size_t,
-             "tt_route_index_rejected_offset": c_size_t, "tt_router_loss_workspace": c_size_t}
+             "tt_route_index_rejected_offset": c_size_t, "tt_router_loss_workspace": c_size_t,
+             "tt_moe_experts_workspace": c_size_t}
 ABI_VERSION = 1
 
 _LIB: ctypes.CDLL | None = None

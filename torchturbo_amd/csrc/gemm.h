@@ -267,16 +267,26 @@ __device__ __forceinline__ bool row_tile(const int64_t* __restrict__ counts, int
 }  // namespace
 
 // fwd / dgrad for experts of few rows (gmm_thin.hip): operands as
-// tt_gmm_fwd / tt_gmm_dgrad, already checked; see thin_rows in gmm.hip.
+// tt_gmm_fwd / tt_gmm_dgrad, already checked; see thin_rows in gmm.hip. With
+// arow, activation row r is row arow[r] of p0 (src_rows rows, under 2 GiB).
 int tt_gmm_thin(int mode, bool tb, int dtype, const void* p0, const void* p1, void* out,
-                int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s);
+                int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s,
+                const int32_t* arow = nullptr, int64_t src_rows = 0);
 // The same with e4m3 weights and block scales, as tt_gmm_fp8_fwd / _dgrad, at
 // most TT_THIN8_SCALES scale blocks along the reduction; see thin8_rows in
 // gmm.hip.
 #define TT_THIN8_SCALES 128
 int tt_gmm_thin8(int mode, const void* p0, const uint8_t* qw, const void* scale, int sdt,
                  void* out, int64_t M, int64_t K, int64_t N, int E, const int64_t* counts,
-                 hipStream_t s);
+                 hipStream_t s, const int32_t* arow = nullptr, int64_t src_rows = 0);
+
+// fc1 of a forward over few rows with the token rows gathered (gmm.hip): 1
+// when the launch was made, 0 when the shape takes another kernel (the caller
+// permutes), or an error. scale (with its dtype) for e4m3 weights [E, N, K],
+// else w is 16-bit [E, K, N].
+int tt_gmm_rows_fwd(const void* x, int64_t src_rows, const int32_t* arow, const void* w,
+                    const void* scale, int sdt, int dtype, int64_t M, int64_t K, int64_t N, int E,
+                    const int64_t* counts, void* y, hipStream_t s);
 
 // Router logits of few tokens (gate.hip): logits [T, E] = x [T, H] w [E, H]^T
 // in 16 bits (dtype), E a multiple of 32, H of 64; ldt is TT_F32 or dtype.

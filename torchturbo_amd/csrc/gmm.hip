@@ -2599,6 +2599,11 @@ int launch_p64_k(const void* p0, const void* p1, void* out, int64_t M, int64_t K
 // 54 + 37 / 50 + 24 + 39 + 26 us, at 144 66 + 31 + 52 + 35 / 63 + 35 + 60 + 41.
 constexpr int64_t THIN_ROWS = 96;
 bool thin_rows(int64_t M, int E) { return M <= (int64_t)E * THIN_ROWS; }
+// Whether fwd / dgrad (reduction R) take it, for a problem within the limits
+// of launch_mfma.
+bool thin_takes(int64_t M, int64_t K, int64_t N, int64_t R, int E) {
+  return thin_rows(M, E) && (R + 2 * P_BK) * (K > N ? K : N) * 2 < (int64_t)DM_OOB;
+}
 
 template <int MODE, bool TB, int ET>
 int launch_mfma(const void* p0, const void* p1, void* out, int64_t M, int64_t K, int64_t N,
@@ -2619,7 +2624,7 @@ int launch_mfma(const void* p0, const void* p1, void* out, int64_t M, int64_t K,
   const int64_t R = MODE == MODE_FWD ? K : N;  // reduction length of fwd / dgrad
   const bool p64_lds = p64_lds_bytes(E) <= 160 * 1024;
   if constexpr (MODE != MODE_WGRAD) {
-    if (thin_rows(M, E) && (R + 2 * P_BK) * ld * 2 < (int64_t)DM_OOB)
+    if (thin_takes(M, K, N, R, E))
       return tt_gmm_thin(MODE, TB, ET, p0, p1, out, M, K, N, E, counts, s);
     // The persistent kernel needs two k-tiles per output tile, its LDS
     // (stages, epilogue staging, schedule) and 32-bit offsets for loads that
@@ -2751,6 +2756,10 @@ int launch_q8_k(const void* p0, const uint8_t* qw, const void* scale, int sdt, v
 // 1081 and 1693 + 863 / 2100 + 1047.
 constexpr int64_t THIN8_ROWS = 40;
 bool thin8_rows(int64_t M, int E) { return M <= (int64_t)E * THIN8_ROWS; }
+bool thin8_takes(int64_t M, int64_t K, int64_t N, int64_t R, int E) {
+  return thin8_rows(M, E) && (R + 127) / 128 <= TT_THIN8_SCALES &&
+         (M + DM_BM) * R * 2 < (int64_t)DM_OOB && (N + 2 * Q_BK + Q_BN) * K < (int64_t)DM_OOB;
+}
 
 template <int MODE>
 int launch_fp8(const void* p0, const uint8_t* qw, const void* scale, int sdt, void* out, int64_t M,
@@ -2765,8 +2774,7 @@ int launch_fp8(const void* p0, const uint8_t* qw, const void* scale, int sdt, vo
     const int tjq = (int)((J + Q_BN - 1) / Q_BN);
     const int64_t nq = ((M + Q_BM - 1) / Q_BM + E) * (int64_t)tjq;
     if (nq == 0) return TT_OK;
-    if (thin8_rows(M, E) && (R + 127) / 128 <= TT_THIN8_SCALES &&
-        (M + DM_BM) * lda * 2 < (int64_t)DM_OOB && (N + 2 * Q_BK + Q_BN) * K < (int64_t)DM_OOB)
+    if (thin8_takes(M, K, N, R, E))
       return tt_gmm_thin8(MODE, p0, qw, scale, sdt, out, M, K, N, E, counts, s);
     if (R > Q_BK && (R + 127) / 128 <= Q_SMAX &&
         schedule_bytes(E) + 2 * Q_STAGE + 4 * P_EPI + 4 * Q_SMAX * sizeof(float) + 64 <=
@@ -2946,6 +2954,31 @@ extern "C" int tt_gmm_fp8_dgrad(const void* dy, const uint8_t* qw, const void* s
   if (rc != TT_OK) return rc;
   return launch_fp8<MODE_DGRAD>(dy, qw, scale, scale_dtype, dx, m, k, n, num_experts, counts,
                                S(stream));
+}
+
+int tt_gmm_rows_fwd(const void* x, int64_t src_rows, const int32_t* arow, const void* w,
+                    const void* scale, int sdt, int dtype, int64_t M, int64_t K, int64_t N, int E,
+                    const int64_t* counts, void* y, hipStream_t s) {
+  // Operands that the launchers refuse go to them, so that they say why; rows
+  // of an unaligned source are permuted into aligned ones.
+  if (M == 0 || K % 16 || N % 16 || E < 1 || E > 4096 ||
+      src_rows * K * 2 >= (int64_t)GA_NOROW ||
+      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+        reinterpret_cast<uintptr_t>(y)) & 15) != 0)
+    return 0;
+  int rc = TT_OK;
+  if (scale != nullptr) {
+    if (!thin8_takes(M, K, N, K, E)) return 0;
+    rc = tt_gmm_thin8(MODE_FWD, x, static_cast<const uint8_t*>(w), scale, sdt, y, M, K, N, E,
+                      counts, s, arow, src_rows);
+  } else {
+    const int64_t ld = K > N ? K : N;
+    if (!thin_takes(M, K, N, K, E) || (M + DM_BM) * ld * 2 >= (int64_t)DM_OOB ||
+        K * N * 2 >= (int64_t)DM_OOB)
+      return 0;
+    rc = tt_gmm_thin(MODE_FWD, false, dtype, x, w, y, M, K, N, E, counts, s, arow, src_rows);
+  }
+  return rc == TT_OK ? 1 : rc;
 }
 
 extern "C" int tt_gmm_gather_supported(int32_t op, int dtype, int64_t src_rows, int64_t m,

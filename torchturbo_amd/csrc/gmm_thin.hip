@@ -28,6 +28,21 @@ constexpr int64_t T_CACHED = 128 << 20;
 constexpr int64_t T_ROWS64 = 40;
 constexpr int T_B = T_BN * T_BK * 2;  // weight tile (16 KiB)
 
+// Byte offset of row r of a tile (first packed row `at`, `rows` valid): from
+// the tile's first row, or, with rows gathered through arow, in the source
+// [src_rows, R]. Gathered rows past the expert's end, or out of the source,
+// read as zeros: T_NOROW and a lane's chunk lie past any resource (sources are
+// smaller than 2 GiB), as rows past the packed tile's resource do.
+constexpr uint32_t T_NOROW = 0x80000000u;
+__device__ __forceinline__ uint32_t thin_row_offset(const int32_t* __restrict__ arow, int64_t at,
+                                                    int r, int64_t rows, int64_t src_rows,
+                                                    int64_t R) {
+  if (arow == nullptr) return (uint32_t)(r * R * 2);
+  if (r >= rows) return T_NOROW;
+  const uint32_t v = (uint32_t)arow[at + r];
+  return v < (uint64_t)src_rows ? (uint32_t)(v * R * 2) : T_NOROW;
+}
+
 // Epilogue: the BM x 128 tile row-major through LDS (256-byte rows, 16-byte
 // chunk c of row r in slot c ^ (r % 16)), stored as whole row segments.
 // Block mi, register 4g + e of lane l is row 32 mi + l % 32, column
@@ -71,7 +86,8 @@ __device__ __forceinline__ void thin_store(const f32x16 (&acc)[BM / 32], char* o
 template <int MODE, bool TRANS_B, int ET, bool KMASK, int BM, int S, int OCC>
 __global__ __launch_bounds__(T_NT, OCC) void gmm_thin_kernel(
     const char* __restrict__ p0, const char* __restrict__ p1, char* __restrict__ out, int64_t K,
-    int64_t N, int E, const int64_t* __restrict__ counts, int tiles_j, int stream) {
+    int64_t N, int E, const int64_t* __restrict__ counts, int tiles_j, int stream,
+    const int32_t* __restrict__ arow, int64_t src_rows) {
   constexpr bool B_K = Layout<MODE, TRANS_B>::B_K;
   constexpr int T_A = BM * T_BK * 2, STAGE = T_A + T_B;
   constexpr int FM = BM / 32;           // 32-row blocks
@@ -91,7 +107,9 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin_kernel(
   const bool once = stream && t.nrows <= BM;
 
   // Resources at the tile origin, advanced by a k-tile at a time.
-  const i32x4 ra = make_rsrc(p0 + (t.seg0 + i0) * R * 2, (rows < BM ? rows : BM) * R * 2);
+  const i32x4 ra = arow != nullptr
+                       ? make_rsrc(p0, src_rows * R * 2)
+                       : make_rsrc(p0 + (t.seg0 + i0) * R * 2, (rows < BM ? rows : BM) * R * 2);
   const char* wb = p1 + (int64_t)t.e * K * N * 2;
   const int64_t boff = B_K ? j0 * ldb * 2 : j0 * 2;
   const i32x4 rb = make_rsrc(wb + boff, K * N * 2 - boff);
@@ -108,7 +126,7 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin_kernel(
     const int r = 8 * LA * wave + 8 * q + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
     akof[q] = 8 * c;
-    aoff[q] = (uint32_t)((r * R + 8 * c) * 2);
+    aoff[q] = thin_row_offset(arow, t.seg0 + i0, r, rows, src_rows, R) + (uint32_t)(16 * c);
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -235,7 +253,8 @@ template <int MODE, bool KMASK, int BM, int S, int OCC>
 __global__ __launch_bounds__(T_NT, OCC) void gmm_thin8_kernel(
     const char* __restrict__ p0, const char* __restrict__ qw, const char* __restrict__ scale,
     int sdt, char* __restrict__ out, int64_t K, int64_t N, int E,
-    const int64_t* __restrict__ counts, int tiles_j, int stream) {
+    const int64_t* __restrict__ counts, int tiles_j, int stream,
+    const int32_t* __restrict__ arow, int64_t src_rows) {
   constexpr bool FW = MODE == MODE_FWD;
   constexpr int T_A = BM * T8_BK * 2, STAGE = T_A + T_B;
   constexpr int FM = BM / 32;
@@ -250,7 +269,9 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin8_kernel(
   const int64_t i0 = (int64_t)t.mt * BM, j0 = (int64_t)t.nt * T_BN;
   const int64_t rows = t.nrows - i0;
   const bool once = stream && t.nrows <= BM;
-  const i32x4 ra = make_rsrc(p0 + (t.seg0 + i0) * R * 2, (rows < BM ? rows : BM) * R * 2);
+  const i32x4 ra = arow != nullptr
+                       ? make_rsrc(p0, src_rows * R * 2)
+                       : make_rsrc(p0 + (t.seg0 + i0) * R * 2, (rows < BM ? rows : BM) * R * 2);
   const int64_t boff = FW ? j0 * K : j0;
   const i32x4 rb = make_rsrc(qw + (int64_t)t.e * K * N + boff, K * N - boff);
   const uint32_t ks_b = FW ? (uint32_t)T8_BK : (uint32_t)(T8_BK * K);
@@ -267,7 +288,7 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin8_kernel(
     const int r = (BM / 4) * wave + 8 * (q % (LA / 2)) + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
     akof[q] = 64 * (q / (LA / 2)) + 8 * c;
-    aoff[q] = (uint32_t)((r * R + akof[q]) * 2);
+    aoff[q] = thin_row_offset(arow, t.seg0 + i0, r, rows, src_rows, R) + (uint32_t)(2 * akof[q]);
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -387,7 +408,8 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin8_kernel(
 
 template <int MODE, bool TB, int ET, bool KMASK, int BM, int S, int OCC>
 int launch_thin_k(const void* p0, const void* p1, void* out, int64_t M, int64_t K, int64_t N,
-                  int E, const int64_t* counts, hipStream_t s) {
+                  int E, const int64_t* counts, hipStream_t s, const int32_t* arow,
+                  int64_t src_rows) {
   const int64_t J = MODE == MODE_FWD ? N : K;
   const int tj = (int)((J + T_BN - 1) / T_BN);
   // Each used expert adds at most one partial row tile.
@@ -398,7 +420,7 @@ int launch_thin_k(const void* p0, const void* p1, void* out, int64_t M, int64_t 
   hipLaunchKernelGGL((gmm_thin_kernel<MODE, TB, ET, KMASK, BM, S, OCC>), dim3((unsigned)nblk),
                      dim3(T_NT), 0, s, static_cast<const char*>(p0),
                      static_cast<const char*>(p1), static_cast<char*>(out), K, N, E, counts, tj,
-                     stream);
+                     stream, arow, src_rows);
   return tt_check_launch("gmm");
 }
 
@@ -406,21 +428,27 @@ int launch_thin_k(const void* p0, const void* p1, void* out, int64_t M, int64_t 
 // rows per expert, 128-row tiles (64 KiB, two stages) above.
 template <int MODE, bool TB, int ET>
 int launch_thin(const void* p0, const void* p1, void* out, int64_t M, int64_t K, int64_t N,
-                int E, const int64_t* counts, hipStream_t s) {
+                int E, const int64_t* counts, hipStream_t s, const int32_t* arow,
+                int64_t src_rows) {
   const int64_t R = MODE == MODE_FWD ? K : N;
   if (M <= (int64_t)E * T_ROWS64) {
     if (R % T_BK)
-      return launch_thin_k<MODE, TB, ET, true, 64, 3, 2>(p0, p1, out, M, K, N, E, counts, s);
-    return launch_thin_k<MODE, TB, ET, false, 64, 3, 2>(p0, p1, out, M, K, N, E, counts, s);
+      return launch_thin_k<MODE, TB, ET, true, 64, 3, 2>(p0, p1, out, M, K, N, E, counts, s, arow,
+                                                              src_rows);
+    return launch_thin_k<MODE, TB, ET, false, 64, 3, 2>(p0, p1, out, M, K, N, E, counts, s, arow,
+                                                              src_rows);
   }
   if (R % T_BK)
-    return launch_thin_k<MODE, TB, ET, true, 128, 2, 2>(p0, p1, out, M, K, N, E, counts, s);
-  return launch_thin_k<MODE, TB, ET, false, 128, 2, 2>(p0, p1, out, M, K, N, E, counts, s);
+    return launch_thin_k<MODE, TB, ET, true, 128, 2, 2>(p0, p1, out, M, K, N, E, counts, s, arow,
+                                                              src_rows);
+  return launch_thin_k<MODE, TB, ET, false, 128, 2, 2>(p0, p1, out, M, K, N, E, counts, s, arow,
+                                                              src_rows);
 }
 
 template <int MODE, bool KMASK, int BM, int S>
 int launch_thin8_k(const void* p0, const uint8_t* qw, const void* scale, int sdt, void* out,
-                   int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s) {
+                   int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s,
+                   const int32_t* arow, int64_t src_rows) {
   const int64_t J = MODE == MODE_FWD ? N : K;
   const int tj = (int)((J + T_BN - 1) / T_BN);
   const int64_t nblk = (M / BM + (M < E ? M : E)) * tj;
@@ -430,39 +458,45 @@ int launch_thin8_k(const void* p0, const uint8_t* qw, const void* scale, int sdt
   hipLaunchKernelGGL((gmm_thin8_kernel<MODE, KMASK, BM, S, 2>), dim3((unsigned)nblk), dim3(T_NT),
                      0, s, static_cast<const char*>(p0), reinterpret_cast<const char*>(qw),
                      static_cast<const char*>(scale), sdt, static_cast<char*>(out), K, N, E,
-                     counts, tj, stream);
+                     counts, tj, stream, arow, src_rows);
   return tt_check_launch("gmm_fp8");
 }
 
 template <int MODE>
 int launch_thin8(const void* p0, const uint8_t* qw, const void* scale, int sdt, void* out,
-                 int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s) {
+                 int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s,
+                 const int32_t* arow, int64_t src_rows) {
   const int64_t R = MODE == MODE_FWD ? K : N;
   if (M <= (int64_t)E * T8_ROWS32) {
     if (R % T8_BK)
-      return launch_thin8_k<MODE, true, 32, 3>(p0, qw, scale, sdt, out, M, K, N, E, counts, s);
-    return launch_thin8_k<MODE, false, 32, 3>(p0, qw, scale, sdt, out, M, K, N, E, counts, s);
+      return launch_thin8_k<MODE, true, 32, 3>(p0, qw, scale, sdt, out, M, K, N, E, counts, s, arow,
+                                              src_rows);
+    return launch_thin8_k<MODE, false, 32, 3>(p0, qw, scale, sdt, out, M, K, N, E, counts, s, arow,
+                                              src_rows);
   }
   if (R % T8_BK)
-    return launch_thin8_k<MODE, true, 64, 2>(p0, qw, scale, sdt, out, M, K, N, E, counts, s);
-  return launch_thin8_k<MODE, false, 64, 2>(p0, qw, scale, sdt, out, M, K, N, E, counts, s);
+    return launch_thin8_k<MODE, true, 64, 2>(p0, qw, scale, sdt, out, M, K, N, E, counts, s, arow,
+                                              src_rows);
+  return launch_thin8_k<MODE, false, 64, 2>(p0, qw, scale, sdt, out, M, K, N, E, counts, s, arow,
+                                              src_rows);
 }
 
 }  // namespace
 
 int tt_gmm_thin8(int mode, const void* p0, const uint8_t* qw, const void* scale, int sdt,
                  void* out, int64_t M, int64_t K, int64_t N, int E, const int64_t* counts,
-                 hipStream_t s) {
+                 hipStream_t s, const int32_t* arow, int64_t src_rows) {
   if (mode == MODE_FWD)
-    return launch_thin8<MODE_FWD>(p0, qw, scale, sdt, out, M, K, N, E, counts, s);
-  return launch_thin8<MODE_DGRAD>(p0, qw, scale, sdt, out, M, K, N, E, counts, s);
+    return launch_thin8<MODE_FWD>(p0, qw, scale, sdt, out, M, K, N, E, counts, s, arow, src_rows);
+  return launch_thin8<MODE_DGRAD>(p0, qw, scale, sdt, out, M, K, N, E, counts, s, arow, src_rows);
 }
 
 int tt_gmm_thin(int mode, bool tb, int dtype, const void* p0, const void* p1, void* out,
-                int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s) {
+                int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s,
+                const int32_t* arow, int64_t src_rows) {
   auto go = [&](auto mode_c, auto tb_c, auto et_c) {
     return launch_thin<decltype(mode_c)::value, decltype(tb_c)::value, decltype(et_c)::value>(
-        p0, p1, out, M, K, N, E, counts, s);
+        p0, p1, out, M, K, N, E, counts, s, arow, src_rows);
   };
   using FW = std::integral_constant<int, MODE_FWD>;
   using DG = std::integral_constant<int, MODE_DGRAD>;

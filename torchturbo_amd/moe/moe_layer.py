@@ -17,7 +17,7 @@ import torch.distributed as dist
 import torch.nn.functional as F
 
 from ..dispatch import ops
-from .experts import GroupedMLP
+from .experts import Fp8GroupedMLP, GroupedMLP
 from .module import ModuleSpec, build_module
 from .moe_config import MoEConfig
 from .router import TopKRouter
@@ -106,6 +106,47 @@ class MoELayer(BaseMoELayer):
         return fused_experts.eligible(tokens, self.experts.weight1, expert_indices.shape[1],
                                       self.num_local_experts)
 
+    def _inference_experts(self, tokens, probs, expert_indices):
+        """The experts' output for a small batch without gradients, in one native call where
+        the HIP providers serve the ops it stands for (the conditions are in
+        ``providers.hip.fused_experts.inference_eligible``); None otherwise."""
+        if torch.is_grad_enabled() or not tokens.is_cuda:
+            return None
+        e = self.experts
+        fp8 = type(e) is Fp8GroupedMLP
+        if not fp8 and (type(e) is not GroupedMLP or not self.config.gated_linear_unit
+                        or self.config.moe_apply_probs_on_input):
+            return None
+        if type(self.token_dispatcher) is not MoEAlltoAllTokenDispatcher:
+            return None
+        plain = fp8 or e._fused_swiglu
+        wanted = (("moe_permutation", "hip_moe_mask_permutation"),
+                  ("grouped_matmul_fp8", "hip_grouped_matmul_fp8") if fp8 else
+                  ("grouped_matmul", "hip_grouped_matmul"),
+                  ("swiglu_probs", "hip_swiglu_probs") if plain else
+                  ("gated_activation_probs", "hip_gated_activation_probs"),
+                  ("moe_unpermutation", "hip_moe_mask_unpermutation"))
+        try:
+            if any(ops.selected_impl_name(op) != impl for op, impl in wanted):
+                return None
+        except RuntimeError:
+            return None
+        from ..providers.hip import fused_experts
+        weights = (e.q1, e.q2) if fp8 else (e.weight1, e.weight2)
+        scales = (e.s1, e.s2) if fp8 else None
+        if not fused_experts.inference_eligible(e, weights, scales, tokens, probs, expert_indices):
+            return None
+        cfg = self.config
+        output, counts = fused_experts.experts_forward(
+            tokens, probs, expert_indices, self.num_local_experts, cfg.moe_ffn_hidden_size,
+            weights, scales, F.silu if fp8 else cfg.activation_func,
+            0.0 if fp8 else e.swiglu_limit,
+            False if fp8 else cfg.moe_swiglu_clamp_gate_after_activation)
+        d = self.token_dispatcher
+        d.tokens_per_expert = counts
+        d.hidden_shape = d.hidden_shape_before_permute = tokens.shape
+        return output
+
     def _experts_and_combine(self, hidden_states, probs, routing_map, expert_indices):
         flat = hidden_states.view(-1, hidden_states.shape[-1])
         if self._gathering_experts(flat, expert_indices):
@@ -117,7 +158,12 @@ class MoELayer(BaseMoELayer):
             self.token_dispatcher.tokens_per_expert = counts
             output = tokens.view(hidden_states.shape).to(hidden_states.dtype)
         else:
-            output = self._dispatched_experts(hidden_states, probs, routing_map, expert_indices)
+            output = self._inference_experts(flat, probs, expert_indices)
+            if output is not None:
+                output = output.view(hidden_states.shape)
+            else:
+                output = self._dispatched_experts(hidden_states, probs, routing_map,
+                                                  expert_indices)
         if self.shared_expert is not None:
             shared = self.shared_expert(hidden_states)
             output = output + F.sigmoid(self.shared_expert_gate(hidden_states)) * shared

@@ -28,6 +28,8 @@ import os
 
 import torch
 
+import torch.nn.functional as F
+
 from ... import _lib as L
 from ... import checks
 from ._functions import route_index
@@ -216,3 +218,74 @@ def grouped_mlp_tokens(experts, tokens, probs, routing_map, expert_indices):
     fc1 = GatherGroupedMatmul.apply(tokens, w1, counts, rows, token_of_row, False)
     act = experts.activation_func_with_probs(fc1, pprobs)
     return GroupedMatmulCombine.apply(act, w2, counts, rows, token_of_row, False), counts
+
+
+# ---------------------------------------------------------------------------
+# Forward without gradients, in one call
+# ---------------------------------------------------------------------------
+# Up to this many routed rows the experts' forward without gradients is one
+# native call (decode, short prefill): the host's work of six separate ops
+# (about 100 us) is then what a call costs. Its scratch, one allocation, holds
+# all intermediates at once, which larger batches would rather not.
+MAX_INFERENCE_ROWS = 32768
+
+
+def _plain(t, dtypes) -> bool:
+    return type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype in dtypes and t.is_contiguous()
+
+
+def _hooked(module) -> bool:
+    m = torch.nn.modules.module
+    return bool(module._forward_hooks or module._forward_pre_hooks or m._global_forward_hooks
+                or m._global_forward_pre_hooks or "forward" in module.__dict__)
+
+
+def inference_eligible(experts, weights, scales, tokens, probs, expert_indices) -> bool:
+    """Whether ``experts_forward`` stands in for permute -> ``experts`` -> unpermute: no
+    gradients, tangents, function transforms or tracing that the separate ops' autograd
+    functions would have to see, no hooks on the experts, plain contiguous 16-bit tensors
+    on one device, and no input checks asked for."""
+    if (torch.is_grad_enabled() or checks.enabled() or torch.compiler.is_compiling()
+            or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0 or _hooked(experts)):
+        return False
+    if expert_indices is None or tokens.dim() != 2 or expert_indices.dim() != 2:
+        return False
+    T, k = expert_indices.shape
+    if not 0 < T * k <= MAX_INFERENCE_ROWS or tokens.shape[0] != T or probs.shape[0] != T:
+        return False
+    half = (torch.bfloat16, torch.float16)
+    if not (_plain(tokens, half) and _plain(probs, (torch.float32, *half))
+            and _plain(expert_indices, (torch.int64,))):
+        return False
+    if scales is None:
+        if not all(_plain(w, (tokens.dtype,)) for w in weights):
+            return False
+    elif not (tokens.dtype == torch.bfloat16
+              and all(_plain(w, (torch.float8_e4m3fn,)) for w in weights)
+              and all(_plain(s, (torch.bfloat16, torch.float32)) for s in scales)
+              and scales[0].dtype == scales[1].dtype):
+        return False
+    dev = tokens.device
+    return all(t.device == dev for t in (probs, expert_indices, *weights, *(scales or ())))
+
+
+def experts_forward(tokens, probs, expert_indices, num_experts, ffn, weights, scales=None,
+                    activation_func=F.silu, limit=0.0, clamp_after=False):
+    """(output [T, H], per-expert counts) of the experts for the routed tokens, without
+    gradients (``tt_moe_experts_fwd``); the values of the separate ops bit for bit."""
+    T, H = tokens.shape
+    k = expert_indices.shape[1]
+    dev = tokens.device
+    out = torch.empty_like(tokens)
+    counts = torch.empty((num_experts,), dtype=torch.int64, device=dev)
+    nbytes = L.load().tt_moe_experts_workspace(T, k, num_experts, H, ffn)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev)
+    act = -1 if activation_func is F.silu and limit == 0.0 else int(activation_func is F.gelu)
+    s1, s2 = scales or (None, None)
+    L.call("tt_moe_experts_fwd", L.ptr(tokens), L.dtype_code(tokens.dtype), T, H,
+           L.ptr(expert_indices), L.ptr(probs), L.dtype_code(probs.dtype), k, num_experts,
+           L.ptr(weights[0]), L.ptr(weights[1]), L.ptr(s1), L.ptr(s2),
+           L.dtype_code(s1.dtype) if s1 is not None else 0, ffn, act, float(limit),
+           int(clamp_after), L.ptr(counts), L.ptr(out), L.ptr(ws), nbytes, L.stream(dev))
+    return out, counts
