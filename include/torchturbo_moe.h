@@ -109,6 +109,21 @@ int tt_router_loss_bwd(const void* logits, int logits_dtype, int64_t num_tokens,
                        int32_t num_experts, int32_t score_function, const uint8_t* padding_mask,
                        const float* grad_prob_sum, const float* grad_z_sum, void* grad_logits,
                        void* stream);
+/* The losses themselves for one sequence-parallel rank and no padding
+ * (router.py:164-270): losses [8] f32 = scaled aux loss, aux loss, scaled
+ * z-loss, z-loss, then the factors the backward uses; a loss whose coefficient
+ * is 0 is left out. sums [E + 1] f32 and tokens_per_expert [E] are written;
+ * workspace as tt_router_loss_fwd. Backward: d logits from the gradients of
+ * the two scaled losses (f32 scalars on the device, NULL for none). */
+int tt_router_losses_fwd(const void* logits, int logits_dtype, int64_t num_tokens,
+                         int32_t num_experts, int32_t topk, int32_t score_function,
+                         float aux_coeff, float z_coeff, float* sums, int64_t* tokens_per_expert,
+                         float* losses, void* workspace, size_t workspace_bytes, void* stream);
+int tt_router_losses_bwd(const void* logits, int logits_dtype, int64_t num_tokens,
+                         int32_t num_experts, int32_t score_function,
+                         const int64_t* tokens_per_expert, const float* losses,
+                         const float* grad_aux, const float* grad_z, void* grad_logits,
+                         void* stream);
 
 /* ---- Routing index (counting sort by expert) ----------------------------
  * Replaces the index build of TorchMoEMaskPermutation

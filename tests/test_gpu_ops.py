@@ -1472,3 +1472,37 @@ def test_lora_residual_matches_fp64(hip_ops, counts, K, N, r, dtype):
         if not c:
             assert not got_da[e].any() and not got_db[e].any()
         r0 += c
+
+
+@pytest.mark.parametrize("aux,z", [(0.01, 0.001), (0.02, 0.0), (0.0, 0.003)])
+@pytest.mark.parametrize("score,T,E,k", [("softmax", 777, 33, 3), ("sigmoid", 1, 64, 8), ("sigmoid", 2500, 256, 8)])
+def test_router_losses_in_one_op_match_the_sums(process_ops, monkeypatch, score, T, E, k, aux, z):
+    """The losses formed on the device (no padding mask) against the scalar formulas on the sums
+    of ``router_loss_stats``, which an all-false padding mask takes: probabilities and map the
+    same, metrics and gradients within a few fp32 roundings (the scalar chain has under 16, and
+    the per-expert sum of E terms adds in another order), for a float and a tensor loss scale."""
+    from torchturbo_amd.moe import MoEConfig, TopKRouter
+    from torchturbo_amd.moe.router import MoEAuxLossAutoScaler
+    from torchturbo_amd.runtime import CudaRuntime
+
+    process_ops(CudaRuntime(), OpPolicy.CUSTOM)
+    torch.manual_seed(T + E)
+    cfg = MoEConfig(hidden_size=64, num_moe_experts=E, moe_router_topk=k, moe_router_dtype="fp32",
+                    moe_router_score_function=score, moe_aux_loss_coeff=aux, moe_z_loss_coeff=z,
+                    params_dtype=torch.bfloat16)
+    router = TopKRouter(cfg).to(DEV)
+    x = torch.randn(T, 64, device=DEV).bfloat16()
+    for scale in (3.0, torch.tensor(0.5, device=DEV)):
+        monkeypatch.setattr(MoEAuxLossAutoScaler, "loss_scale", scale)
+        got = []
+        for pad in (None, torch.zeros(T, dtype=torch.bool, device=DEV)):
+            logits = (x.float() @ router.weight.float().t()).detach().requires_grad_()
+            probs, rmap, _ = router.routing(logits, padding_mask=pad)
+            (probs * 0).sum().backward()  # the losses' gradient alone
+            got.append((probs, rmap, logits.grad, router.pop_metrics()))
+        (p0, m0, g0, s0), (p1, m1, g1, s1) = got
+        assert torch.equal(p0, p1) and torch.equal(m0, m1) and set(s0) == set(s1)
+        for name in s0:
+            torch.testing.assert_close(s0[name], s1[name], rtol=2.0 ** -23 * (16 + E), atol=0)
+        bound = 2.0 ** -23 * (16 + E) * float(g1.abs().max())
+        assert float((g0 - g1).abs().max()) <= bound and float(g1.abs().max()) > 0

@@ -638,6 +638,50 @@ __global__ __launch_bounds__(64) void router_loss_reduce_kernel(
   }
 }
 
+// The losses from the sums (router.py:164-270, one sequence-parallel rank, no
+// padding), one block: aux = prob_sum . counts * E / (k total^2) * aux_coeff
+// with total = max(sum counts / k, 1), z = z_sum / T * z_coeff, and the factors
+// of their gradients. It replaces about 25 scalar launches forward and
+// backward.
+enum { kLossAux = 0, kLossAuxRaw = 1, kLossZ = 2, kLossZRaw = 3, kLossDaux = 4, kLossDz = 5 };
+__global__ __launch_bounds__(256) void router_loss_final_kernel(
+    const float* __restrict__ prob_sum, const int64_t* __restrict__ counts,
+    const float* __restrict__ z_sum, int64_t T, int E, int K, float aux_coeff, float z_coeff,
+    float* __restrict__ scal) {
+  __shared__ float sdot[4];
+  __shared__ int64_t stot[4];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  float dot = 0.f;
+  int64_t tot = 0;
+  if (prob_sum != nullptr)
+    for (int e = tid; e < E; e += 256) {
+      dot += prob_sum[e] * (float)counts[e];
+      tot += counts[e];
+    }
+  dot = wave_sum(dot);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off, TT_WAVE);
+  if (lane_id() == 0) {
+    sdot[wave] = dot;
+    stot[wave] = tot;
+  }
+  __syncthreads();
+  if (tid != 0) return;
+  dot = (sdot[0] + sdot[1]) + (sdot[2] + sdot[3]);
+  const float total = fmaxf((float)(stot[0] + stot[1] + stot[2] + stot[3]) / (float)K, 1.0f);
+  const float den = (float)K * total * total;
+  const float raw = prob_sum != nullptr ? dot * (float)E / den : 0.f;
+  const float zraw = z_sum != nullptr ? *z_sum / (float)(T > 0 ? T : 1) : 0.f;
+  scal[kLossAux] = raw * aux_coeff;
+  scal[kLossAuxRaw] = raw;
+  scal[kLossZ] = zraw * z_coeff;
+  scal[kLossZRaw] = zraw;
+  scal[kLossDaux] = aux_coeff * (float)E / den;
+  scal[kLossDz] = z_coeff / (float)(T > 0 ? T : 1);
+}
+
+// With loads and scal (router_loss_final_kernel's), g_p and g_z are the
+// gradients of the two losses themselves: the sums' follow from the factors.
 // d logits of  sum_e g_p[e] * prob_sum[e] + g_z * z_sum  (one wave per token;
 // padding tokens get zeros). Softmax scores: s * (g - <s, g>); normalised
 // sigmoid / sqrt(softplus) r / (sum r + 1e-20): dr = g / D - <g, r> / D^2,
@@ -651,6 +695,7 @@ template <int EPL>
 __global__ __launch_bounds__(256) void router_loss_bwd_kernel(
     const void* __restrict__ logits, int ldt, int64_t T, int E, int score_fn,
     const uint8_t* __restrict__ pad, const float* __restrict__ g_p, const float* __restrict__ g_z,
+    const int64_t* __restrict__ loads, const float* __restrict__ scal,
     void* __restrict__ grad_logits) {
   const int lane = lane_id();
   const int64_t t = (int64_t)blockIdx.x * kRouterWaves + (threadIdx.x >> 6);
@@ -683,15 +728,16 @@ __global__ __launch_bounds__(256) void router_loss_bwd_kernel(
 #pragma unroll
     for (int i = 0; i < EPL; ++i) zt[i] = 0.f;
     if (g_z != nullptr) {
+      const float gz = scal != nullptr ? *g_z * scal[kLossDz] : *g_z;
       const float lse = lse_like_torch(lg, valid, mx, se, ldt);
       if (low) {
-        const float gl = round_to(round_to(*g_z, ldt) * (2.f * lse), ldt);
+        const float gl = round_to(round_to(gz, ldt) * (2.f * lse), ldt);
 #pragma unroll
         for (int i = 0; i < EPL; ++i)
           zt[i] = valid[i] ? round_to(gl * round_to(expf(round_to(lg[i] - lse, ldt)), ldt), ldt)
                            : 0.f;
       } else {
-        const float f = *g_z * 2.f * lse;
+        const float f = gz * 2.f * lse;
 #pragma unroll
         for (int i = 0; i < EPL; ++i) zt[i] = f * (ex[i] / se);
       }
@@ -699,7 +745,12 @@ __global__ __launch_bounds__(256) void router_loss_bwd_kernel(
     if (g_p != nullptr) {
       float g[EPL];
 #pragma unroll
-      for (int i = 0; i < EPL; ++i) g[i] = valid[i] ? g_p[lane * EPL + i] : 0.f;
+      for (int i = 0; i < EPL; ++i) {
+        const int e = lane * EPL + i;
+        g[i] = !valid[i] ? 0.f
+               : scal != nullptr ? *g_p * scal[kLossDaux] * (float)loads[e]
+                                 : g_p[e];
+      }
       if (score_fn == TT_SCORE_SOFTMAX) {
         float dot = 0.f;
 #pragma unroll
@@ -1594,10 +1645,11 @@ extern "C" int tt_router_loss_fwd(const void* logits, int logits_dtype, int64_t 
   return tt_check_launch("router_loss_fwd");
 }
 
-extern "C" int tt_router_loss_bwd(const void* logits, int logits_dtype, int64_t num_tokens,
+static int loss_bwd_run(const void* logits, int logits_dtype, int64_t num_tokens,
                                   int32_t num_experts, int32_t score_function,
                                   const uint8_t* padding_mask, const float* grad_prob_sum,
-                                  const float* grad_z_sum, void* grad_logits, void* stream) {
+                                  const float* grad_z_sum, const int64_t* loads, const float* scal,
+                        void* grad_logits, void* stream) {
   TT_REQUIRE(logits_dtype_ok(logits_dtype), "router_loss_bwd: unsupported logits dtype %d",
              logits_dtype);
   TT_REQUIRE(num_tokens >= 0, "router_loss_bwd: negative token count");
@@ -1611,7 +1663,7 @@ extern "C" int tt_router_loss_bwd(const void* logits, int logits_dtype, int64_t 
   case N:                                                                                        \
     hipLaunchKernelGGL(router_loss_bwd_kernel<N>, grid, dim3(256), 0, S(stream), logits,         \
                        logits_dtype, num_tokens, num_experts, score_function, padding_mask,      \
-                       grad_prob_sum, grad_z_sum, grad_logits);                                  \
+                       grad_prob_sum, grad_z_sum, loads, scal, grad_logits);                                \
     break;
     TT_CASE(1) TT_CASE(2) TT_CASE(4) TT_CASE(8) TT_CASE(16)
 #undef TT_CASE
@@ -1620,6 +1672,43 @@ extern "C" int tt_router_loss_bwd(const void* logits, int logits_dtype, int64_t 
       return TT_ERR_UNSUPPORTED;
   }
   return tt_check_launch("router_loss_bwd");
+}
+
+extern "C" int tt_router_loss_bwd(const void* logits, int logits_dtype, int64_t num_tokens,
+                                  int32_t num_experts, int32_t score_function,
+                                  const uint8_t* padding_mask, const float* grad_prob_sum,
+                                  const float* grad_z_sum, void* grad_logits, void* stream) {
+  return loss_bwd_run(logits, logits_dtype, num_tokens, num_experts, score_function, padding_mask,
+                      grad_prob_sum, grad_z_sum, nullptr, nullptr, grad_logits, stream);
+}
+
+extern "C" int tt_router_losses_fwd(const void* logits, int logits_dtype, int64_t num_tokens,
+                                    int32_t num_experts, int32_t topk, int32_t score_function,
+                                    float aux_coeff, float z_coeff, float* sums,
+                                    int64_t* tokens_per_expert, float* losses, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  const bool aux = aux_coeff != 0.f, zz = z_coeff != 0.f;
+  const int rc = tt_router_loss_fwd(logits, logits_dtype, num_tokens, num_experts, topk,
+                                    score_function, nullptr, aux ? sums : nullptr,
+                                    aux ? tokens_per_expert : nullptr,
+                                    zz ? sums + num_experts : nullptr, workspace, workspace_bytes,
+                                    stream);
+  if (rc != TT_OK) return rc;
+  hipLaunchKernelGGL(router_loss_final_kernel, dim3(1), dim3(256), 0, S(stream),
+                     aux ? sums : nullptr, tokens_per_expert, zz ? sums + num_experts : nullptr,
+                     num_tokens, num_experts, topk, aux_coeff, z_coeff, losses);
+  return tt_check_launch("router_losses_fwd");
+}
+
+extern "C" int tt_router_losses_bwd(const void* logits, int logits_dtype, int64_t num_tokens,
+                                    int32_t num_experts, int32_t score_function,
+                                    const int64_t* tokens_per_expert, const float* losses,
+                                    const float* grad_aux, const float* grad_z, void* grad_logits,
+                                    void* stream) {
+  TT_REQUIRE(losses != nullptr && tokens_per_expert != nullptr,
+             "router_losses_bwd: the forward's losses and counts are required");
+  return loss_bwd_run(logits, logits_dtype, num_tokens, num_experts, score_function, nullptr,
+                      grad_aux, grad_z, tokens_per_expert, losses, grad_logits, stream);
 }
 
 extern "C" int tt_router_gate_fwd(const void* x, const void* weight, int in_dtype,

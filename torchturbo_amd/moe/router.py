@@ -57,7 +57,10 @@ class MoEAuxLossAutoScaler(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         (aux_loss,) = ctx.saved_tensors
-        return grad_output, torch.ones_like(aux_loss) * MoEAuxLossAutoScaler.loss_scale
+        scale = MoEAuxLossAutoScaler.loss_scale
+        if isinstance(scale, (int, float)):
+            return grad_output, torch.full_like(aux_loss, scale)
+        return grad_output, torch.ones_like(aux_loss) * scale
 
     @classmethod
     def set_loss_scale(cls, scale: float) -> None:
@@ -259,16 +262,40 @@ class TopKRouter(Router):
         want_z = bool(self.config.moe_z_loss_coeff) and training
         want_aux = (training and not self.use_hash_routing
                     and self.config.moe_aux_loss_coeff > 0.0)
-        stats = None
+        stats = losses = None
         if want_z or want_aux:
-            stats = ops.router_loss_stats(logits, self.topk, self.score_function, padding_mask,
-                                          aux=want_aux, z=want_z)
-        return want_z, want_aux, stats
+            losses = self._fused_losses(logits, padding_mask, want_aux, want_z)
+            if losses is None:
+                stats = ops.router_loss_stats(logits, self.topk, self.score_function,
+                                              padding_mask, aux=want_aux, z=want_z)
+        return want_z, want_aux, stats, losses
 
-    def _finish_routing(self, probs, routing_map, want_aux, stats, padding_mask,
+    def _fused_losses(self, logits, padding_mask, want_aux, want_z):
+        """``(scaled aux loss, scaled z-loss)`` formed on the device by one op (metrics
+        recorded), for fp32 logits on a GPU without padding or sequence parallelism; None
+        otherwise."""
+        if (padding_mask is not None or logits.dtype != torch.float32 or not logits.is_cuda
+                or logits.dim() != 2 or _group_size(self.sp_group) > 1
+                or not op_resolves("router_losses")):
+            return None
+        aux, z, aux_raw, z_raw = ops.router_losses(
+            logits, self.topk, self.score_function,
+            self.config.moe_aux_loss_coeff if want_aux else 0.0,
+            self.config.moe_z_loss_coeff if want_z else 0.0)
+        metrics = dict(self._metrics or {})
+        if want_z:
+            metrics.update(z_loss=z_raw.detach(), z_loss_scaled=z.detach())
+        if want_aux:
+            metrics.update(aux_loss=aux_raw.detach(), aux_loss_scaled=aux.detach())
+        self._metrics = metrics
+        return aux, z
+
+    def _finish_routing(self, probs, routing_map, want_aux, stats, losses, padding_mask,
                         accumulate_tokens_per_expert):
         """Aux loss and expert-bias token counts (``router.py:319-354``)."""
-        if want_aux:
+        if want_aux and losses is not None:
+            probs = MoEAuxLossAutoScaler.apply(probs, losses[0])
+        elif want_aux:
             probs = self._apply_aux_loss(probs, stats[0], stats[1])
         if self.enable_expert_bias and accumulate_tokens_per_expert and torch.is_grad_enabled():
             with torch.no_grad():
@@ -286,14 +313,17 @@ class TopKRouter(Router):
         if self.use_hash_routing and input_ids is None:
             raise ValueError("Hash routing requires input_ids.")
         # One pass over the logits for both losses (router.py:299, 319-334).
-        want_z, want_aux, stats = self._loss_stats(logits, padding_mask)
-        logits = self.apply_z_loss(logits, padding_mask=padding_mask,
-                                   z_sum=stats[2] if want_z else None)
+        want_z, want_aux, stats, losses = self._loss_stats(logits, padding_mask)
+        if want_z and losses is not None:
+            logits = MoEAuxLossAutoScaler.apply(logits, losses[1])
+        else:
+            logits = self.apply_z_loss(logits, padding_mask=padding_mask,
+                                       z_sum=stats[2] if want_z else None)
         if self.routing_type != "none":
             raise ValueError(f"Unsupported MoE routing type: {self.routing_type}")
         probs, routing_map, expert_indices = ops.topk_softmax_with_capacity(
             logits, self.topk, **self._routing_kwargs(input_ids))
-        probs = self._finish_routing(probs, routing_map, want_aux, stats, padding_mask,
+        probs = self._finish_routing(probs, routing_map, want_aux, stats, losses, padding_mask,
                                      accumulate_tokens_per_expert)
         return probs, routing_map, expert_indices
 
@@ -323,10 +353,11 @@ class TopKRouter(Router):
         probs, routing_map, expert_indices, logits = ops.router_gate_topk(
             input, self.weight, self.router_dtype(input.dtype), self.topk,
             **self._routing_kwargs(ids))
-        want_z, want_aux, stats = self._loss_stats(logits, padding_mask)
+        want_z, want_aux, stats, losses = self._loss_stats(logits, padding_mask)
         if want_z:
             probs = MoEAuxLossAutoScaler.apply(
-                probs, self._z_loss(logits, padding_mask, stats[2]))
-        probs = self._finish_routing(probs, routing_map, want_aux, stats, padding_mask,
+                probs, losses[1] if losses is not None
+                else self._z_loss(logits, padding_mask, stats[2]))
+        probs = self._finish_routing(probs, routing_map, want_aux, stats, losses, padding_mask,
                                      accumulate_tokens_per_expert)
         return probs, routing_map, expert_indices, logits.view(*input.shape[:-1], -1)

@@ -207,6 +207,46 @@ class RouterLossStats(torch.autograd.Function):
         return out, None, None, None, None, None
 
 
+class RouterLosses(torch.autograd.Function):
+    """``(scaled aux loss, scaled z-loss, aux loss, z-loss)`` of fp32 logits
+    (``tt_router_losses_fwd``); the first two carry gradients, the others are
+    for metrics. A loss whose coefficient is 0 comes back as 0."""
+
+    @staticmethod
+    def forward(ctx, logits, topk, score_function, aux_coeff, z_coeff):
+        logits = logits.contiguous()
+        T, E = logits.shape
+        dev = logits.device
+        sf = L.TT_SCORE[score_function]
+        sums = torch.empty((E + 1,), dtype=torch.float32, device=dev)
+        counts = torch.empty((E,), dtype=torch.int64, device=dev)
+        losses = torch.empty((8,), dtype=torch.float32, device=dev)
+        ws_bytes = L.router_loss_workspace(T, E)
+        ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
+        L.call("tt_router_losses_fwd", L.ptr(logits), L.dtype_code(logits.dtype), T, E, topk, sf,
+               aux_coeff, z_coeff, L.ptr(sums), L.ptr(counts), L.ptr(losses), L.ptr(ws), ws_bytes,
+               L.stream(dev))
+        ctx.save_for_backward(logits, counts, losses)
+        ctx.sf = sf
+        ctx.set_materialize_grads(False)
+        aux, aux_raw, z, z_raw = losses[:4].unbind()
+        ctx.mark_non_differentiable(aux_raw, z_raw)
+        return aux, z, aux_raw, z_raw
+
+    @staticmethod
+    def backward(ctx, g_aux, g_z, _g_aux_raw, _g_z_raw):
+        if g_aux is None and g_z is None:
+            return None, None, None, None, None
+        logits, counts, losses = ctx.saved_tensors
+        T, E = logits.shape
+        ga, gz = (None if g is None else g.to(torch.float32) for g in (g_aux, g_z))
+        out = torch.empty_like(logits)
+        L.call("tt_router_losses_bwd", L.ptr(logits), L.dtype_code(logits.dtype), T, E, ctx.sf,
+               L.ptr(counts), L.ptr(losses), L.ptr(ga), L.ptr(gz), L.ptr(out),
+               L.stream(logits.device))
+        return out, None, None, None, None
+
+
 # ---------------------------------------------------------------------------
 # Permutation
 # ---------------------------------------------------------------------------

@@ -13,7 +13,8 @@ from __future__ import annotations
 from ...dispatch import OpImpl, OpImplKind, register_op
 from ...runtime import TurboDevice
 from . import PRIORITY
-from ._functions import RouterGateTopK, RouterLossStats, TopKRouting, require_cuda
+from ._functions import (RouterGateTopK, RouterLosses, RouterLossStats, TopKRouting,
+                         require_cuda)
 from .available import hip_available
 
 
@@ -64,6 +65,24 @@ class HipRouterLossStats(OpImpl):
             raise ValueError(f"topk must be in [1, {logits.shape[1]}], got {topk}")
         return RouterLossStats.apply(logits, int(topk), score_function, padding_mask, bool(aux),
                                      bool(z))
+
+
+@register_op(op_name="router_losses", impl_name="hip_router_losses",
+             kind=OpImplKind.CUSTOM, priority=PRIORITY, devices=(TurboDevice.CUDA,))
+class HipRouterLosses(OpImpl):
+    """``(scaled aux loss, scaled z-loss, aux loss, z-loss)`` of fp32 logits for
+    one sequence-parallel rank without padding (``router.py:164-270``), formed on
+    the device from the sums of ``router_loss_stats``."""
+
+    def available(self) -> bool:
+        return hip_available()
+
+    def __call__(self, logits, topk, score_function, aux_coeff, z_coeff):
+        require_cuda(logits)
+        if aux_coeff and not 1 <= int(topk) <= logits.shape[1]:
+            raise ValueError(f"topk must be in [1, {logits.shape[1]}], got {topk}")
+        return RouterLosses.apply(logits, int(topk), score_function, float(aux_coeff),
+                                  float(z_coeff))
 
 
 @register_op(op_name="router_gate_topk", impl_name="hip_router_gate_topk",
