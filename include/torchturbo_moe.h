@@ -258,13 +258,14 @@ int tt_gated_act_bwd(const void* x, int dtype, int64_t rows, int64_t ffn, int ac
  * TorchGroupedMatmul (ops/providers/native/grouped_matmul.py:16-56) and
  * grouped_gemm.ops.gmm (ops/providers/cuda/grouped_matmul.py:34-36).
  * dtype bf16/f16 (MFMA, fp32 accumulation) or f32.
- * Concurrency: every bf16 / f16 weight-gradient launch (tt_gmm_wgrad,
- * tt_gmm_wgrad_gather) keeps per-launch state in one of 64 slots of a
- * per-process device array, taken in turn by successive launches and written
- * on the launch stream before the GEMM kernel runs: the persistent kernel's
- * work queue (at most 512 rows per expert on average, M <= 512 * E, or at
- * least 512 output tiles of 256x256 per expert; tt_gmm_wgrad_persistent), or
- * the one-tile-per-block kernel's expert ranking. At most 64 weight-gradient
+ * Concurrency: the bf16 / f16 weight-gradient launches (tt_gmm_wgrad,
+ * tt_gmm_wgrad_gather) of more than a few rows per expert keep per-launch
+ * state in one of 64 slots of a per-process device array, taken in turn by
+ * successive launches and written on the launch stream before the GEMM kernel
+ * runs: the persistent kernel's work queue (tt_gmm_wgrad_persistent), or the
+ * one-tile-per-block kernel's expert ranking. Launches of few rows per expert
+ * (160 on average, 96 for experts of more than 192 output tiles of 256x256)
+ * keep none. At most 64 weight-gradient
  * launches may be in flight at once across all streams of a device; launches
  * on one stream never overlap, so a single stream has no limit. A launch
  * captured into a graph keeps its slot in every replay, so replays of one
@@ -322,9 +323,11 @@ int tt_gmm_wgrad_gather(const void* x, int64_t x_src_rows, const int32_t* x_src_
 int tt_gmm_gather_supported(int32_t op, int dtype, int64_t src_rows, int64_t m, int64_t k,
                             int64_t n, int32_t num_experts);
 /* Whether tt_gmm_wgrad runs this shape (bf16 / f16) on its persistent kernel
- * (1) rather than the one-tile-per-block kernel (0), without launching: short
+ * (1) rather than a kernel of one tile per block (0), without launching: short
  * reductions (m <= 512 * num_experts) or at least 512 output tiles of 256x256
- * per expert. No counterpart in the reference: it reports the launcher's
+ * per expert, unless there are few rows per expert (at most 160 on average, 96
+ * for more than 192 tiles per expert, 512 for at most 256 tiles in all), which
+ * take the small-tile kernel. No counterpart in the reference: it reports the launcher's
  * kernel choice, so that tests and tools can tell which kernel a shape
  * exercises. */
 int tt_gmm_wgrad_persistent(int dtype, int64_t m, int64_t k, int64_t n, int32_t num_experts,

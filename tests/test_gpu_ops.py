@@ -940,6 +940,45 @@ def test_grouped_matmul_wgrad_writes_every_tile(dtype, E, rows, trans_b):
         assert torch.equal(dw[e], ref), (e, int(counts[e]))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("E,K,N,rows", [
+    (12, 8, 8, 40), (12, 136, 264, 200),    # one tile per expert and less, four
+    (31, 1032, 776, 12),                    # 128-row tiles: few rows, a ragged last run of tiles
+    (24, 1032, 776, 130),                   # 256-row tiles, both edges ragged
+    (17, 1544, 1288, 140),                  # a partial group of tile columns
+])
+def test_grouped_matmul_wgrad_few_rows_exact(dtype, trans_b, E, K, N, rows):
+    """The weight gradient of few rows per expert on small-integer operands, so that every
+    sum is exact in fp32 (and below the dtype's exact integers or rounded once): experts
+    of no rows, one row and one more or less than a 16- or 32-deep k-tile or two, rows of
+    the next expert and NaNs behind the operands' ends never reached."""
+    from torchturbo_amd import _lib
+
+    torch.backends.cuda.matmul.allow_tf32 = False
+    g = torch.Generator().manual_seed(K + rows)
+    counts = torch.randint(rows // 2, rows + rows // 2 + 1, (E,), generator=g)
+    edges = torch.tensor([0, 1, 15, 16, 17, 31, 32, 33, 48, 0])
+    counts[:10] = edges if E <= 12 else torch.minimum(edges, counts[:10])
+    counts[10] = rows * 3  # an expert of more rows than the others
+    M = int(counts.sum())
+    assert _lib.load().tt_gmm_wgrad_persistent(_lib.dtype_code(dtype), M, K, N, E, int(trans_b)) == 0
+    assert M <= 512 * E
+    full = [torch.full((M + 64, w), float("nan"), dtype=dtype, device=DEV) for w in (K, N)]
+    x, dy = (f[:M].copy_(torch.randint(-2, 3, (M, f.shape[1]), generator=g)) for f in full)
+    dw = torch.full((E, N, K) if trans_b else (E, K, N), float("nan"), dtype=dtype, device=DEV)
+    cnt = counts.to(DEV)
+    _lib.call("tt_gmm_wgrad", _lib.ptr(x), _lib.ptr(dy), _lib.dtype_code(dtype), M, K, N, E,
+              int(trans_b), _lib.ptr(cnt), _lib.ptr(dw), _lib.stream())
+    torch.cuda.synchronize()
+    xs = torch.split(x.float(), counts.tolist())
+    ds = torch.split(dy.float(), counts.tolist())
+    for e in range(E):
+        ref = xs[e].t() @ ds[e]
+        ref = (ref.t() if trans_b else ref).to(dtype)
+        assert torch.equal(dw[e], ref), (e, int(counts[e]))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("E", [5, 13])
 @pytest.mark.parametrize("K,N", [(512, 768), (64, 64)])

@@ -272,7 +272,11 @@ __device__ __forceinline__ bool row_tile(const int64_t* __restrict__ counts, int
 int tt_gmm_thin(int mode, bool tb, int dtype, const void* p0, const void* p1, void* out,
                 int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s,
                 const int32_t* arow = nullptr, int64_t src_rows = 0);
-// The same with e4m3 weights and block scales, as tt_gmm_fp8_fwd / _dgrad, at
+// Weight gradient for experts of few rows (gmm_wgrad_thin.hip): operands as
+// tt_gmm_wgrad, already checked; see wgrad_thin in gmm.hip.
+int tt_gmm_wgrad_thin(bool tb, int dtype, const void* x, const void* dy, void* dw, int64_t M,
+                      int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s);
+// tt_gmm_thin with e4m3 weights and block scales, as tt_gmm_fp8_fwd / _dgrad, at
 // most TT_THIN8_SCALES scale blocks along the reduction; see thin8_rows in
 // gmm.hip.
 #define TT_THIN8_SCALES 128

@@ -46,7 +46,7 @@
 //   weight-streaming pipeline of their own (two weight k-tiles in flight
 //   while a third is multiplied), and an expert of at most 64 rows takes its
 //   tiles two per schedule slot. Launches of few rows per expert on average
-//   (thin_rows) run on gmm_thin.hip instead.
+//   run on gmm_thin.hip (thin_rows) and gmm_wgrad_thin.hip (wgrad_thin) instead.
 // * gmm_q8_kernel (fwd/dgrad with e4m3 weights and 128x128 block scales,
 //   launches of more than a few rows per expert (thin8_rows; the others run on
 //   gmm_thin.hip) whose reduction is longer than one 64-deep k-tile):
@@ -853,8 +853,8 @@ constexpr int P_BK = 64;
 constexpr int P_OPND = 256 * P_BK * 2;  // one operand tile (32 KiB)
 constexpr int P_STAGE = 2 * P_OPND;     // A then B
 constexpr int P_EPI = 4096;             // epilogue staging per wave
-// wgrad takes the persistent kernel when the mean rows per expert are at most
-// this (a handful of 64-deep k-tiles per output tile).
+// wgrad takes the persistent kernel, or the small-tile one, when the mean rows
+// per expert are at most this (a handful of 64-deep k-tiles per output tile).
 constexpr int64_t P_WGRAD_ROWS = 512;
 // ... or experts of at least this many 256x256 output tiles.
 constexpr int P_WGRAD_TILES = 512;
@@ -2545,7 +2545,30 @@ size_t p64_schedule_bytes(int E) { return schedule_bytes(E) + (size_t)E * sizeof
 // the cost-sorted schedule's slot lists).
 size_t p64_lds_bytes(int E) { return p64_schedule_bytes(E) + 2 * P_STAGE + 4 * P_EPI + 1024; }
 
-// Weight gradients (ti x tj output tiles per expert) run on the persistent
+// Weight gradients of at most W_THIN_ROWS rows per expert on average run on
+// gmm_wgrad_thin.hip: up to W_WIDE_ROWS for experts of more than W_WIDE_TILES
+// 256x256 tiles, whose operand panels pass through L2 once per row of tiles,
+// which smaller tiles pay twice; up to P_WGRAD_ROWS for launches whose 256x256
+// tiles would leave CUs idle. Persistent / thin, fc1 + fc2, even loads: 128
+// experts of 2048 x 1536 and 768 x 2048 at 62 rows 164 + 96 / 138 + 73 us, 128
+// rows 199 + 114 / 162 + 84; 64 of 1024 x 1408 and 704 x 1024 at 144 rows 65 +
+// 47 / 46 + 26; 64 of 7168 x 4096 and 2048 x 7168 (448 and 224 tiles) at 64
+// rows 781 + 376 / 656 + 307, 128 rows 853 + 442 / 852 + 430; 8 of 512 x 1024
+// and 512 x 512 at 500 rows 24 + 35 / 15 + 11. Zipf loads (exponent 0.8, the
+// longest expert about 15 times the mean): the first layer at 62 rows 175 + 96
+// / 152 + 79, 128 rows 203 + 112 / 207 + 106, 256 rows 270 + 154 / 300 + 163
+// (even loads 291 + 161 / 260 + 118): above the line the long experts are
+// bound by their products, which the larger tiles do better.
+constexpr int64_t W_THIN_ROWS = 160, W_WIDE_ROWS = 96;
+constexpr int W_WIDE_TILES = 192;
+bool wgrad_thin(int64_t M, int64_t E, int ti, int tj) {
+  const int64_t rows = (int64_t)ti * tj > W_WIDE_TILES ? W_WIDE_ROWS
+                       : E * ti * tj <= 256            ? P_WGRAD_ROWS
+                                                       : W_THIN_ROWS;
+  return M <= E * rows && E * ti * tj * 4 < 0x7fffffff;
+}
+
+// The others (ti x tj output tiles per expert) run on the persistent
 // kernel for short reductions (few rows per expert on average, known without
 // the counts), and for experts of at least P_WGRAD_TILES output tiles: it
 // spreads an expert's tiles over the eight XCDs in rectangles that share
@@ -2558,6 +2581,7 @@ size_t p64_lds_bytes(int E) { return p64_schedule_bytes(E) + 2 * P_STAGE + 4 * P
 // Qwen3-30B-A3B fc1 (48) 860 against 842 us, fc2 (24) 516 against 443 us;
 // the varlen stress layer's fc1 (48) 3276 against 2974 us.
 bool wgrad_persistent(int64_t M, int64_t K, int64_t N, int E, int ti, int tj) {
+  if (wgrad_thin(M, E, ti, tj)) return false;
   const int64_t ld = K > N ? K : N;
   return (M <= (int64_t)E * P_WGRAD_ROWS || (int64_t)ti * tj >= P_WGRAD_TILES) &&
          p64_lds_bytes(E) <= 160 * 1024 &&
@@ -2637,10 +2661,12 @@ int launch_mfma(const void* p0, const void* p1, void* out, int64_t M, int64_t K,
                                                tj);
     }
   } else {
-    // The persistent kernel for short reductions and large tile grids (see
-    // wgrad_persistent), the four-stage one-tile-per-block kernel otherwise.
+    // The small-tile kernel (see wgrad_thin) or the persistent kernel for short
+    // reductions, the latter also for large tile grids (see wgrad_persistent), the four-stage one-tile-per-block kernel otherwise.
     // wgrad reduces over each expert's rows (at most M; the loads run up to
     // two k-tiles past an expert's end).
+    if (wgrad_thin(M, E, ti, tj))
+      return tt_gmm_wgrad_thin(TB, ET, p0, p1, out, M, K, N, E, counts, s);
     if (wgrad_persistent(M, K, N, E, ti, tj))
       return launch_p64_k<MODE, TB, ET, false>(p0, p1, out, M, K, N, E, counts, s, nblk, ti, tj);
   }
