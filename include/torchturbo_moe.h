@@ -70,14 +70,28 @@ int tt_router_topk_bwd(const void* logits, int logits_dtype, int64_t num_tokens,
  * exact 16-bit products rounded once, then routed exactly as
  * tt_router_topk_fwd routes logits of that dtype (same outputs and
  * arguments). E in {32, 64, ..., 256}, hidden a multiple of 64, x and weight
- * 16-byte aligned. The backward is tt_router_topk_bwd plus the two plain
- * GEMMs of the linear. */
+ * 16-byte aligned. The backward is tt_router_topk_bwd, then the two
+ * products of the linear (tt_router_gate_bwd for bf16 operands with fp32
+ * logits). */
 int tt_router_gate_fwd(const void* x, const void* weight, int in_dtype, int64_t num_tokens,
                        int64_t hidden, int32_t num_experts, int logits_dtype, int32_t topk,
                        int32_t score_function, int32_t pre_softmax, const float* expert_bias,
                        int32_t num_groups, int32_t group_topk, float scaling_factor,
                        const int64_t* fixed_indices, void* logits, void* probs,
                        uint8_t* routing_map, int64_t* top_indices, void* stream);
+
+/* Backward of the gating linear of bf16 x [T, hidden], weight [E, hidden] and
+ * fp32 logits (models/modules/moe/router.py:44-58): with g = grad + grad2
+ * (fp32 [T, E], grad2 may be NULL), dx [T, hidden] = bf16(g weight) and dw
+ * [E, hidden] = bf16(g^T x), each skipped when NULL. fp32 products and sums: g
+ * enters as three bf16 parts that add up to it exactly. Sizes as
+ * tt_router_gate_fwd with operands under 4 GiB; everything 16-byte aligned.
+ * tt_router_gate_bwd_workspace: bytes of scratch, or -1 when the size is not
+ * taken. */
+int64_t tt_router_gate_bwd_workspace(int64_t num_tokens, int64_t hidden, int64_t num_experts);
+int tt_router_gate_bwd(const float* grad, const float* grad2, const void* x, const void* weight,
+                       int64_t num_tokens, int64_t hidden, int64_t num_experts, void* workspace,
+                       int64_t workspace_bytes, void* dx, void* dw, void* stream);
 
 /* ---- Router loss statistics (aux load-balancing loss, z-loss) ------------
  * Replaces the [T, E] work of compute_routing_scores_for_aux_loss and

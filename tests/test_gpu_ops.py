@@ -940,6 +940,57 @@ def test_grouped_matmul_wgrad_writes_every_tile(dtype, E, rows, trans_b):
         assert torch.equal(dw[e], ref), (e, int(counts[e]))
 
 
+@pytest.mark.parametrize("T,H,E", [(1, 64, 32), (31, 192, 64), (129, 320, 96), (700, 2048, 256),
+                                   (2051, 1024, 128), (9000, 128, 32)])
+def test_router_gate_bwd_matches_fp64(T, H, E):
+    """dx and dw of the gating linear against float64 products rounded to bf16: from fp32
+    gradients over a wide range with a second addend, ragged token counts, every output
+    written, and no larger error than the fp32 composition's. An infinity or a NaN among
+    the activations or weights gives what the fp32 products give."""
+    from torchturbo_amd.providers.hip._functions import router_gate_bwd
+
+    torch.backends.cuda.matmul.allow_tf32 = False
+    gen = torch.Generator().manual_seed(T + H)
+    g = torch.randn(T, E, generator=gen) * torch.exp2(torch.randint(-12, 5, (T, E), generator=gen).float())
+    g2 = torch.randn(T, E, generator=gen) * 1e-3
+    x, w = (torch.randn(n, H, generator=gen).to(torch.bfloat16).to(DEV) for n in (T, E))
+    g, g2 = g.to(DEV), g2.to(DEV)
+
+    def errors(dx, dw):
+        s = (g + g2).double()
+        out = []
+        for got, a, b in ((dx, s, w), (dw, s.t(), x)):
+            ref, mag = a @ b.double(), a.abs() @ b.double().abs()
+            # one bf16 rounding of the result, and fp32 sums of exact products
+            bound = ref.abs() * 2.0 ** -8 + mag * a.shape[1] * 2.0 ** -24 * 2
+            assert bool(((got.double() - ref).abs() <= bound).all())
+            out.append(float((got.double() - ref).square().mean()))
+        return out
+
+    native = router_gate_bwd(g, g2, x, w, True, True)
+    assert native is not None
+    s = g + g2
+    plain = (s.mm(w.float()).to(w.dtype), s.t().mm(x.float()).to(w.dtype))
+    for a, b in zip(errors(*native), errors(*plain)):
+        # bf16 roundings of nearly the same values; a few flip either way
+        assert a <= b * 1.01 + 1e-30
+    dx, none = router_gate_bwd(g, g2, x, w, True, False)
+    assert none is None and torch.equal(dx, native[0])
+    none, dw = router_gate_bwd(g, g2, x, w, False, True)
+    assert none is None and torch.equal(dw, native[1])
+    # one fp32 addend, not split between g and g2
+    dx, dw = router_gate_bwd(s, None, x, w, True, True)
+    assert torch.equal(dx, native[0]) and torch.equal(dw, native[1])
+
+    x[T // 2, H // 2], w[E - 1, 1], w[0, 2] = float("inf"), float("-inf"), float("nan")
+    dx, dw = router_gate_bwd(g, g2, x, w, True, True)
+    for got, ref in ((dx, s.mm(w.float())), (dw, s.t().mm(x.float()))):
+        assert torch.equal(got.isnan(), ref.isnan())
+        inf = ref.isinf()
+        assert bool(inf.any()) and torch.equal(got[inf].float(), ref[inf])
+        assert torch.equal(got.isinf(), ref.to(torch.bfloat16).isinf())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("E,K,N,rows", [

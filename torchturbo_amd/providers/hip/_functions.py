@@ -102,12 +102,35 @@ def router_topk_bwd(logits, top, grad_probs, topk, sf, pre, scale):
     return out
 
 
+def router_gate_bwd(g, g2, x, w, want_x, want_w):
+    """``(dx, dw)`` of the gating linear from fp32 gradients ``g + g2`` of its logits
+    (``tt_router_gate_bwd``), None for a part not wanted; or None when the operands are
+    not bf16 with fp32 gradients, dense and aligned, of a size the kernels take."""
+    if not (g.dtype is torch.float32 and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16):
+        return None
+    tensors = (g, x, w) if g2 is None else (g, g2, x, w)
+    if any(not t.is_contiguous() or t.data_ptr() % 16 for t in tensors):
+        return None
+    T, H = x.shape
+    E = w.shape[0]
+    ws_bytes = L.load().tt_router_gate_bwd_workspace(T, H, E)
+    if ws_bytes < 0:
+        return None
+    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=x.device)
+    dx = torch.empty_like(x) if want_x else None
+    dw = torch.empty_like(w) if want_w else None
+    L.call("tt_router_gate_bwd", L.ptr(g), L.ptr(g2), L.ptr(x), L.ptr(w), T, H, E, L.ptr(ws),
+           ws_bytes, L.ptr(dx), L.ptr(dw), L.stream(x.device))
+    return dx, dw
+
+
 class RouterGateTopK(torch.autograd.Function):
-    """Gating linear and top-k routing in one kernel (``tt_router_gate_fwd``):
+    """Gating linear and top-k routing (``tt_router_gate_fwd``):
     ``(probs, routing_map, top_indices, logits)`` with ``logits = x W^T`` in
     the router dtype. Backward: the routing gradient (``tt_router_topk_bwd``)
     plus the gradient reaching the logits directly, then the gating linear's
-    backward as ``RouterGatingLinearFunction`` forms it (``router.py:44-58``)."""
+    backward as ``RouterGatingLinearFunction`` forms it (``router.py:44-58``), for
+    bf16 operands and fp32 logits in kernels of its own (``tt_router_gate_bwd``)."""
 
     @staticmethod
     def forward(ctx, x, weight, router_dtype, topk, score_function, pre_softmax, num_groups,
@@ -141,10 +164,17 @@ class RouterGateTopK(torch.autograd.Function):
         none = (None,) * 9
         x2, w, logits, top = ctx.saved_tensors
         g = None
-        if g_probs is not None:
-            g = router_topk_bwd(logits, top, g_probs, *ctx.cfg)
         if g_logits is not None:
             g_logits = g_logits.reshape(logits.shape).to(logits.dtype)
+        if g_probs is not None:
+            g = router_topk_bwd(logits, top, g_probs, *ctx.cfg)
+            # Native products unless the backward is itself being recorded.
+            grads = None if torch.is_grad_enabled() else router_gate_bwd(
+                g, g_logits, x2, w, ctx.needs_input_grad[0], ctx.needs_input_grad[1])
+            if grads is not None:
+                gx, gw = grads
+                return None if gx is None else gx.view(ctx.x_shape), gw, *none
+        if g_logits is not None:
             g = g_logits if g is None else g + g_logits
         if g is None:
             return None, None, *none
