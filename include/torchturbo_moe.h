@@ -86,12 +86,12 @@ int tt_router_gate_fwd(const void* x, const void* weight, int in_dtype, int64_t 
  * [E, hidden] = bf16(g^T x), each skipped when NULL. fp32 products and sums: g
  * enters as three bf16 parts that add up to it exactly. Sizes as
  * tt_router_gate_fwd with operands under 4 GiB; everything 16-byte aligned.
- * tt_router_gate_bwd_workspace: bytes of scratch, or -1 when the size is not
+ * tt_router_gate_bwd_workspace: bytes of scratch, or 0 when the size is not
  * taken. */
-int64_t tt_router_gate_bwd_workspace(int64_t num_tokens, int64_t hidden, int64_t num_experts);
+size_t tt_router_gate_bwd_workspace(int64_t num_tokens, int64_t hidden, int64_t num_experts);
 int tt_router_gate_bwd(const float* grad, const float* grad2, const void* x, const void* weight,
                        int64_t num_tokens, int64_t hidden, int64_t num_experts, void* workspace,
-                       int64_t workspace_bytes, void* dx, void* dw, void* stream);
+                       size_t workspace_bytes, void* dx, void* dw, void* stream);
 
 /* ---- Router loss statistics (aux load-balancing loss, z-loss) ------------
  * Replaces the [T, E] work of compute_routing_scores_for_aux_loss and

@@ -40,7 +40,7 @@ _PROTOS: dict[str, list] = {
     "tt_router_gate_fwd": [P, P, c_int, I64, I64, I32, c_int, I32, I32, I32, P, I32, I32, c_float,
                            P, P, P, P, P, P],
     "tt_router_gate_bwd_workspace": [I64, I64, I64],
-    "tt_router_gate_bwd": [P, P, P, P, I64, I64, I64, P, I64, P, P, P],
+    "tt_router_gate_bwd": [P, P, P, P, I64, I64, I64, P, c_size_t, P, P, P],
     "tt_router_loss_workspace": [I64, I32],
     "tt_router_loss_fwd": [P, c_int, I64, I32, I32, I32, P, P, P, P, P, c_size_t, P],
     "tt_router_loss_bwd": [P, c_int, I64, I32, I32, P, P, P, P, P],
@@ -77,7 +77,7 @@ _PROTOS: dict[str, list] = {
 }
 _RESTYPES = {"tt_last_error": ctypes.c_char_p, "tt_route_index_workspace": c_size_t,
              "tt_route_index_rejected_offset": c_size_t, "tt_router_loss_workspace": c_size_t,
-             "tt_moe_experts_workspace": c_size_t, "tt_router_gate_bwd_workspace": I64}
+             "tt_moe_experts_workspace": c_size_t, "tt_router_gate_bwd_workspace": c_size_t}
 ABI_VERSION = 1
 
 _LIB: ctypes.CDLL | None = None

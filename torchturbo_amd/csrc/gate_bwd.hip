@@ -294,13 +294,13 @@ bool takes(int64_t T, int64_t H, int64_t E) {
 
 }  // namespace
 
-extern "C" int64_t tt_router_gate_bwd_workspace(int64_t T, int64_t H, int64_t E) {
-  return takes(T, H, E) ? plan(T, (int)H, (int)E).bytes : -1;
+extern "C" size_t tt_router_gate_bwd_workspace(int64_t T, int64_t H, int64_t E) {
+  return takes(T, H, E) ? (size_t)plan(T, (int)H, (int)E).bytes : 0;
 }
 
 extern "C" int tt_router_gate_bwd(const float* grad, const float* grad2, const void* x,
                                   const void* w, int64_t T, int64_t H, int64_t E, void* workspace,
-                                  int64_t workspace_bytes, void* dx, void* dw, void* stream) {
+                                  size_t workspace_bytes, void* dx, void* dw, void* stream) {
   TT_REQUIRE(takes(T, H, E), "router_gate_bwd: unsupported size T=%lld H=%lld E=%lld",
              (long long)T, (long long)H, (long long)E);
   TT_REQUIRE(grad != nullptr && (dx == nullptr || w != nullptr) && (dw == nullptr || x != nullptr),
@@ -310,7 +310,7 @@ extern "C" int tt_router_gate_bwd(const float* grad, const float* grad2, const v
               15) == 0,
              "router_gate_bwd: operands must be 16-byte aligned");
   const Plan p = plan(T, (int)H, (int)E);
-  TT_REQUIRE(workspace != nullptr && workspace_bytes >= p.bytes,
+  TT_REQUIRE(workspace != nullptr && workspace_bytes >= (size_t)p.bytes,
              "router_gate_bwd: workspace of %lld bytes required", (long long)p.bytes);
   if (dx == nullptr && dw == nullptr) return TT_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -114,7 +114,7 @@ def router_gate_bwd(g, g2, x, w, want_x, want_w):
     T, H = x.shape
     E = w.shape[0]
     ws_bytes = L.load().tt_router_gate_bwd_workspace(T, H, E)
-    if ws_bytes < 0:
+    if ws_bytes == 0:
         return None
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=x.device)
     dx = torch.empty_like(x) if want_x else None
