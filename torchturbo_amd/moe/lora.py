@@ -4,10 +4,11 @@ Mirrors ``src/torchturbo/engine/peft/lora.py:54-725``:
 
 * ``GroupedLoRALinear`` (``lora.py:54-125``) holds one fp32 matrix per expert,
   ``[E, in, out]``, and multiplies expert-major packed rows by it with the
-  ``grouped_matmul`` op (the same grouped GEMM as the base layer);
+  ``grouped_matmul`` op when called on its own;
 * ``GroupedMLPLoRA`` (``lora.py:128-725``) wraps a :class:`GroupedMLP` and adds
   ``scaling * gmm(gmm(dropout(x).float(), A), B).to(out.dtype)`` to its fc1 and
-  fc2 outputs (additive residual, no ``[E, in, out]`` delta is formed), with
+  fc2 outputs (additive residual, no ``[E, in, out]`` delta is formed; on the
+  GPU the ``lora_residual`` op, without fp32 copies of the rows), with
   the reference's adapter management: ranks, ``lora_alpha`` scaling (plain or
   rank-stabilised), dropout, Kaiming-uniform or Gaussian initialisation, active
   adapter selection, merge / unmerge into the base weights and the conversion

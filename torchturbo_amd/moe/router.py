@@ -8,13 +8,14 @@ top-k selection, attaches the aux loss and accumulates expert-bias counts
 op, and the [T, E] sums behind the aux loss and the z-loss (per-expert score
 sums and top-k counts of the bias-free scores, the sum of squared
 log-sum-exps) through the ``router_loss_stats`` op, so the GPU runs one HIP
-kernel for each per direction. The scalar formulas on top of those sums, the
-sequence-parallel all-reduce and the metrics are the reference's
-(``router.py:164-270``). ``compute_routing_scores_for_aux_loss`` and
+kernel for each per direction. For fp32 logits on one sequence-parallel rank
+without padding the losses themselves come from the ``router_losses`` op;
+otherwise the scalar formulas on top of those sums, the sequence-parallel
+all-reduce and the metrics are the reference's (``router.py:164-270``). ``compute_routing_scores_for_aux_loss`` and
 ``z_loss_func`` (``moe_utils.py:15-70``) remain importable.
 
 ``forward`` runs the gating linear and the top-k as one op
-(``router_gate_topk``: one HIP kernel on the GPU) when the inputs and the
+(``router_gate_topk``: one or two HIP kernels on the GPU) when the inputs and the
 router weight share a 16-bit dtype, the router dtype is that dtype or fp32,
 E is a multiple of 32 up to 256 and the hidden size a multiple of 64; the
 z-loss is then attached to the probabilities instead of the logits the

@@ -90,8 +90,8 @@ class HipRouterLosses(OpImpl):
 class HipRouterGateTopK(OpImpl):
     """``(probs, routing_map, top_indices, logits)`` of ``TopKRouter.gating``
     (``router.py:25-58,84-101``) followed by ``topk_softmax_with_capacity``
-    (``utils.py:127-230``), in one kernel: x and the router weight in bf16 or
-    f16 (the same dtype), logits in that dtype or fp32, E a multiple of 32 up
+    (``utils.py:127-230``), in one kernel, or in two for few tokens: x and
+    the router weight in bf16 or f16 (the same dtype), logits in that dtype or fp32, E a multiple of 32 up
     to 256, hidden a multiple of 64 (``TopKRouter`` checks this before it
     asks)."""
 
