@@ -1308,6 +1308,34 @@ def test_grouped_matmul_fp8_few_rows_exact(counts, K, N, sdt):
         s0 += c
 
 
+@pytest.mark.parametrize("counts", [[3, 17, 40], [40, 33, 39]], ids=["tiles32", "tiles64"])
+def test_grouped_matmul_fp8_bits_do_not_depend_on_the_batch(counts):
+    """A row's products are summed in one order: a launch of few rows per expert gives the
+    bits of a longer launch over the same rows (reductions with a tail). The second half of
+    every reduction cancels the first, so that the results are the rounding of the sums."""
+    from torchturbo_amd import _lib
+
+    g = torch.Generator().manual_seed(sum(counts))
+    E, K, N, LONG = len(counts), 400, 272, 200
+    q = torch.randn(E, N // 2, K // 2, generator=g).to(torch.float8_e4m3fn).view(torch.uint8)
+    q = q.repeat(1, 2, 2).to(DEV)
+    s = torch.full((E, -(-N // 128), -(-K // 128)), 0.71, dtype=torch.bfloat16, device=DEV)
+    for name, width, out_width in (("tt_gmm_fp8_fwd", K, N), ("tt_gmm_fp8_dgrad", N, K)):
+        long = torch.randn(E, LONG, width // 2, generator=g).to(torch.bfloat16)
+        long = torch.cat([long, -long], dim=2).to(DEV)
+
+        def run(rows, counts):
+            y = torch.empty(rows.shape[0], out_width, dtype=torch.bfloat16, device=DEV)
+            cnt = torch.tensor(counts, dtype=torch.int64, device=DEV)
+            _lib.call(name, _lib.ptr(rows), _lib.ptr(q), _lib.ptr(s), _lib.dtype_code(s.dtype),
+                      rows.shape[0], K, N, E, _lib.ptr(cnt), _lib.ptr(y), _lib.stream())
+            return y
+
+        few = run(torch.cat([x[:c] for x, c in zip(long, counts)]), counts)
+        many = run(long.view(E * LONG, width), [LONG] * E).view(E, LONG, out_width)
+        assert torch.equal(few, torch.cat([y[:c] for y, c in zip(many, counts)])), name
+
+
 # more 256x256 output tiles than the GPU has compute units, so every persistent block
 # walks many tiles (tile switch, cross-tile prefetch, XCD remap); mean expert loads above
 # 512 rows take the four-stage weight-gradient kernel, at most 512 the persistent

@@ -231,15 +231,22 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin_kernel(
 // K-major weight row is a whole 128-byte line and a block has one scale per
 // k-tile (T_BN is the scale blocks' width), kept in two registers across the
 // lanes. fwd reads 16 bytes of a row per lane, two MFMA steps at once: lane
-// half h holds reduction elements 32 p + 16 h .. + 15 of step pair p, and the
-// activations' fragments take the same elements, so the order of the products
-// inside a pair of steps differs from the other kernels. dgrad reads N-major
-// weight rows with the transposing 8-bit read (two lanes per row and 16
-// columns). LDS: weights 16 KiB, activations 256 bytes per row, as two
+// half h reads reduction elements 32 p + 16 h .. + 15 of step pair p, and the
+// halves exchange eight of them, so that each step multiplies 16 consecutive
+// elements as gmm_q8_kernel does: the same bits whichever kernel a launch
+// takes. dgrad reads N-major weight rows with the transposing 8-bit read (two
+// lanes per row and 16 columns). LDS: weights 16 KiB, activations 256 bytes per row, as two
 // 64-deep tiles. Measured on DeepSeek-V3's fc1 and fc2 (256 experts), forward,
 // gmm_q8_kernel / this kernel: one token 187 + 58 / 49 + 25 us, 24 tokens (137
 // experts used) 947 + 470 / 610 + 319 us (6.6 TB/s), 1024 tokens 1718 + 879 /
 // 1418 + 802; data gradient at 512 tokens 1567 + 751 / 1353 + 630.
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+  // The upper 32 lanes of a against the lower 32 of b.
+  const auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = v[0];
+  b = v[1];
+}
+
 constexpr int T8_BK = 128;
 constexpr int T8_SMAX = TT_THIN8_SCALES;  // scale blocks along the reduction
 static_assert(T8_SMAX == 128, "two registers of one scale per lane");
@@ -342,14 +349,13 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin8_kernel(
     asm volatile("" : "+v"(sv[0]), "+v"(sv[1]));  // awaited here, with the first k-tiles
   }
 
-  // Fragment offsets within a stage. A: step s of the 64-deep half s / 4; fwd
-  // takes chunk 4 (s / 2) + 2 h + s % 2 of the k-tile (see above), dgrad chunk
-  // 2 s + h.
+  // Fragment offsets within a stage. A: chunk 2 s + h of the k-tile, in its
+  // 64-deep half s / 4.
   uint32_t fa[8], fb[8];
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
     const int h = lane >> 5, r = lane & 31;
-    const int c = FW ? 4 * (s >> 1) + 2 * h + (s & 1) : 2 * s + h;  // of 16
+    const int c = 2 * s + h;  // of 16
     fa[s] = (uint32_t)((c >> 3) * (BM * 128) + r * 128 + (((c & 7) ^ ((r >> 1) & 7)) << 4));
     if constexpr (FW) {  // steps 2 p, 2 p + 1: chunk 2 p + h of row 32 w + lane % 32
       fb[s] = T_A + fragk64(32 * wave, s >> 1, lane);
@@ -382,7 +388,13 @@ __global__ __launch_bounds__(T_NT, OCC) void gmm_thin8_kernel(
       for (int s = 0; s < 8; ++s) {
         uint2 q;
         if constexpr (FW) {
-          if ((s & 1) == 0) pair = read_k(stg, fb[s]);
+          if ((s & 1) == 0) {
+            // Elements 0-7 | 16-23 and 8-15 | 24-31 of the pair's 32 (lower |
+            // upper lane half) become 0-7 | 8-15 and 16-23 | 24-31.
+            pair = read_k(stg, fb[s]);
+            swap_halves(pair.x, pair.z);
+            swap_halves(pair.y, pair.w);
+          }
           q = (s & 1) ? uint2{pair.z, pair.w} : uint2{pair.x, pair.y};
         } else {
           typedef __attribute__((ext_vector_type(2))) int i32x2_t;
