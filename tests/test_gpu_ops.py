@@ -1592,6 +1592,31 @@ def test_lora_residual_matches_fp64(hip_ops, counts, K, N, r, dtype):
         r0 += c
 
 
+@pytest.mark.parametrize("counts,K,N,r,dtype", LORA_CASES, ids=[f"E{len(c[0])}K{c[1]}N{c[2]}r{c[3]}" for c in LORA_CASES])
+def test_lora_residual_bits_of_the_composition(hip_ops, counts, K, N, r, dtype):
+    """The adapter kernels sum in the fp32 grouped products' order: output and every gradient
+    are the composition's bit for bit."""
+    g = torch.Generator().manual_seed(K + 3 * N + r)
+    E, M, s = len(counts), sum(counts), 0.3
+
+    def leaf(*shape, dtype):
+        return torch.randn(*shape, generator=g).to(dtype).to(DEV).requires_grad_()
+
+    leaves = (leaf(M, N, dtype=dtype), leaf(M, K, dtype=dtype), leaf(E, K, r, dtype=torch.float32),
+              leaf(E, r, N, dtype=torch.float32))
+    dy = torch.randn(M, N, generator=g).to(dtype).to(DEV)
+    cnt = torch.tensor(counts, device=DEV)
+    y = hip_ops.lora_residual(*leaves, cnt, s)
+    got = (y, *torch.autograd.grad(y, leaves, dy))
+    base, x, a, b = leaves
+    delta = hip_ops.grouped_matmul(hip_ops.grouped_matmul(x.float(), a, cnt, trans_b=False), b, cnt,
+                                   trans_b=False)
+    ref = base + delta.to(dtype) * s
+    want = (ref, *torch.autograd.grad(ref, leaves, dy))
+    for name, v, w in zip(("y", "dbase", "dx", "da", "db"), got, want):
+        assert torch.equal(v, w), name
+
+
 @pytest.mark.parametrize("aux,z", [(0.01, 0.001), (0.02, 0.0), (0.0, 0.003)])
 @pytest.mark.parametrize("score,T,E,k", [("softmax", 777, 33, 3), ("sigmoid", 1, 64, 8), ("sigmoid", 2500, 256, 8)])
 def test_router_losses_in_one_op_match_the_sums(process_ops, monkeypatch, score, T, E, k, aux, z):

@@ -4,19 +4,21 @@
 // B [E, r, N] in fp32, r at most 64. Every product and sum runs in fp32 on
 // v_mfma_f32_16x16x4_f32 (16-bit activations widen exactly), and only the r-wide
 // h is kept in fp32: a composition of grouped products instead writes and reads
-// an fp32 copy of x and the fp32 product h B.
+// an fp32 copy of x and the fp32 product h B. The results are the composition's
+// bit for bit (chain16 below).
 //
 // * lora_down_kernel: h = x A_e, and dh = round(dy s) B_e^T in the backward.
 // * lora_up_kernel: y from h, and dx = round(dh A_e^T).
 // * lora_wgrad_kernel: dA_e = x_e^T dh_e and dB_e = h_e^T round(dy_e s).
 //
 // Low ranks are bound by the 16-bit activations that they stream and by the
-// latency of a block's few loads, ranks above about 32 by the fp32 MFMAs.
-// Layer of 128 experts, 2048 tokens, top-8, H 2048, F 768, r 16 (16384 rows),
-// both linears: down 49 us forward and 68 backward, up 90 and 63, wgrad 37 (A)
-// and 48 (B), 354 us in place of 1609 us of fp32 grouped products and 380 us of
-// casts, scalings and sums; forward and backward 2821 -> 1204 us. At 4096
-// tokens r 8 takes 4099 -> 1833 us, r 64 5018 -> 3043.
+// chain of products, ranks above about 32 by the fp32 MFMAs. Layer of 128
+// experts, 2048 tokens, top-8, H 2048, F 768, r 16 (16384 rows), both linears:
+// down 53 us forward and 77 backward, up 89 and 63, wgrad 38 (A) and 52 (B),
+// 372 us in place of 1609 us of fp32 grouped products and 380 us of casts,
+// scalings and sums; forward and backward 2821 -> 1211 us, at 4096 tokens r 8
+// 4098 -> 1843 us, r 64 5017 -> 2980. (Sums split over the waves of a block
+// took 354 us, but in an order of their own: other last bits.)
 #include "gemm.h"
 
 #include <type_traits>
@@ -27,8 +29,8 @@ struct BF { static constexpr int code = TT_BF16; };
 struct HF { static constexpr int code = TT_F16; };
 
 constexpr int LR_NT = 256;
-constexpr int LD_NT = 512;  // lora_down: eight waves share a reduction
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((address_space(3))) float lds_float;
 
 __device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -68,116 +70,166 @@ __device__ __forceinline__ void widen8(const uint4& v, float s, float (&x)[8]) {
   }
 }
 
+// Every sum runs in the order of the fp32 grouped products (gmm_f32_kernel),
+// one chain of products per result: 0, 8, 1, 9, ... 7, 15 of each 16
+// reduction elements, so that the results are a composition's bit for bit.
+// Lane group g = lane / 16 of product q of such a 16 takes element
+// 2 q + g / 2 + 8 (g % 2), the element chain16(4 q + g) of a position in the chain.
+__device__ __forceinline__ int chain16(int p) {
+  return (p & ~15) + 2 * ((p & 15) >> 2) + ((p >> 1) & 1) + 8 * (p & 1);
+}
+
+// The position of element j: chain16(place16(j)) = j.
+__device__ __forceinline__ int place16(int j) {
+  return (j & ~15) + 4 * ((j & 7) >> 1) + 2 * (j & 1) + ((j >> 3) & 1);
+}
+
+// Element `odd` of a packed pair, widened; with SCALE times s and rounded to
+// 16 bits first.
+template <class TT, bool SCALE>
+__device__ __forceinline__ float widen1(uint32_t w, bool odd, float s) {
+  float v = odd ? hi16<TT>(w) : lo16<TT>(w);
+  if constexpr (SCALE) v = lo16<TT>(pack2<TT>(v * s, 0.f));
+  return v;
+}
+
 // ---------------------------------------------------------------------------
 // out[m, j] (fp32 [M, r]) = sum over c of in[m, c] W_e(c, j), in [M, C] 16-bit.
 // W_e: [C, r] (forward), or [r, C] (WT, the backward's B) with in scaled by s
-// and rounded first (SCALE). A block takes 64 rows and every column; wave w
-// takes the 32-deep steps w, w + 8, ... of the reduction and the waves' sums
-// meet in LDS. Operands go straight to registers: lane (l % 16, l / 16) holds
-// eight consecutive c of its row, or of its W column, and MFMA i of a step
-// multiplies element i of each, so that no operand is transposed.
+// and rounded first (SCALE). A block takes 64 rows and every column, wave w
+// rows 16 w .. + 15 over the whole reduction; 64-deep k-tiles of in and W_e
+// stream into a ring of S LDS stages (48 KiB, three blocks per CU), one barrier
+// per k-tile, as in gmm_thin_kernel. LDS of a stage: in 128 bytes per row, chunk c of row r in
+// slot c ^ ((r >> 1) & 7); then W_e's 64 x r elements as they lie in memory,
+// or (WT) 256 bytes per row j, chunk c in slot c ^ (j % 16).
 // ---------------------------------------------------------------------------
 template <class TT, int RT, bool WT, bool SCALE>
-__global__ __launch_bounds__(LD_NT) void lora_down_kernel(const uint16_t* __restrict__ in,
+__global__ __launch_bounds__(LR_NT) void lora_down_kernel(const uint16_t* __restrict__ in,
                                                           const float* __restrict__ W,
                                                           float* __restrict__ out, int C, int r,
                                                           float s, int E,
                                                           const int64_t* __restrict__ counts) {
-  constexpr int BM = 64, MI = BM / 16, NW = LD_NT / 64;
-  constexpr int RS = 16 * RT + 1;  // row stride of the partial sums
-  __shared__ __align__(16) float part[NW * BM * RS];
+  constexpr int BM = 64, BK = 64, S = RT == 1 ? 4 : RT == 2 ? 3 : 2;
+  constexpr int T_X = BM * BK * 2, T_W = 16 * RT * BK * 4, STAGE = T_X + T_W;
+  constexpr int LD = 2 + RT;  // loads per wave and k-tile
+  __shared__ __align__(16) char lds_raw[S * STAGE];
   RowTile t;
-  if (!row_tile<BM, LD_NT>(counts, E, 1, reinterpret_cast<char*>(part), t)) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (!row_tile<BM, LR_NT>(counts, E, 1, lds_raw, t)) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int64_t row0 = t.seg0 + (int64_t)t.mt * BM;
   const int rows = (int)(t.nrows - (int64_t)t.mt * BM < BM ? t.nrows - (int64_t)t.mt * BM : BM);
-  const float* We = W + (int64_t)t.e * C * r;
-  const uint16_t* src[MI];
+  const int nkt = (C + BK - 1) / BK;
+  const i32x4 rx = make_rsrc(in + row0 * C, (int64_t)rows * C * 2);
+  const i32x4 rw = make_rsrc(W + (int64_t)t.e * C * r, (int64_t)C * r * 4);
+  uint32_t xoff[2], woff[RT];
+  int xk[2], wk[RT];
 #pragma unroll
-  for (int mi = 0; mi < MI; ++mi) {
-    const int m = 16 * mi + l16;
-    src[mi] = in + (row0 + (m < rows ? m : rows - 1)) * C;  // rows past the end: unused
+  for (int q = 0; q < 2; ++q) {
+    const int m = 16 * wave + 8 * q + (lane >> 3), c = (lane & 7) ^ ((m >> 1) & 7);
+    xk[q] = 8 * c;
+    xoff[q] = (uint32_t)(((int64_t)m * C + 8 * c) * 2);
   }
-  int jl[RT];
 #pragma unroll
-  for (int jt = 0; jt < RT; ++jt) jl[jt] = 16 * jt + l16 < r ? 16 * jt + l16 : 0;
-  f32x4 acc[MI][RT] = {};
-  const int steps = (C + 31) / 32;
-#pragma unroll 4
-  for (int st = wave; st < steps; st += NW) {
-    // Lanes past the end (C is a multiple of 8) or past the rank read a valid
-    // element and drop it: no branch around a load.
-    const int c0 = 32 * st + 8 * g;
-    const bool live = c0 < C;
-    const int cl = live ? c0 : 0;
-    uint4 xv[MI];
-    float wv[RT][8];
+  for (int q = 0; q < RT; ++q) {
+    if constexpr (WT) {
+      const int j = 4 * (RT * wave + q) + g, c = l16 ^ (j & 15);
+      wk[q] = 4 * c;
+      woff[q] = j < r ? (uint32_t)(((int64_t)j * C + 4 * c) * 4) : DM_OOB;
+    } else {
+      const int at = 16 * (64 * (RT * wave + q) + lane);  // of the k-tile's 256 r bytes
+      wk[q] = 0;
+      woff[q] = at < 256 * r ? (uint32_t)at : DM_OOB;
+    }
+  }
+  lds_char* const lds = (lds_char*)lds_raw;
+  auto issue = [&](int kt, int slot) {
+    const uint32_t base = lds_addr_of(lds) + (uint32_t)slot * STAGE;
+    const i32x4 ax = advance_rsrc(rx, (uint32_t)kt * (BK * 2));
+    const i32x4 aw = advance_rsrc(rw, (uint32_t)kt * (uint32_t)(BK * 4 * (WT ? 1 : r)));
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi) xv[mi] = *reinterpret_cast<const uint4*>(src[mi] + cl);
+    for (int q = 0; q < 2; ++q)
+      dma16(kt * BK + xk[q] < C ? xoff[q] : DM_OOB, ax, base + (uint32_t)(2 * wave + q) * 1024u);
 #pragma unroll
-    for (int jt = 0; jt < RT; ++jt) {
-      const bool ok = live && 16 * jt + l16 < r;
-      if constexpr (WT) {
-        const float4* p = reinterpret_cast<const float4*>(We + (int64_t)jl[jt] * C + cl);
-        const float4 a = p[0], b = p[1];
-        wv[jt][0] = ok ? a.x : 0.f; wv[jt][1] = ok ? a.y : 0.f;
-        wv[jt][2] = ok ? a.z : 0.f; wv[jt][3] = ok ? a.w : 0.f;
-        wv[jt][4] = ok ? b.x : 0.f; wv[jt][5] = ok ? b.y : 0.f;
-        wv[jt][6] = ok ? b.z : 0.f; wv[jt][7] = ok ? b.w : 0.f;
-      } else {
+    for (int q = 0; q < RT; ++q)
+      dma16(WT && kt * BK + wk[q] >= C ? DM_OOB : woff[q], aw,
+            base + T_X + (uint32_t)(RT * wave + q) * 1024u);
+  };
+  const bool odd = g >> 1;
+  const int row = 16 * wave + l16;
+  f32x4 acc[RT] = {};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) wv[jt][i] = We[(int64_t)(cl + i) * r + jl[jt]];
+  for (int i = 0; i < S - 1; ++i)
+    if (i < nkt) issue(i, i);
+  int slot = 0;
+  for (int kt = 0; kt < nkt; ++kt) {
+    // k-tile kt has landed once at most the later ones are outstanding.
+    const int later = nkt - 1 - kt;
+    if (S >= 4 && later >= 2) TT_WAIT_VMCNT(2 * LD);
+    else if (S >= 3 && later >= 1) TT_WAIT_VMCNT(LD);
+    else TT_WAIT_VMCNT(0);
+    TT_LDS_BARRIER();
+    if (kt + S - 1 < nkt) issue(kt + S - 1, slot == 0 ? S - 1 : slot - 1);  // the stage of kt - 1
+    lds_char* const stg = lds + slot * STAGE;
+    const lds_float* const wl = reinterpret_cast<const lds_float*>(stg + T_X);
+    // The fragments of 16 elements are read while the 16 before are multiplied.
+    uint4 xv[2];
+    float wv[2][4][RT];
+    auto read = [&](int b) {
+      xv[b & 1] = read_k(
+          stg, (uint32_t)(row * 128 + (((2 * b + (g & 1)) ^ ((row >> 1) & 7)) << 4)));
 #pragma unroll
-        for (int i = 0; i < 8; ++i) wv[jt][i] = ok ? wv[jt][i] : 0.f;
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int jt = 0; jt < RT; ++jt) {
+          const int c = 16 * b + 8 * (g & 1) + 2 * q + (g >> 1);
+          const int j = 16 * jt + l16;  // results of j >= r are not stored
+          wv[b & 1][q][jt] = WT ? wl[j * 64 + (((c >> 2) ^ (j & 15)) << 2) + (c & 3)]
+                                : wl[c * r + (j < r ? j : 0)];
+        }
+    };
+    if (16 * wave < rows) {
+      read(0);
+#pragma unroll
+      for (int b = 0; b < BK / 16; ++b) {
+        if (b + 1 < BK / 16) read(b + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t x[4] = {xv[b & 1].x, xv[b & 1].y, xv[b & 1].z, xv[b & 1].w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float a = widen1<TT, SCALE>(x[q], odd, s);
+#pragma unroll
+          for (int jt = 0; jt < RT; ++jt) acc[jt] = mfma16(a, wv[b & 1][q][jt], acc[jt]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
+    slot = slot == S - 1 ? 0 : slot + 1;
+  }
+  // Lane l holds rows 16 wave + 4 (l / 16) + 0..3, column 16 jt + l % 16.
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi) {
-      float x[8];
-      widen8<TT, SCALE>(live ? xv[mi] : uint4{0, 0, 0, 0}, s, x);
+  for (int jt = 0; jt < RT; ++jt)
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int jt = 0; jt < RT; ++jt) acc[mi][jt] = mfma16(x[i], wv[jt][i], acc[mi][jt]);
+    for (int e = 0; e < 4; ++e) {
+      const int m = 16 * wave + 4 * g + e, j = 16 * jt + l16;
+      if (m < rows && j < r) out[(row0 + m) * r + j] = acc[jt][e];
     }
-  }
-  // Lane l holds rows 16 mi + 4 (l / 16) + 0..3, column 16 jt + l % 16.
-  __syncthreads();
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-    for (int jt = 0; jt < RT; ++jt)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        part[(wave * BM + 16 * mi + 4 * g + e) * RS + 16 * jt + l16] = acc[mi][jt][e];
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < rows * r; idx += LD_NT) {
-    const int m = idx / r, j = idx - m * r;
-    const float* p = part + m * RS + j;
-    float sum = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) sum += p[w * BM * RS];
-    out[(row0 + m) * r + j] = sum;
-  }
 }
 
 // ---------------------------------------------------------------------------
 // d[m, n] = sum over j of h[m, j] W_e(j, n), h fp32 [M, r]. W_e: [r, N]
 // (forward), or [N, r] (WT, the backward's A). y = base + round(round(d) s)
 // (BASE), or y = round(d). A block takes 64 rows x 256 columns: W_e's columns
-// go to LDS once, wave w multiplies columns 64 w .. + 63 for all rows, and the
-// rounded products pass through LDS so that base and y move as whole 128-byte
-// row segments.
+// go to LDS once (row j in the order of the chain), wave w multiplies columns
+// 64 w .. + 63 for all rows, and the rounded products pass through LDS so that
+// base and y move as whole 128-byte row segments.
 // ---------------------------------------------------------------------------
 template <class TT, int RT, bool WT, bool BASE>
-__global__ __launch_bounds__(LR_NT) void lora_up_kernel(const float* __restrict__ h,
-                                                        const float* __restrict__ W,
-                                                        const uint16_t* __restrict__ base,
-                                                        uint16_t* __restrict__ y, int N, int r,
-                                                        float s, int E,
-                                                        const int64_t* __restrict__ counts,
-                                                        int tiles_n) {
+__global__ __launch_bounds__(LR_NT, RT == 2 && WT ? 3 : 1) void lora_up_kernel(
+    const float* __restrict__ h, const float* __restrict__ W, const uint16_t* __restrict__ base,
+    uint16_t* __restrict__ y, int N, int r, float s, int E, const int64_t* __restrict__ counts,
+    int tiles_n) {
   constexpr int BM = 64, BN = 256, MI = BM / 16, R = 16 * RT;
   constexpr int WS = BN + 16;  // row stride of W in LDS: four rows on distinct banks
   constexpr int LDS = R * WS * 4 > BM * BN * 2 ? R * WS * 4 : BM * BN * 2;
@@ -221,19 +273,19 @@ __global__ __launch_bounds__(LR_NT) void lora_up_kernel(const float* __restrict_
                                                (n0 + nn < N ? n0 + nn : 0));
     }
   }
-  // Step q of the reduction takes j = 4 q + l / 16.
+  // Step q of the reduction takes j = chain16(4 q + l / 16).
   float hv[MI][4 * RT];
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi) {
     const int m = 16 * mi + l16;
     const float* p = h + (row0 + (m < rows ? m : rows - 1)) * r;
 #pragma unroll
-    for (int q = 0; q < 4 * RT; ++q) hv[mi][q] = p[4 * q + g < r ? 4 * q + g : 0];
+    for (int q = 0; q < 4 * RT; ++q) hv[mi][q] = p[chain16(4 * q + g) < r ? chain16(4 * q + g) : 0];
   }
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-    for (int q = 0; q < 4 * RT; ++q) hv[mi][q] = 4 * q + g < r ? hv[mi][q] : 0.f;
+    for (int q = 0; q < 4 * RT; ++q) hv[mi][q] = chain16(4 * q + g) < r ? hv[mi][q] : 0.f;
 #pragma unroll
   for (int i = 0; i < WL; ++i) {
     const int idx = threadIdx.x + i * LR_NT;
@@ -241,10 +293,11 @@ __global__ __launch_bounds__(LR_NT) void lora_up_kernel(const float* __restrict_
       const int nn = idx / (R / 4), j = 4 * (idx % (R / 4));
       const float* const d = &wr[i].x;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) wl[(j + k) * WS + nn] = n0 + nn < N && j + k < r ? d[k] : 0.f;
+      for (int k = 0; k < 4; ++k)
+        wl[place16(j + k) * WS + nn] = n0 + nn < N && j + k < r ? d[k] : 0.f;
     } else {
       const int j = idx / (BN / 4), nn = 4 * (idx % (BN / 4));
-      *reinterpret_cast<float4*>(wl + j * WS + nn) =
+      *reinterpret_cast<float4*>(wl + place16(j) * WS + nn) =
           n0 + nn < N && j < r ? wr[i] : float4{0.f, 0.f, 0.f, 0.f};
     }
   }
@@ -295,11 +348,10 @@ __global__ __launch_bounds__(LR_NT) void lora_up_kernel(const float* __restrict_
 // ---------------------------------------------------------------------------
 // G_e[c, j] = sum over e's rows m of in[m, c] v[m, j], in [M, C] 16-bit (scaled
 // by s and rounded first with SCALE), v fp32 [M, r]; written [C, r], or [r, C]
-// (GT). A block takes 128 columns of one expert; the waves split its rows four
-// at a time and their sums meet in LDS. Lane (l % 16, l / 16) loads columns
-// 8 (l % 16) .. + 7 of row l / 16, and MFMA i multiplies element i, column
-// 8 (l % 16) + i: whole 256-byte row segments without a transpose. An expert
-// without rows gets zeros.
+// (GT). A block takes 128 columns of one expert, wave w columns 32 w .. + 31
+// over all of its rows: lane (l % 16, l / 16) loads columns 2 (l % 16) and
+// + 1 of the four rows of a step, and MFMA i multiplies column 2 (l % 16) + i,
+// so that no operand is transposed. An expert without rows gets zeros.
 // ---------------------------------------------------------------------------
 template <class TT, int RT, bool GT, bool SCALE>
 __global__ __launch_bounds__(LR_NT) void lora_wgrad_kernel(const uint16_t* __restrict__ in,
@@ -307,76 +359,80 @@ __global__ __launch_bounds__(LR_NT) void lora_wgrad_kernel(const uint16_t* __res
                                                            float* __restrict__ out, int C, int r,
                                                            float s,
                                                            const int64_t* __restrict__ counts) {
-  __shared__ __align__(16) float red[4 * 8 * 4 * 64];  // [wave][i][reg][lane], one j tile
-  __shared__ int64_t seg_part[LR_NT / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int e = blockIdx.y;
+  const int cw = blockIdx.x * 128 + 32 * wave;
+  if (cw >= C) return;
   int64_t before = 0;  // rows of the experts before e
-  for (int i = tid; i < e; i += LR_NT) before += counts[i];
+  for (int i = lane; i < e; i += 64) before += counts[i];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
-  if (lane == 0) seg_part[wave] = before;
-  __syncthreads();
-  const int64_t row0 = seg_part[0] + seg_part[1] + seg_part[2] + seg_part[3];
-  const int64_t rows = counts[e];
-  const int c0 = blockIdx.x * 128 + 8 * l16;
+  const int64_t row0 = before, rows = counts[e];
+  const int c0 = cw + 2 * l16;
   const bool live = c0 < C;  // C is a multiple of 8
-  f32x4 acc[RT][8] = {};
-#pragma unroll 4
-  for (int64_t m0 = 4 * wave; m0 < rows; m0 += 16) {
-    const int64_t m = m0 + g;
-    const bool ok = m < rows;
-    const int64_t at = row0 + (ok ? m : 0);
-    uint4 x = *reinterpret_cast<const uint4*>(in + at * C + (live ? c0 : 0));
-    float vv[RT];
+  const uint16_t* const src = in + row0 * C + (live ? c0 : 0);
+  const float* const vsrc = v + row0 * r;
+  f32x4 acc[RT][2] = {};
+  const int first = chain16(g);
+  // 16 rows are loaded while the 16 before are multiplied.
+  uint32_t x[2][4];
+  float vv[2][4][RT];
+  auto load = [&](int64_t m0, int buf) {
 #pragma unroll
-    for (int jt = 0; jt < RT; ++jt) {
-      const int j = 16 * jt + l16;
-      vv[jt] = v[at * r + (j < r ? j : 0)];
-      vv[jt] = ok && j < r ? vv[jt] : 0.f;
-    }
-    if (!ok || !live) x = uint4{0, 0, 0, 0};
-    float a[8];
-    widen8<TT, SCALE>(x, s, a);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int q = 0; q < 4; ++q) {
+      const int64_t m = m0 + first + 2 * q;  // chain16(4 q + g)
+      const int64_t at = m < rows ? m : 0;
+      x[buf][q] = *reinterpret_cast<const uint32_t*>(src + at * C);
 #pragma unroll
       for (int jt = 0; jt < RT; ++jt)
-        acc[jt][i] = GT ? mfma16(vv[jt], a[i], acc[jt][i]) : mfma16(a[i], vv[jt], acc[jt][i]);
+        vv[buf][q][jt] = vsrc[at * r + (16 * jt + l16 < r ? 16 * jt + l16 : 0)];
+    }
+  };
+  auto multiply = [&](int64_t m0, int buf) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bool ok = m0 + first + 2 * q < rows;
+      const uint32_t xq = ok && live ? x[buf][q] : 0;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float a = widen1<TT, SCALE>(xq, i == 1, s);
+#pragma unroll
+        for (int jt = 0; jt < RT; ++jt) {
+          const float b = ok && 16 * jt + l16 < r ? vv[buf][q][jt] : 0.f;
+          acc[jt][i] = GT ? mfma16(b, a, acc[jt][i]) : mfma16(a, b, acc[jt][i]);
+        }
+      }
+    }
+  };
+  if (rows > 0) load(0, 0);
+  for (int64_t m0 = 0; m0 < rows; m0 += 32) {
+    if (m0 + 16 < rows) load(m0 + 16, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(m0, 0);
+    if (m0 + 16 >= rows) break;
+    if (m0 + 32 < rows) load(m0 + 32, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(m0 + 16, 1);
   }
   float* const o = out + (int64_t)e * C * r;
 #pragma unroll
-  for (int jt = 0; jt < RT; ++jt) {
-    if (jt) __syncthreads();
+  for (int jt = 0; jt < RT; ++jt)
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) red[((wave * 8 + i) * 4 + q) * 64 + lane] = acc[jt][i][q];
-    __syncthreads();
-    // Thread (lane, wave) sums registers q = wave of the eight tiles.
-    float sum[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float* p = red + (i * 4 + wave) * 64 + lane;
-      sum[i] = (p[0] + p[8 * 4 * 64]) + (p[2 * 8 * 4 * 64] + p[3 * 8 * 4 * 64]);
-    }
-    if constexpr (GT) {
-      // Row j = 16 jt + 4 g + wave, columns 8 l16 + i.
-      const int j = 16 * jt + 4 * g + wave;
-      if (j < r && live) {
-        float4* d = reinterpret_cast<float4*>(o + (int64_t)j * C + c0);
-        d[0] = float4{sum[0], sum[1], sum[2], sum[3]};
-        d[1] = float4{sum[4], sum[5], sum[6], sum[7]};
+    for (int q = 0; q < 4; ++q) {
+      if constexpr (GT) {  // row j = 16 jt + 4 g + q, columns c0 and c0 + 1
+        const int j = 16 * jt + 4 * g + q;
+        if (j < r && live)
+          *reinterpret_cast<float2*>(o + (int64_t)j * C + c0) = float2{acc[jt][0][q], acc[jt][1][q]};
+      } else {  // columns cw + 2 (4 g + q) + i, j = 16 jt + l16
+        const int j = 16 * jt + l16, c = cw + 2 * (4 * g + q);
+        if (j < r && c < C) {
+          o[(int64_t)c * r + j] = acc[jt][0][q];
+          o[(int64_t)(c + 1) * r + j] = acc[jt][1][q];
+        }
       }
-    } else {
-      // Column 8 (4 g + wave) + i, j = 16 jt + l16.
-      const int j = 16 * jt + l16, c = blockIdx.x * 128 + 8 * (4 * g + wave);
-      if (j < r && c < C)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) o[(int64_t)(c + i) * r + j] = sum[i];
     }
-  }
 }
 
 inline hipStream_t S(void* s) { return reinterpret_cast<hipStream_t>(s); }
@@ -398,7 +454,7 @@ int64_t row_blocks(int64_t M, int E) { return M / 64 + (M < E ? M : E); }
 template <class TT, int RT, bool WT, bool SCALE>
 int launch_down(const LoraArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((lora_down_kernel<TT, RT, WT, SCALE>), dim3((unsigned)row_blocks(a.M, a.E)),
-                     dim3(LD_NT), 0, s, a.in, a.w, static_cast<float*>(a.out), a.C, a.r, a.s, a.E,
+                     dim3(LR_NT), 0, s, a.in, a.w, static_cast<float*>(a.out), a.C, a.r, a.s, a.E,
                      a.counts);
   return tt_check_launch("lora_down");
 }
