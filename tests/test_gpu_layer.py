@@ -395,3 +395,34 @@ def test_inference_forward_equals_the_separate_ops(process_ops, kind, tokens):
     with torch.no_grad():
         assert torch.equal(layer.forward_with_logits(flat.view(tokens, H), logits),
                            layer.forward_with_logits(x, logits))
+
+
+def test_inference_sizes_that_differ_keep_the_separate_ops(process_ops):
+    """Without gradients as with them: tokens of another width and FP8 scales of another shape
+    are refused on the host, experts whose weights were replaced by wider ones are served."""
+    process_ops(CudaRuntime(), OpPolicy.CUSTOM)
+    E, H, Fd, T = 8, 128, 128, 16
+    layers = {}
+    for experts in (GroupedMLP, Fp8GroupedMLP):
+        cfg = MoEConfig(hidden_size=H, num_moe_experts=E, moe_ffn_hidden_size=Fd, moe_router_topk=2,
+                        gated_linear_unit=True, activation_func=F.silu, params_dtype=torch.bfloat16)
+        layers[experts] = MoELayer(
+            cfg, None, submodules=MoESubmodules(experts=ModuleSpec(module=experts))).to(DEV)
+    g = torch.Generator().manual_seed(3)
+    logits = torch.randn(T, E, generator=g).to(DEV)
+    x = torch.randn(T, 2 * H, generator=g).bfloat16().to(DEV)
+    for layer in layers.values():
+        for width in (H // 2, 2 * H):
+            with torch.no_grad(), pytest.raises(ValueError):
+                layer.forward_with_logits(x[:, :width].contiguous(), logits)
+    fp8 = layers[Fp8GroupedMLP].experts
+    fp8.s2 = torch.ones(E, 1, 2, dtype=torch.bfloat16, device=DEV)
+    with torch.no_grad(), pytest.raises(ValueError):
+        layers[Fp8GroupedMLP].forward_with_logits(x[:, :H].contiguous(), logits)
+    plain = layers[GroupedMLP]
+    for name, shape in (("weight1", (E * H, 4 * Fd)), ("weight2", (2 * E * Fd, H))):
+        w = (torch.randn(shape, generator=g) * 0.05).bfloat16().to(DEV)
+        setattr(plain.experts, name, torch.nn.Parameter(w))
+    with torch.no_grad():
+        out = plain.forward_with_logits(x[:, :H].contiguous(), logits)
+    assert torch.equal(out, plain.forward_with_logits(x[:, :H].contiguous(), logits).detach())

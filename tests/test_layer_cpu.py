@@ -127,3 +127,72 @@ def test_folded_permutation_shape_rule():
     # the layer keeps the permutation instead of failing in forward
     assert shapes_pay(40000, 2048, 1536, 8, 600, bf)
     assert not shapes_pay(131072, 2048, 1536, 8, 1024, bf)
+
+
+def one_call_operands(fp8=False):
+    """``inference_eligible``'s operands for a layer of 4 experts (no GPU is needed to ask)."""
+    from torchturbo_amd.moe import Fp8GroupedMLP
+
+    E, H, Fd, T, k = 4, 128, 256, 3, 2
+    cfg = MoEConfig(hidden_size=H, num_moe_experts=E, moe_ffn_hidden_size=Fd, gated_linear_unit=True,
+                    activation_func=F.silu, moe_router_topk=k, params_dtype=torch.bfloat16)
+    experts = (Fp8GroupedMLP if fp8 else GroupedMLP)(E, False, cfg)
+    weights = ((experts.q1, experts.q2) if fp8 else (experts.weight1, experts.weight2))
+    return dict(experts=experts, weights=weights, scales=(experts.s1, experts.s2) if fp8 else None,
+                tokens=torch.zeros(T, H, dtype=torch.bfloat16), probs=torch.zeros(T, E),
+                expert_indices=torch.zeros(T, k, dtype=torch.int64), num_experts=E, ffn=Fd)
+
+
+def one_call(operands):
+    from torchturbo_amd.providers.hip import fused_experts
+
+    with torch.no_grad():
+        return fused_experts.inference_eligible(**operands)
+
+
+def with_weights(operands, shapes):
+    dtype = operands["weights"][0].dtype
+    operands["weights"] = tuple(torch.zeros(s, dtype=dtype) for s in shapes)
+
+
+ONE_CALL_REFUSED = {
+    "narrower tokens": lambda o: o.update(tokens=o["tokens"][:, :64].contiguous()),
+    "wider tokens": lambda o: o.update(tokens=o["tokens"].repeat(1, 2)),
+    "more tokens than routed": lambda o: o.update(tokens=o["tokens"].repeat(2, 1)),
+    "fewer probabilities' experts": lambda o: o.update(probs=o["probs"][:, :2].contiguous()),
+    "fewer probabilities' tokens": lambda o: o.update(probs=o["probs"][:2].contiguous()),
+    "another expert count": lambda o: o.update(num_experts=8),
+    "no ffn in the config": lambda o: o.update(ffn=None),
+    "wider config": lambda o: o.update(ffn=512),
+}
+
+
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("name", ONE_CALL_REFUSED)
+def test_one_call_experts_need_sizes_that_agree(name, fp8):
+    """The one-call forward of the experts gets addresses and takes every size from one operand:
+    calls whose other operands differ keep the separate ops, which refuse or serve them."""
+    operands = one_call_operands(fp8)
+    assert one_call(operands)
+    ONE_CALL_REFUSED[name](operands)
+    assert not one_call(operands)
+
+
+def test_one_call_experts_need_the_configs_weights():
+    for shapes in (((512, 256), (512, 128)), ((512, 512), (512, 128)), ((256, 512), (1024, 128)),
+                   ((512, 512), (1024, 64)), ((4, 128, 512), (1024, 128))):
+        operands = one_call_operands()
+        with_weights(operands, shapes)
+        assert not one_call(operands), shapes
+    for shapes in (((4, 256, 128), (4, 128, 256)), ((4, 512, 128), (4, 128, 128)),
+                   ((2, 512, 128), (4, 128, 256)), ((4, 512, 64), (4, 128, 256))):
+        operands = one_call_operands(fp8=True)
+        with_weights(operands, shapes)
+        assert not one_call(operands), shapes
+    for shapes in (((4, 4, 1), (4, 1, 1)), ((4, 2, 1), (4, 1, 2)), ((1, 4, 1), (4, 1, 2))):
+        operands = one_call_operands(fp8=True)
+        operands["scales"] = tuple(torch.zeros(s, dtype=torch.bfloat16) for s in shapes)
+        assert one_call(operands) == (shapes == ((4, 4, 1), (4, 1, 2))), shapes
+    operands = one_call_operands(fp8=True)
+    operands["experts"].master2 = torch.nn.Parameter(torch.zeros(4, 128, 128, dtype=torch.bfloat16))
+    assert not one_call(operands)

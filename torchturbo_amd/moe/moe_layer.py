@@ -114,8 +114,9 @@ class MoELayer(BaseMoELayer):
             return None
         e = self.experts
         fp8 = type(e) is Fp8GroupedMLP
-        if not fp8 and (type(e) is not GroupedMLP or not self.config.gated_linear_unit
-                        or self.config.moe_apply_probs_on_input):
+        cfg = self.config
+        if not fp8 and (type(e) is not GroupedMLP or not cfg.gated_linear_unit
+                        or cfg.moe_apply_probs_on_input):
             return None
         if type(self.token_dispatcher) is not MoEAlltoAllTokenDispatcher:
             return None
@@ -134,9 +135,9 @@ class MoELayer(BaseMoELayer):
         from ..providers.hip import fused_experts
         weights = (e.q1, e.q2) if fp8 else (e.weight1, e.weight2)
         scales = (e.s1, e.s2) if fp8 else None
-        if not fused_experts.inference_eligible(e, weights, scales, tokens, probs, expert_indices):
+        if not fused_experts.inference_eligible(e, weights, scales, tokens, probs, expert_indices,
+                                                self.num_local_experts, cfg.moe_ffn_hidden_size):
             return None
-        cfg = self.config
         output, counts = fused_experts.experts_forward(
             tokens, probs, expert_indices, self.num_local_experts, cfg.moe_ffn_hidden_size,
             weights, scales, F.silu if fp8 else cfg.activation_func,

@@ -240,11 +240,31 @@ def _hooked(module) -> bool:
                 or m._global_forward_pre_hooks or "forward" in module.__dict__)
 
 
-def inference_eligible(experts, weights, scales, tokens, probs, expert_indices) -> bool:
+def _sizes_agree(experts, weights, scales, tokens, probs, num_experts, ffn) -> bool:
+    """Whether every operand has the size that ``tt_moe_experts_fwd`` takes from another one
+    or from the config: it gets addresses and cannot check. The separate ops refuse the rest,
+    or serve it from the weights' own widths."""
+    T, H = tokens.shape
+    E, cfg = num_experts, experts.config
+    if not ffn or experts.num_local_experts != E or cfg.hidden_size != H:
+        return False
+    if tuple(probs.shape) != (T, E):
+        return False
+    if scales is None:
+        return [tuple(w.shape) for w in weights] == [(E * H, 2 * ffn), (E * ffn, H)]
+    want = [(E, 2 * ffn, H), (E, H, ffn)]
+    blocks = [(E, -(-n // 128), -(-k // 128)) for _, n, k in want]
+    masters = (experts.master1, experts.master2)
+    return ([tuple(w.shape) for w in weights] == want and [tuple(s.shape) for s in scales] == blocks
+            and all(m is None or tuple(m.shape) == n for m, n in zip(masters, want)))
+
+
+def inference_eligible(experts, weights, scales, tokens, probs, expert_indices, num_experts,
+                       ffn) -> bool:
     """Whether ``experts_forward`` stands in for permute -> ``experts`` -> unpermute: no
     gradients, tangents, function transforms or tracing that the separate ops' autograd
     functions would have to see, no hooks on the experts, plain contiguous 16-bit tensors
-    on one device, and no input checks asked for."""
+    on one device whose sizes agree, and no input checks asked for."""
     if (torch.is_grad_enabled() or checks.enabled() or torch.compiler.is_compiling()
             or torch._C._are_functorch_transforms_active()
             or torch.autograd.forward_ad._current_level >= 0 or _hooked(experts)):
@@ -252,7 +272,9 @@ def inference_eligible(experts, weights, scales, tokens, probs, expert_indices) 
     if expert_indices is None or tokens.dim() != 2 or expert_indices.dim() != 2:
         return False
     T, k = expert_indices.shape
-    if not 0 < T * k <= MAX_INFERENCE_ROWS or tokens.shape[0] != T or probs.shape[0] != T:
+    if not 0 < T * k <= MAX_INFERENCE_ROWS or tokens.shape[0] != T:
+        return False
+    if not _sizes_agree(experts, weights, scales, tokens, probs, num_experts, ffn):
         return False
     half = (torch.bfloat16, torch.float16)
     if not (_plain(tokens, half) and _plain(probs, (torch.float32, *half))
