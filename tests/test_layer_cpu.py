@@ -196,3 +196,11 @@ def test_one_call_experts_need_the_configs_weights():
     operands = one_call_operands(fp8=True)
     operands["experts"].master2 = torch.nn.Parameter(torch.zeros(4, 128, 128, dtype=torch.bfloat16))
     assert not one_call(operands)
+
+
+@pytest.mark.parametrize("name", ["forward", "activation_func", "activation_func_with_probs"])
+def test_one_call_experts_run_replaced_methods(name):
+    """A method replaced on the experts is called, so the separate ops stay."""
+    operands = one_call_operands()
+    setattr(operands["experts"], name, lambda *a: None)
+    assert not one_call(operands)

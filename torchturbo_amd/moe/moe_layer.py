@@ -114,9 +114,11 @@ class MoELayer(BaseMoELayer):
             return None
         e = self.experts
         fp8 = type(e) is Fp8GroupedMLP
-        cfg = self.config
-        if not fp8 and (type(e) is not GroupedMLP or not cfg.gated_linear_unit
-                        or cfg.moe_apply_probs_on_input):
+        if not fp8 and type(e) is not GroupedMLP:
+            return None
+        cfg = e.config
+        if not fp8 and (not cfg.gated_linear_unit or cfg.moe_apply_probs_on_input
+                        or cfg.activation_func not in (F.silu, F.gelu)):
             return None
         if type(self.token_dispatcher) is not MoEAlltoAllTokenDispatcher:
             return None

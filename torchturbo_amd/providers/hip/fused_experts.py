@@ -236,8 +236,9 @@ def _plain(t, dtypes) -> bool:
 
 def _hooked(module) -> bool:
     m = torch.nn.modules.module
+    own = ("forward", "activation_func", "activation_func_with_probs")
     return bool(module._forward_hooks or module._forward_pre_hooks or m._global_forward_hooks
-                or m._global_forward_pre_hooks or "forward" in module.__dict__)
+                or m._global_forward_pre_hooks or any(n in module.__dict__ for n in own))
 
 
 def _sizes_agree(experts, weights, scales, tokens, probs, num_experts, ffn) -> bool:
