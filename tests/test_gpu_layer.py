@@ -426,3 +426,22 @@ def test_inference_sizes_that_differ_keep_the_separate_ops(process_ops):
     with torch.no_grad():
         out = plain.forward_with_logits(x[:, :H].contiguous(), logits)
     assert torch.equal(out, plain.forward_with_logits(x[:, :H].contiguous(), logits).detach())
+
+
+def test_inference_leaves_the_dispatcher_as_the_separate_ops_do(process_ops):
+    """The dispatcher's record of a [S, B, H] input after the one-call forward."""
+    process_ops(CudaRuntime(), OpPolicy.CUSTOM)
+    cfg = MoEConfig(hidden_size=128, num_moe_experts=8, moe_ffn_hidden_size=64, moe_router_topk=2,
+                    gated_linear_unit=True, activation_func=F.silu, params_dtype=torch.bfloat16)
+    layer = MoELayer(cfg, None, submodules=MoESubmodules(experts=ModuleSpec(module=GroupedMLP))).to(DEV)
+    x = torch.randn(6, 2, 128, device=DEV).bfloat16()
+    seen = []
+    for hook in (None, lambda *a: None):
+        if hook is not None:  # keeps the separate ops
+            layer.experts.register_forward_hook(hook)
+        layer.token_dispatcher.hidden_shape = layer.token_dispatcher.hidden_shape_before_permute = None
+        with torch.no_grad():
+            assert layer.forward_with_logits(x, torch.randn(12, 8, device=DEV)).shape == x.shape
+        d = layer.token_dispatcher
+        seen.append((d.hidden_shape, d.hidden_shape_before_permute, d.permutation_row_indices))
+    assert seen[0] == seen[1] == (x.shape, (12, 128), None)

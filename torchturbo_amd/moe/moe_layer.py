@@ -106,10 +106,11 @@ class MoELayer(BaseMoELayer):
         return fused_experts.eligible(tokens, self.experts.weight1, expert_indices.shape[1],
                                       self.num_local_experts)
 
-    def _inference_experts(self, tokens, probs, expert_indices):
+    def _inference_experts(self, hidden_states, probs, expert_indices):
         """The experts' output for a small batch without gradients, in one native call where
         the HIP providers serve the ops it stands for (the conditions are in
         ``providers.hip.fused_experts.inference_eligible``); None otherwise."""
+        tokens = hidden_states.view(-1, hidden_states.shape[-1])
         if torch.is_grad_enabled() or not tokens.is_cuda:
             return None
         e = self.experts
@@ -147,8 +148,8 @@ class MoELayer(BaseMoELayer):
             False if fp8 else cfg.moe_swiglu_clamp_gate_after_activation)
         d = self.token_dispatcher
         d.tokens_per_expert = counts
-        d.hidden_shape = d.hidden_shape_before_permute = tokens.shape
-        return output
+        d.hidden_shape, d.hidden_shape_before_permute = hidden_states.shape, tokens.shape
+        return output.view(hidden_states.shape)
 
     def _experts_and_combine(self, hidden_states, probs, routing_map, expert_indices):
         flat = hidden_states.view(-1, hidden_states.shape[-1])
@@ -161,10 +162,8 @@ class MoELayer(BaseMoELayer):
             self.token_dispatcher.tokens_per_expert = counts
             output = tokens.view(hidden_states.shape).to(hidden_states.dtype)
         else:
-            output = self._inference_experts(flat, probs, expert_indices)
-            if output is not None:
-                output = output.view(hidden_states.shape)
-            else:
+            output = self._inference_experts(hidden_states, probs, expert_indices)
+            if output is None:
                 output = self._dispatched_experts(hidden_states, probs, routing_map,
                                                   expert_indices)
         if self.shared_expert is not None:
