@@ -1649,3 +1649,31 @@ def test_router_losses_in_one_op_match_the_sums(process_ops, monkeypatch, score,
             torch.testing.assert_close(s0[name], s1[name], rtol=2.0 ** -23 * (16 + E), atol=0)
         bound = 2.0 ** -23 * (16 + E) * float(g1.abs().max())
         assert float((g0 - g1).abs().max()) <= bound and float(g1.abs().max()) > 0
+
+
+def test_router_loss_metrics_may_be_changed_in_place(process_ops):
+    """The unscaled metrics are tensors of their own: averaged in place between forward and
+    backward (an all-reduce of a popped metric), they leave the gradients as they are."""
+    from torchturbo_amd.moe import MoEConfig, TopKRouter
+    from torchturbo_amd.runtime import CudaRuntime
+
+    process_ops(CudaRuntime(), OpPolicy.CUSTOM)
+    cfg = MoEConfig(hidden_size=64, num_moe_experts=32, moe_router_topk=4, moe_router_dtype="fp32",
+                    moe_aux_loss_coeff=0.02, moe_z_loss_coeff=0.01, params_dtype=torch.bfloat16)
+    router = TopKRouter(cfg).to(DEV)
+    x = torch.randn(100, 64, device=DEV).bfloat16()
+    got = []
+    for change in (False, True):
+        logits = (x.float() @ router.weight.float().t()).detach().requires_grad_()
+        probs, _, _ = router.routing(logits)
+        metrics = router.pop_metrics()
+        values = {k: float(v) for k, v in metrics.items()}
+        if change:
+            for name in ("aux_loss", "z_loss"):
+                metrics[name].div_(2).add_(1)
+            assert {k: float(v) for k, v in metrics.items()} == pytest.approx(
+                {k: v if k.endswith("scaled") else v / 2 + 1 for k, v in values.items()}, rel=1e-6)
+        (probs * 0).sum().backward()
+        got.append((logits.grad, values))
+    assert torch.equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
+    assert got[0][0].abs().max() > 0

@@ -259,7 +259,10 @@ class RouterLosses(torch.autograd.Function):
         ctx.save_for_backward(logits, counts, losses)
         ctx.sf = sf
         ctx.set_materialize_grads(False)
-        aux, aux_raw, z, z_raw = losses[:4].unbind()
+        # Tensors with version counters of their own, not views of what is saved here: a metric
+        # changed in place (an all-reduce of it) leaves the backward valid. The backward reads
+        # the factors behind the four.
+        aux, aux_raw, z, z_raw = (v.view(()) for v in losses.unsafe_split(1)[:4])
         ctx.mark_non_differentiable(aux_raw, z_raw)
         return aux, z, aux_raw, z_raw
 
