@@ -445,3 +445,23 @@ def test_inference_leaves_the_dispatcher_as_the_separate_ops_do(process_ops):
         d = layer.token_dispatcher
         seen.append((d.hidden_shape, d.hidden_shape_before_permute, d.permutation_row_indices))
     assert seen[0] == seen[1] == (x.shape, (12, 128), None)
+
+
+def test_requantize_into_buffers_elsewhere(process_ops):
+    """Masters on the GPU, codes and scales on the host: the bytes of buffers on the GPU."""
+    process_ops(CudaRuntime(), OpPolicy.CUSTOM)
+    cfg = MoEConfig(hidden_size=128, num_moe_experts=3, moe_ffn_hidden_size=128,
+                    gated_linear_unit=True, activation_func=F.silu, params_dtype=torch.bfloat16)
+    mlp = Fp8GroupedMLP(3, False, cfg).to(DEV)
+    with torch.no_grad():
+        for m in (mlp.master1, mlp.master2):
+            m.copy_(torch.randn(m.shape, device=DEV) * 0.02)
+    mlp.requantize()
+    names = ("q1", "s1", "q2", "s2")
+    want = [getattr(mlp, n).cpu() for n in names]
+    for n in names:
+        setattr(mlp, n, torch.zeros_like(getattr(mlp, n), device="cpu"))
+    mlp.requantize()
+    for n, w in zip(names, want):
+        got = getattr(mlp, n)
+        assert not got.is_cuda and torch.equal(got.view(torch.uint8), w.view(torch.uint8)), n

@@ -4,8 +4,8 @@
 block scales of a weight in one pass over it, the bytes that the torch
 composition in ``Fp8GroupedMLP.requantize`` gives (the inverse of
 ``scripts/dequant/bailing.py:57-102``), and returns True. Operands the kernel
-does not cover (weights that are not bf16, tensors that are not contiguous)
-return False and are left to the caller.
+does not cover (weights that are not bf16, tensors that are not contiguous or
+not all on the weight's GPU) return False and are left to the caller.
 """
 
 from __future__ import annotations
@@ -17,7 +17,6 @@ from ... import _lib as L
 from ...dispatch import OpImpl, OpImplKind, register_op
 from ...runtime import TurboDevice
 from . import PRIORITY
-from ._functions import require_cuda
 from .available import hip_available
 
 
@@ -28,6 +27,8 @@ class HipQuantizeFp8Blocks(OpImpl):
         return hip_available()
 
     def __call__(self, weight, q, scale) -> bool:
+        if not (weight.is_cuda and q.device == weight.device == scale.device):
+            return False
         if (weight.dtype != torch.bfloat16 or q.dtype != torch.float8_e4m3fn
                 or scale.dtype not in (torch.bfloat16, torch.float32)
                 or not (weight.is_contiguous() and q.is_contiguous() and scale.is_contiguous())
@@ -37,9 +38,8 @@ class HipQuantizeFp8Blocks(OpImpl):
         if (R % 128 or C % 128 or q.shape != weight.shape
                 or scale.shape != (E, R // 128, C // 128)):
             return False
-        dev = require_cuda(weight, q, scale)
         L.call("tt_fp8_quantize_blocks", L.ptr(weight), L.dtype_code(weight.dtype), E, R, C,
-               L.ptr(q), L.ptr(scale), L.dtype_code(scale.dtype), L.stream(dev))
+               L.ptr(q), L.ptr(scale), L.dtype_code(scale.dtype), L.stream(weight.device))
         # Written in place: a backward that saved the old values must see it.
         increment_version(q)
         increment_version(scale)
