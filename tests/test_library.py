@@ -62,6 +62,8 @@ def test_library_exports_every_declared_symbol(lib):
     ("tt_gmm_fwd_gather", (None, 8, None, None, 0, 16, 128, 16, 2, 0, None, None, None), "dtype"),
     ("tt_route_index", (None, 4, 2, 8, None, 0, None, None, None, None, None, 0, None),
      "workspace"),
+    ("tt_moe_experts_fwd", (None, 1, 1, 128, None, 16, 0, 1, 2, None, None, 16, 16, 2, 128, -1, 0.0,
+                            0, None, None, None, 0, None), "scales must be bf16 or f32"),
     ("tt_sort_chunks", (None, 0, 4, 4, None, None, 5000, None, 0, None, None, None), "4096"),
 ])
 def test_invalid_arguments_fail_before_any_launch(lib, name, args, msg):

@@ -49,6 +49,8 @@ extern "C" int tt_moe_experts_fwd(const void* x, int dtype, int64_t num_tokens, 
              "moe_experts: bad sizes");
   TT_REQUIRE((scale1 == nullptr) == (scale2 == nullptr), "moe_experts: both scales or none");
   TT_REQUIRE(scale1 == nullptr || dtype == TT_BF16, "moe_experts: FP8 experts take bf16 tokens");
+  TT_REQUIRE(scale1 == nullptr || scale_dtype == TT_BF16 || scale_dtype == TT_F32,
+             "moe_experts: scales must be bf16 or f32");
   TT_REQUIRE(probs != nullptr && tt_elem_size(probs_dtype) <= 4 && tt_elem_size(probs_dtype) >= 2,
              "moe_experts: probabilities must be f32, bf16 or f16");
   if (num_tokens == 0) return TT_OK;
