@@ -1617,6 +1617,33 @@ def test_lora_residual_bits_of_the_composition(hip_ops, counts, K, N, r, dtype):
         assert torch.equal(v, w), name
 
 
+@pytest.mark.parametrize("which", range(4), ids=["base", "x", "a", "b"])
+def test_lora_residual_leaves_unaligned_operands_to_the_composition(hip_ops, which):
+    """An operand that starts between 16-byte lines (an adapter in a flat buffer) is left to the
+    composition; an unaligned gradient is copied."""
+    E, K, N, r = 2, 64, 32, 8
+    counts = torch.tensor([5, 9], device=DEV)
+    shapes = ((14, N), (14, K), (E, K, r), (E, r, N))
+    leaves = [torch.randn(s, device=DEV) if i > 1 else torch.randn(s, device=DEV).bfloat16()
+              for i, s in enumerate(shapes)]
+    want = hip_ops.lora_residual(*leaves, counts, 0.5)
+
+    def shifted(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:]
+        return flat.copy_(t.reshape(-1)).view(t.shape)
+
+    moved = [shifted(t) if i == which else t for i, t in enumerate(leaves)]
+    assert hip_ops.lora_residual(*moved, counts, 0.5) is None
+    strided = [t if i != which else torch.stack([t, t], dim=-1)[..., 0] for i, t in enumerate(leaves)]
+    assert torch.equal(hip_ops.lora_residual(*strided, counts, 0.5), want)  # copied
+    for t in leaves:
+        t.requires_grad_()
+    dy = torch.randn(14, N, device=DEV).bfloat16()
+    y = hip_ops.lora_residual(*leaves, counts, 0.5)
+    grads = [torch.autograd.grad(y, leaves, g, retain_graph=True) for g in (dy, shifted(dy))]
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
 @pytest.mark.parametrize("aux,z", [(0.01, 0.001), (0.02, 0.0), (0.0, 0.003)])
 @pytest.mark.parametrize("score,T,E,k", [("softmax", 777, 33, 3), ("sigmoid", 1, 64, 8), ("sigmoid", 2500, 256, 8)])
 def test_router_losses_in_one_op_match_the_sums(process_ops, monkeypatch, score, T, E, k, aux, z):

@@ -4,7 +4,7 @@
 ``base + grouped_matmul(grouped_matmul(x.to(a.dtype), a), b).to(base.dtype) * scaling``
 (``engine/peft/lora.py:640-725``) with the same roundings, without the fp32
 copy of ``x`` and the fp32 product behind it; ``supported`` says which operands
-it takes (16-bit rows, fp32 adapters of rank 64 or less).
+it takes (16-bit rows, fp32 adapters of rank 64 or less, 16-byte aligned).
 """
 
 from __future__ import annotations
@@ -49,6 +49,8 @@ class LoRAResidual(torch.autograd.Function):
         need = ctx.needs_input_grad
         E, K, r = a.shape
         g = dy.to(x.dtype).contiguous()
+        if not aligned(g):
+            g = g.clone()
         M, N = g.shape
         dev, code = x.device, L.dtype_code(x.dtype)
         st = L.stream(dev)
@@ -72,13 +74,19 @@ class LoRAResidual(torch.autograd.Function):
         return dy if need[0] else None, dx, da, db, None, None
 
 
+def aligned(t) -> bool:
+    """Whether the kernels can read ``t``: a tensor that is not contiguous is copied first."""
+    return t.data_ptr() % 16 == 0 or not t.is_contiguous()
+
+
 def supported(base, x, a, b) -> bool:
     r = a.shape[-1]
     return (base.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and base.dtype == x.dtype
             and base.dim() == 2 and x.dim() == 2 and a.dtype == b.dtype == torch.float32
             and 1 <= r <= MAX_RANK and x.shape[1] % 8 == 0 and base.shape[1] % 8 == 0
             and x.shape[0] == base.shape[0] and a.shape[1] == x.shape[1]
-            and b.shape[1:] == (r, base.shape[1]) and a.shape[0] == b.shape[0])
+            and b.shape[1:] == (r, base.shape[1]) and a.shape[0] == b.shape[0]
+            and all(aligned(t) for t in (base, x, a, b)))
 
 
 @register_op(op_name="lora_residual", impl_name="hip_lora_residual", kind=OpImplKind.CUSTOM,
