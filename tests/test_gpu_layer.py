@@ -465,3 +465,41 @@ def test_requantize_into_buffers_elsewhere(process_ops):
     for n, w in zip(names, want):
         got = getattr(mlp, n)
         assert not got.is_cuda and torch.equal(got.view(torch.uint8), w.view(torch.uint8)), n
+
+
+def test_lora_residual_honours_a_chosen_grouped_matmul(process_ops, monkeypatch):
+    """With ``grouped_matmul`` overridden, the adapters' products run through it too."""
+    import sys
+    import types
+
+    from torchturbo_amd.dispatch import (OpImplKind, add_provider_package, get_or_create_ops,
+                                         register_op, remove_provider_package)
+    from torchturbo_amd.moe import GroupedMLPLoRA
+    from torchturbo_amd.providers.hip.grouped_matmul import HipGroupedMatmul
+    from torchturbo_amd.runtime import TurboDevice
+
+    calls = []
+
+    @register_op(op_name="grouped_matmul", impl_name="counting_grouped_matmul",
+                 kind=OpImplKind.CUSTOM, priority=-1, devices=(TurboDevice.CUDA,))
+    class Counting(HipGroupedMatmul):
+        def __call__(self, *args, **kwargs):
+            calls.append(args[1].dtype)
+            return super().__call__(*args, **kwargs)
+
+    module = types.ModuleType("counting_provider")
+    Counting.__module__ = module.__name__
+    module.Counting = Counting
+    monkeypatch.setitem(sys.modules, module.__name__, module)
+    add_provider_package(module.__name__)
+    try:
+        get_or_create_ops(device_runtime=CudaRuntime(), default_policy=OpPolicy.CUSTOM,
+                          overrides={"grouped_matmul": "counting_grouped_matmul"})
+        cfg = MoEConfig(hidden_size=64, moe_ffn_hidden_size=64, gated_linear_unit=True,
+                        activation_func=F.silu, params_dtype=torch.bfloat16)
+        lora = GroupedMLPLoRA(GroupedMLP(2, False, cfg), "default", r=4, lora_alpha=8).to(DEV)
+        x = torch.randn(10, 64, device=DEV).bfloat16()
+        lora(x, torch.tensor([4, 6], device=DEV), torch.rand(10, device=DEV))
+    finally:
+        remove_provider_package(module.__name__)
+    assert calls.count(torch.bfloat16) == 2 and calls.count(torch.float32) == 4

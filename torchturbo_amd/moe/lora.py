@@ -267,7 +267,9 @@ class GroupedMLPLoRA(nn.Module, _TunerBase):
         """``base`` plus adapter ``name``'s residual of ``x``."""
         a, b = a_group[name], b_group[name]
         xd, scale = self.lora_dropout[name](x), self.scaling[name]
-        if x.is_cuda and op_resolves("lora_residual"):
+        # In place of the HIP grouped product only: another one chosen for it is called.
+        if (x.is_cuda and op_resolves("lora_residual")
+                and ops.selected_impl_name("grouped_matmul") == "hip_grouped_matmul"):
             y = ops.lora_residual(base, xd, a.weight, b.weight, counts, scale)
             if y is not None:
                 return y
