@@ -204,3 +204,17 @@ def test_one_call_experts_run_replaced_methods(name):
     operands = one_call_operands()
     setattr(operands["experts"], name, lambda *a: None)
     assert not one_call(operands)
+
+
+def test_gathering_products_check_the_feature_width():
+    """The GEMMs that gather their rows get addresses: rows of another width than the weights'
+    are refused on the host, as the grouped product refuses them."""
+    from torchturbo_amd.providers.hip.fused_experts import GatherGroupedMatmul, GroupedMatmulCombine
+
+    counts, rows = torch.tensor([2, 1]), torch.tensor([[0], [1], [2]], dtype=torch.int32)
+    x, w = torch.zeros(3, 64, dtype=torch.bfloat16), torch.zeros(2, 128, 8, dtype=torch.bfloat16)
+    for trans_b, weight in ((False, w), (True, w.transpose(1, 2).contiguous())):
+        with pytest.raises(ValueError, match="64 features, weight expects 128"):
+            GatherGroupedMatmul.apply(x, weight, counts, rows, rows.view(-1), trans_b)
+        with pytest.raises(ValueError, match="64 features, weight expects 128"):
+            GroupedMatmulCombine.apply(x, weight, counts, rows, rows.view(-1), trans_b)

@@ -56,6 +56,14 @@ def device_counts(counts, num_experts: int, device: torch.device, m: int | None 
     return torch.tensor(counts, dtype=torch.int64, device=device)
 
 
+def check_features(features: int, w: torch.Tensor, trans_b: bool) -> None:
+    """``ValueError`` unless the rows are as wide as the weights [E, in, out] (or [E, out, in])
+    expect; the kernels get addresses."""
+    expected = w.shape[2] if trans_b else w.shape[1]
+    if expected != features:
+        raise ValueError(f"grouped_matmul: x has {features} features, weight expects {expected}")
+
+
 # ---------------------------------------------------------------------------
 # Router
 # ---------------------------------------------------------------------------
@@ -501,9 +509,7 @@ class GroupedMatmul(torch.autograd.Function):
         E = w.shape[0]
         M, K = x.shape
         N = w.shape[1] if trans_b else w.shape[2]
-        kw = w.shape[2] if trans_b else w.shape[1]
-        if kw != K:
-            raise ValueError(f"grouped_matmul: x has {K} features, weight expects {kw}")
+        check_features(K, w, trans_b)
         if x.dtype != w.dtype:
             raise ValueError("grouped_matmul: x and weight dtypes differ")
         y = x.new_empty((M, N))
