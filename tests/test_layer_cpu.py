@@ -206,9 +206,9 @@ def test_one_call_experts_run_replaced_methods(name):
     assert not one_call(operands)
 
 
-def test_gathering_products_check_the_feature_width():
-    """The GEMMs that gather their rows get addresses: rows of another width than the weights'
-    are refused on the host, as the grouped product refuses them."""
+def test_gathering_products_check_their_operands():
+    """The GEMMs that gather their rows get addresses: rows of another width or dtype than the
+    weights' are refused on the host, as the grouped product refuses them."""
     from torchturbo_amd.providers.hip.fused_experts import GatherGroupedMatmul, GroupedMatmulCombine
 
     counts, rows = torch.tensor([2, 1]), torch.tensor([[0], [1], [2]], dtype=torch.int32)
@@ -218,3 +218,8 @@ def test_gathering_products_check_the_feature_width():
             GatherGroupedMatmul.apply(x, weight, counts, rows, rows.view(-1), trans_b)
         with pytest.raises(ValueError, match="64 features, weight expects 128"):
             GroupedMatmulCombine.apply(x, weight, counts, rows, rows.view(-1), trans_b)
+        wide = torch.zeros(3, 128)
+        with pytest.raises(ValueError, match="dtypes differ"):
+            GatherGroupedMatmul.apply(wide, weight, counts, rows, rows.view(-1), trans_b)
+        with pytest.raises(ValueError, match="dtypes differ"):
+            GroupedMatmulCombine.apply(wide, weight, counts, rows, rows.view(-1), trans_b)

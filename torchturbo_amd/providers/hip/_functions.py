@@ -56,12 +56,14 @@ def device_counts(counts, num_experts: int, device: torch.device, m: int | None 
     return torch.tensor(counts, dtype=torch.int64, device=device)
 
 
-def check_features(features: int, w: torch.Tensor, trans_b: bool) -> None:
-    """``ValueError`` unless the rows are as wide as the weights [E, in, out] (or [E, out, in])
-    expect; the kernels get addresses."""
+def check_weight(x: torch.Tensor, w: torch.Tensor, trans_b: bool) -> None:
+    """``ValueError`` unless rows ``x`` [M, in] are as wide as the weights [E, in, out] (or
+    [E, out, in]) expect, in their dtype; the kernels get addresses."""
     expected = w.shape[2] if trans_b else w.shape[1]
-    if expected != features:
-        raise ValueError(f"grouped_matmul: x has {features} features, weight expects {expected}")
+    if expected != x.shape[1]:
+        raise ValueError(f"grouped_matmul: x has {x.shape[1]} features, weight expects {expected}")
+    if x.dtype != w.dtype:
+        raise ValueError("grouped_matmul: x and weight dtypes differ")
 
 
 # ---------------------------------------------------------------------------
@@ -509,9 +511,7 @@ class GroupedMatmul(torch.autograd.Function):
         E = w.shape[0]
         M, K = x.shape
         N = w.shape[1] if trans_b else w.shape[2]
-        check_features(K, w, trans_b)
-        if x.dtype != w.dtype:
-            raise ValueError("grouped_matmul: x and weight dtypes differ")
+        check_weight(x, w, trans_b)
         y = x.new_empty((M, N))
         if M > 0:
             L.call("tt_gmm_fwd", L.ptr(x), L.ptr(w), L.dtype_code(x.dtype), M, K, N, E, int(trans_b),

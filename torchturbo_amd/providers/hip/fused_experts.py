@@ -32,7 +32,7 @@ import torch.nn.functional as F
 
 from ... import _lib as L
 from ... import checks
-from ._functions import check_features, route_index
+from ._functions import check_weight, route_index
 from .moe_permutation import _check_map_matches_indices
 
 
@@ -78,7 +78,7 @@ class GatherGroupedMatmul(torch.autograd.Function):
         M = token_of_row.shape[0]
         E = w.shape[0]
         N = w.shape[1] if trans_b else w.shape[2]
-        check_features(K, w, trans_b)
+        check_weight(tokens, w, trans_b)
         y = tokens.new_empty((M, N))
         if M > 0:
             L.call("tt_gmm_fwd_gather", L.ptr(tokens), T, L.ptr(token_of_row), L.ptr(w),
@@ -128,7 +128,7 @@ class GroupedMatmulCombine(torch.autograd.Function):
         T, topk = rows.shape
         E = w.shape[0]
         N = w.shape[1] if trans_b else w.shape[2]
-        check_features(K, w, trans_b)
+        check_weight(act, w, trans_b)
         dev = act.device
         code = L.dtype_code(act.dtype)
         y = act.new_empty((M, N))
