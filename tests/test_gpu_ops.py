@@ -287,7 +287,10 @@ def test_router_gate_small_batches_equal_the_one_kernel_gate(H, E, dtype, rdt):
 
 @pytest.mark.parametrize("T,E,k", [(1, 8, 2), (63, 64, 8), (64, 128, 8), (65, 1000, 16), (256, 33, 1),
                                    (257, 128, 8), (1000, 300, 6), (1024, 256, 16), (1536, 320, 8),
-                                   (1537, 64, 4), (513, 1097, 2), (700, 2048, 3)])
+                                   (1537, 64, 4), (513, 1097, 2), (700, 2048, 3),
+                                   # every table width of the kernel above eight ids
+                                   (300, 40, 9), (1400, 64, 10), (1536, 33, 11), (257, 128, 12),
+                                   (1000, 70, 13), (700, 64, 14), (1300, 96, 15)])
 def test_route_index_small_batches(T, E, k):
     """The one-launch routing index (up to 1536 tokens) and sizes just past its limits: rows,
     tokens, counts, packed probabilities and rejected slots (ids out of range, repeats),

@@ -1019,7 +1019,9 @@ __global__ __launch_bounds__(kIdxBlock) void route_rank_kernel(
 // kernels / this one: 1 token 15.4 / 8.1 us, 256 18.4 / 10.4, 1000 19.2 / 15.1,
 // 1531 19.8 / 18.0, 2048 19.8 / 20.5; E 64, k 16: 48 31.9 / 14.2, 1531 45.2 /
 // 40.1. (One block of 1024 threads for the whole batch took 31 us at 1000
-// tokens: one CU's scattered accesses.)
+// tokens: one CU's scattered accesses.) The search for repeated ids goes with
+// the square of the table width KMAX: E 128, k 9 at 1300 tokens three kernels
+// 19.8, here 27.6 us with 16 and 17.8 with 10; k 12 24.9, 30.1 and 23.2 with 12.
 template <int KMAX>
 __global__ __launch_bounds__(kIdxBlock) void route_small_kernel(
     const int64_t* __restrict__ ids, int T, int K, int E, const void* __restrict__ probs,
@@ -1539,6 +1541,9 @@ int route_index_run(const int64_t* expert_indices, int64_t num_tokens, int32_t t
                      packed_probs, tokens_per_expert, bad_total)
     if (topk <= 2) TT_SMALL(2);
     else if (topk <= 8) TT_SMALL(8);
+    else if (topk <= 10) TT_SMALL(10);
+    else if (topk <= 12) TT_SMALL(12);
+    else if (topk <= 14) TT_SMALL(14);
     else TT_SMALL(16);
 #undef TT_SMALL
     return tt_check_launch("route_small");
