@@ -285,6 +285,59 @@ def test_router_gate_small_batches_equal_the_one_kernel_gate(H, E, dtype, rdt):
             assert torch.equal(got, ref[:T]), T
 
 
+@pytest.mark.parametrize("dtype,rdt", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("E", [32, 64, 96, 160, 224, 256])
+def test_router_gate_tile_shapes_equal_the_one_kernel_gate(E, dtype, rdt):
+    """The split gate on both sides of its tile rules (32x32, 32x64 and 64x64 blocks; the last
+    block of an odd number of 32-expert tiles is half empty) against the same rows of the
+    one-kernel gate, bit for bit, in NaN-filled outputs with a guard row."""
+    from torchturbo_amd import _lib
+
+    H, full_T = 128, 16384
+    g = torch.Generator().manual_seed(E)
+    x = torch.randn(full_T, H, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(E, H, generator=g) * H ** -0.5).to(dtype).to(DEV)
+
+    def run(T):
+        out = (torch.full((T + 1, E), float("nan"), dtype=rdt, device=DEV),
+               torch.full((T + 1, E), float("nan"), dtype=rdt, device=DEV),
+               torch.full((T + 1, E), 7, dtype=torch.uint8, device=DEV),
+               torch.full((T + 1, 4), -1, dtype=torch.int64, device=DEV))
+        _lib.call("tt_router_gate_fwd", _lib.ptr(x), _lib.ptr(w), _lib.dtype_code(dtype), T, H, E,
+                  _lib.dtype_code(rdt), 4, 1, 0, None, 0, 0, 2.5, None, *map(_lib.ptr, out),
+                  _lib.stream())
+        assert out[0][T].isnan().all() and out[1][T].isnan().all()
+        assert (out[2][T] == 7).all() and (out[3][T] == -1).all()
+        return out
+
+    full = run(full_T)
+    per = E // 32
+    sizes = {32 * (limit // per) + d for limit in (288, 576) for d in (-1, 0, 1, 33)}
+    for T in sorted(t for t in sizes | {12001, 16320} if t < 16321):
+        for got, ref in zip(run(T), full):
+            assert torch.equal(got[:T], ref[:T]), T
+
+
+def test_router_gate_long_rows_leave_the_split_earlier():
+    """Rows of 2048 and more and over 64 experts take the one-kernel gate from four fifths of
+    the CUs (13057 tokens on 256): the same bits on both sides."""
+    from torchturbo_amd import _lib
+
+    H, E = 2048, 96
+    x = torch.randn(13100, H, device=DEV).bfloat16()
+    w = (torch.randn(E, H, device=DEV) * H ** -0.5).bfloat16()
+    got = []
+    for T in (13000, 13057, 13100):
+        out = (torch.empty((T, E), device=DEV), torch.empty((T, E), device=DEV),
+               torch.empty((T, E), dtype=torch.uint8, device=DEV),
+               torch.empty((T, 8), dtype=torch.int64, device=DEV))
+        _lib.call("tt_router_gate_fwd", _lib.ptr(x), _lib.ptr(w), _lib.TT_BF16, T, H, E, _lib.TT_F32,
+                  8, 0, 0, None, 0, 0, 0.0, None, *map(_lib.ptr, out), _lib.stream())
+        got.append(out)
+    for a, b, c in zip(*got):
+        assert torch.equal(a, b[:13000]) and torch.equal(b, c[:13057])
+
+
 @pytest.mark.parametrize("T,E,k", [(1, 8, 2), (63, 64, 8), (64, 128, 8), (65, 1000, 16), (256, 33, 1),
                                    (257, 128, 8), (1000, 300, 6), (1024, 256, 16), (1536, 320, 8),
                                    (1537, 64, 4), (513, 1097, 2), (700, 2048, 3),

@@ -58,7 +58,8 @@ __global__ __launch_bounds__(GL_NT) void gate_logits_kernel(const char* __restri
               lds0 + (uint32_t)(slot * STAGE + c * CHUNK + (LD * wave + q) * 1024));
     }
   };
-  const bool busy = wave < MT * NE;  // the wave has a tile
+  // The wave has a tile (the last block's may lie past the experts).
+  const bool busy = wave < MT * NE && e0 + 32 * (wave / MT) < E;
   const int mt = wave % MT, ne = busy ? wave / MT : 0;
   uint32_t fa[4], fb[4];
 #pragma unroll
@@ -106,19 +107,24 @@ __global__ __launch_bounds__(GL_NT) void gate_logits_kernel(const char* __restri
   }
 }
 
-// One 32x32 tile per block (two chunks a stage, four stages) while that makes
-// at most this many blocks, 64x64 tiles (two stages) above. Logits and top-k,
-// one-kernel gate / 32x32 / 64x64 tiles: H 2048, E 128, 1 token 18.1 / 15.4 /
-// 17.3 us, 1000 tokens 26.0 / 17.0 / 19.2, 4096 27.4 / 21.0 / 21.7, 8192 28.4
-// / 35.5 / 27.2; H 7168, E 256, 48 tokens 74.6 / 37.2 / 44.4, 1000 77.8 / 37.8
-// / 49.0, 4096 79.8 / 68.6 / 53.4, 8192 80.5 / 125 / 66.6, 12000 150 / 225 /
-// 126. What is left is the chain of dependent MFMAs (H / 16 of them).
-constexpr int64_t GL_BLOCKS = 512;
+// Tokens x experts per block by the number of 32x32 tiles: 32x32 (two chunks a
+// stage, four stages) while they make about a block per CU, 32x64 (three
+// stages) while those do, 64x64 (two stages) above, which reads x once per 64
+// experts and w once per 64 tokens. Logits and top-k, one-kernel gate / 32x32 /
+// 32x64 / 64x64 (tiles): H 2048, E 128, 1000 tokens (128) 23.0 / 13.9 / 15.3 /
+// 16.0 us, 4000 (500) 23.9 / 23.0 / 18.3 / 20.0, 8192 (1024) 25.5 / 32.1 / 25.4
+// / 24.9; H 7168, E 256, 1000 (256) 67.7 / 32.0 / 35.2 / 42.8, 2000 (504) 67.4 /
+// 47.9 / 37.1 / 43.4, 4000 (1000) 69.5 / 80.9 / 51.1 / 53.3, 8192 (2048) 71.6 /
+// 127 / 80.6 / 59.1; H 4096, E 224, 1000 (224) 42.2 / 22.7 / 24.4 / 26.2, 8192
+// (1792) 45.3 / 104 / 72.2 / 40.0; H 4096, E 64, 8192 (512) 30.5 / 39.1 / 30.5 /
+// 31.5. What is left is the chain of dependent MFMAs (H / 16 of them).
+constexpr int64_t GL_TILES1 = 288, GL_TILES2 = 576;
 
 template <int MT, int NE, int CH, int S>
 int launch_gate_logits(const void* x, const void* w, int dtype, int64_t T, int H, int E, int ldt,
                        void* logits, hipStream_t s) {
-  const dim3 grid((unsigned)((T + 32 * MT - 1) / (32 * MT)), (unsigned)(E / (32 * NE)));
+  const dim3 grid((unsigned)((T + 32 * MT - 1) / (32 * MT)),
+                  (unsigned)((E + 32 * NE - 1) / (32 * NE)));
   if (dtype == TT_BF16)
     hipLaunchKernelGGL((gate_logits_kernel<TT_BF16, MT, NE, CH, S>), grid, dim3(GL_NT), 0, s,
                        static_cast<const char*>(x), static_cast<const char*>(w), T, H, E, ldt,
@@ -134,7 +140,8 @@ int launch_gate_logits(const void* x, const void* w, int dtype, int64_t T, int H
 
 int tt_gate_logits(const void* x, const void* w, int dtype, int64_t T, int H, int E, int ldt,
                    void* logits, hipStream_t s) {
-  if (E % 64 != 0 || (T + 31) / 32 * (E / 32) <= GL_BLOCKS)
-    return launch_gate_logits<1, 1, 2, 4>(x, w, dtype, T, H, E, ldt, logits, s);
+  const int64_t tiles = (T + 31) / 32 * (E / 32);
+  if (tiles <= GL_TILES1) return launch_gate_logits<1, 1, 2, 4>(x, w, dtype, T, H, E, ldt, logits, s);
+  if (tiles <= GL_TILES2) return launch_gate_logits<1, 2, 2, 3>(x, w, dtype, T, H, E, ldt, logits, s);
   return launch_gate_logits<2, 2, 2, 2>(x, w, dtype, T, H, E, ldt, logits, s);
 }

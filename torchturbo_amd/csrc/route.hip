@@ -1754,12 +1754,15 @@ extern "C" int tt_router_gate_fwd(const void* x, const void* weight, int in_dtyp
   const int gk = fixed_indices ? 0 : group_topk;
   const int H = (int)hidden;
   const int NE = num_experts / 32;
-  if ((num_tokens + 63) / 64 < gate_cu_count()) {
-    // 64-token blocks would leave compute units idle: the logits with the
-    // experts spread over blocks too (gate.hip), then the top-k on its own;
-    // the same bits. H 2048, E 128: 26.0 -> 17.0 us at 1000 tokens, 28.4 ->
-    // 27.2 at 8192; with 16384 tokens (256 blocks) 41.2 here, 37.8 split; H
-    // 7168, E 256: 135 here, 162 split.
+  // 64-token blocks would leave compute units idle: the logits with the
+  // experts spread over blocks too (gate.hip), then the top-k on its own; the
+  // same bits. Rows of experts re-read by many blocks cost more than a fifth of
+  // the CUs left idle, for long rows and more than two blocks across. One
+  // kernel / split: H 2048, E 128, 1000 tokens 33.6 / 13.9 us, 8192 36.3 / 24.9,
+  // 14000 37.5 / 35.9; H 7168, E 256, 8192 104 / 59.1, 14000 105 / 140, 16384 117
+  // / 140; H 4096, E 64, 14000 39.2 / 37.6; H 512, E 128, 14000 28.7 / 25.4.
+  const int64_t blocks = (num_tokens + 63) / 64, cus = gate_cu_count();
+  if (blocks < cus && !(blocks * 5 >= cus * 4 && num_experts > 64 && H >= 2048)) {
     const int rc = tt_gate_logits(x, weight, in_dtype, num_tokens, H, num_experts, logits_dtype,
                                   logits, S(stream));
     if (rc != TT_OK) return rc;
