@@ -1320,6 +1320,45 @@ def test_grouped_matmul_few_rows_exact(counts, K, N, dtype, trans_b):
         s0 += c
 
 
+# (experts, columns of the output, limit of the few-row kernel): one launch in each class of
+# its rule, by the number of 256-wide column tiles.
+THIN_LIMITS = [(100, 256, 96), (100, 512, 60), (100, 768, 96), (100, 2048, 96), (25, 8192, 40),
+               (130, 2056, 40)]
+
+
+@pytest.mark.parametrize("E,J,limit", THIN_LIMITS, ids=[f"E{c[0]}J{c[1]}" for c in THIN_LIMITS])
+def test_grouped_matmul_few_rows_rule(E, J, limit):
+    """fwd and dgrad on both sides of the few-row kernel's row limit, even and one-sided loads,
+    both weight layouts: small-integer operands (exact sums) into NaN-filled outputs."""
+    from torchturbo_amd import _lib
+
+    g = torch.Generator().manual_seed(E + J)
+    R = 72
+    for rows in (limit, limit + 1):
+        M = E * rows
+        even = torch.full((E,), rows)
+        skew = torch.full((E,), rows // 2)
+        skew[E // 3] += M - int(skew.sum())
+        skew[E // 2], skew[0] = 0, skew[0] + skew[E // 2]
+        x = torch.randint(-2, 3, (M, R), generator=g).bfloat16().to(DEV)
+        for trans_b in (0, 1):
+            for name, shape in (("tt_gmm_fwd", (E, J, R) if trans_b else (E, R, J)),
+                                ("tt_gmm_dgrad", (E, R, J) if trans_b else (E, J, R))):
+                K, N = (R, J) if name == "tt_gmm_fwd" else (J, R)
+                w = torch.randint(-2, 3, shape, generator=g).bfloat16().to(DEV)
+                wide = w if shape[1] == R else w.transpose(1, 2)  # [E, R, J]
+                for counts in (even, skew):
+                    assert int(counts.sum()) == M
+                    y = torch.full((M + 1, J), float("nan"), dtype=torch.bfloat16, device=DEV)
+                    cnt = counts.to(torch.int64).to(DEV)
+                    _lib.call(name, _lib.ptr(x), _lib.ptr(w), _lib.TT_BF16, M, K, N, E, trans_b,
+                              _lib.ptr(cnt), _lib.ptr(y), _lib.stream())
+                    assert y[M].isnan().all()
+                    ref = torch.cat([a.float() @ b.float().contiguous()
+                                     for a, b in zip(x.split(counts.tolist()), wide)])
+                    assert torch.equal(y[:M], ref.bfloat16()), (name, rows, trans_b)
+
+
 # FP8 launches of at most 40 rows per expert on average: 32-row tiles up to 20 rows, 64-row
 # tiles above; reductions with partial scale blocks and tails, both scale dtypes.
 FEW_ROWS_FP8 = [

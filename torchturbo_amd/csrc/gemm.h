@@ -267,7 +267,7 @@ __device__ __forceinline__ bool row_tile(const int64_t* __restrict__ counts, int
 }  // namespace
 
 // fwd / dgrad for experts of few rows (gmm_thin.hip): operands as
-// tt_gmm_fwd / tt_gmm_dgrad, already checked; see thin_rows in gmm.hip. With
+// tt_gmm_fwd / tt_gmm_dgrad, already checked; see thin_row_limit in gmm.hip. With
 // arow, activation row r is row arow[r] of p0 (src_rows rows, under 2 GiB).
 int tt_gmm_thin(int mode, bool tb, int dtype, const void* p0, const void* p1, void* out,
                 int64_t M, int64_t K, int64_t N, int E, const int64_t* counts, hipStream_t s,

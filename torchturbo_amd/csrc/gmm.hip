@@ -46,7 +46,7 @@
 //   weight-streaming pipeline of their own (two weight k-tiles in flight
 //   while a third is multiplied), and an expert of at most 64 rows takes its
 //   tiles two per schedule slot. Launches of few rows per expert on average
-//   run on gmm_thin.hip (thin_rows) and gmm_wgrad_thin.hip (wgrad_thin) instead.
+//   run on gmm_thin.hip (thin_row_limit) and gmm_wgrad_thin.hip (wgrad_thin) instead.
 // * gmm_q8_kernel (fwd/dgrad with e4m3 weights and 128x128 block scales,
 //   launches of more than a few rows per expert (thin8_rows; the others run on
 //   gmm_thin.hip) whose reduction is longer than one 64-deep k-tile):
@@ -2613,20 +2613,37 @@ int launch_p64_k(const void* p0, const void* p1, void* out, int64_t M, int64_t K
   return tt_check_launch("gmm");
 }
 
-// fwd / dgrad with at most this many rows per expert on average run on the
-// kernel of gmm_thin.hip (its loads run up to a k-tile past the reduction end,
-// in 32-bit offsets). Measured, persistent / thin: Qwen3-30B-A3B's fc1 fwd,
-// fc2 fwd, fc1 dgrad, fc2 dgrad at 62 rows per expert 188 + 97 + 181 + 135 /
-// 164 + 90 + 171 + 107 us, at 80 179 + 101 + 193 + 129 / 165 + 94 + 177 + 108,
-// at 96 176 + 97 + 184 + 127 / 168 + 96 + 181 + 110, at 128 188 + 112 + 197 +
-// 140 / 218 + 118 + 224 + 129; 64 experts of 1024 x 1408 at 94 rows 60 + 29 +
-// 54 + 37 / 50 + 24 + 39 + 26 us, at 144 66 + 31 + 52 + 35 / 63 + 35 + 60 + 41.
-constexpr int64_t THIN_ROWS = 96;
-bool thin_rows(int64_t M, int E) { return M <= (int64_t)E * THIN_ROWS; }
-// Whether fwd / dgrad (reduction R) take it, for a problem within the limits
-// of launch_mfma.
-bool thin_takes(int64_t M, int64_t K, int64_t N, int64_t R, int E) {
-  return thin_rows(M, E) && (R + 2 * P_BK) * (K > N ? K : N) * 2 < (int64_t)DM_OOB;
+// fwd / dgrad (J columns) with at most this many rows per expert on average run
+// on the kernel of gmm_thin.hip (its loads run up to a k-tile past the reduction
+// end, in 32-bit offsets). The line depends on how many 256-wide column tiles
+// the launch has: up to 192 of them leave CUs of the persistent kernel idle,
+// about 256 give each CU one, more need a second round; above 1024, and for few
+// experts over many columns, the persistent kernel's rounds are full. Loads even
+// and skewed as a router with a Zipf(0.8) / Zipf(1.1) prior makes them,
+// persistent / thin in us: 8 experts of 512 x 1024 fwd (32 tiles) at 80 rows 12 +
+// 16 + 17 / 8 + 9 + 9; 16 of 1536 x 4096 fwd (256) at 48 rows 59 + 48 + 49 / 35 +
+// 45 + 45, at 66 43 + 51 + 51 / 35 + 57 + 55; 128 of 2048 x 1536 fwd (768) at 32
+// rows 169 + 152 + 138 / 147 + 145 + 122, at 48 173 + 152 + 133 / 157 + 161 +
+// 133, at 66 192 + 193 + 139 / 162 + 170 + 156, at 96 173 + 191 + 180 / 165 + 194
+// + 182, at 128 (even) 188 / 218; its 768 x 2048 fwd (1024) at 66 106 + 91 + 85 /
+// 89 + 98 + 84, dgrad (384) 135 / 108 (even, 62); 128 of 512 x 4096 fwd (2048) at
+// 32 109 + 111 + 88 / 107 + 103 + 87, at 80 134 + 133 + 119 / 134 + 145 + 131; 32
+// of 2048 x 5632 fwd (704, 22 per expert) at 48 153 + 149 + 143 / 140 + 146 +
+// 142, at 66 180 + 144 + 142 / 154 + 170 + 162. Over 26 layers, 14 row counts and
+// these loads the launches take 0.74 of the persistent kernel's time on average;
+// 2.5 % of them are slower by more than 5 % (at most 1.26).
+int64_t thin_row_limit(int64_t E, int64_t J) {
+  const int64_t tiles = E * ((J + DM_BN - 1) / DM_BN);
+  if (tiles <= 192) return 96;
+  if (tiles <= 256) return 60;
+  if (tiles <= 512 || (tiles <= 1024 && J <= 4096)) return 96;
+  return 40;
+}
+// Whether fwd / dgrad (reduction R, J columns) take it, for a problem within the
+// limits of launch_mfma.
+bool thin_takes(int64_t M, int64_t K, int64_t N, int64_t R, int64_t J, int E) {
+  return M <= E * thin_row_limit(E, J) &&
+         (R + 2 * P_BK) * (K > N ? K : N) * 2 < (int64_t)DM_OOB;
 }
 
 template <int MODE, bool TB, int ET>
@@ -2648,7 +2665,7 @@ int launch_mfma(const void* p0, const void* p1, void* out, int64_t M, int64_t K,
   const int64_t R = MODE == MODE_FWD ? K : N;  // reduction length of fwd / dgrad
   const bool p64_lds = p64_lds_bytes(E) <= 160 * 1024;
   if constexpr (MODE != MODE_WGRAD) {
-    if (thin_takes(M, K, N, R, E))
+    if (thin_takes(M, K, N, R, MODE == MODE_FWD ? N : K, E))
       return tt_gmm_thin(MODE, TB, ET, p0, p1, out, M, K, N, E, counts, s);
     // The persistent kernel needs two k-tiles per output tile, its LDS
     // (stages, epilogue staging, schedule) and 32-bit offsets for loads that
@@ -2999,7 +3016,7 @@ int tt_gmm_rows_fwd(const void* x, int64_t src_rows, const int32_t* arow, const 
                       counts, s, arow, src_rows);
   } else {
     const int64_t ld = K > N ? K : N;
-    if (!thin_takes(M, K, N, K, E) || (M + DM_BM) * ld * 2 >= (int64_t)DM_OOB ||
+    if (!thin_takes(M, K, N, K, N, E) || (M + DM_BM) * ld * 2 >= (int64_t)DM_OOB ||
         K * N * 2 >= (int64_t)DM_OOB)
       return 0;
     rc = tt_gmm_thin(MODE_FWD, false, dtype, x, w, y, M, K, N, E, counts, s, arow, src_rows);

@@ -20,12 +20,14 @@ constexpr int T_BN = 128, T_BK = 64, T_NT = 256;
 // them faster: 119 experts of 2048 x 1536 (751 MB) 120 us, 6.3 TB/s, against
 // 135 us with the default policy; 8 of them (50 MB, cached) 20 against 15 us.
 constexpr int64_t T_CACHED = 128 << 20;
-// Rows per expert on average up to which tiles have 64 rows: Qwen3-30B-A3B's
-// four products with 64- / 128-row tiles at 32 rows per expert 148 + 78 + 143
-// + 84 / 148 + 80 + 152 + 102 us, at 48 166 + 87 + 161 + 96 / 159 + 87 + 163
-// + 106, at 62 177 + 90 + 179 + 95 / 164 + 90 + 171 + 107; 16 experts of
-// 4096 x 3072 at 50 rows 85 + 48 + 87 + 45 / 80 + 37 + 71 + 67 us.
-constexpr int64_t T_ROWS64 = 40;
+// Rows per expert on average up to which tiles have 64 rows. 64- / 128-row
+// tiles, even loads and ones skewed by a Zipf(0.8) / Zipf(1.1) prior: 128 experts
+// of 2048 x 1536 fwd at 48 rows 157 + 161 + 133 / 158 + 163 + 126 us, at 60 155 +
+// 168 + 150 / 161 + 164 + 150, at 66 183 + 168 + 159 / 162 + 170 + 156, dgrad at
+// 48 155 + 155 + 132 / 161 + 165 + 127, at 66 190 + 168 + 157 / 172 + 185 + 158;
+// 16 of 1536 x 4096 fwd at 48 35 + 45 + 45 / 34 + 57 + 57; 64 of 1024 x 1408 fwd
+// at 48 34 + 37 + 40 / 41 + 42 + 40, at 66 40 + 42 + 42 / 43 + 43 + 42.
+constexpr int64_t T_ROWS64 = 60;
 constexpr int T_B = T_BN * T_BK * 2;  // weight tile (16 KiB)
 
 // Byte offset of row r of a tile (first packed row `at`, `rows` valid): from
