@@ -278,7 +278,7 @@ int tt_gated_act_bwd(const void* x, int dtype, int64_t rows, int64_t ffn, int ac
  * successive launches and written on the launch stream before the GEMM kernel
  * runs: the persistent kernel's work queue (tt_gmm_wgrad_persistent), or the
  * one-tile-per-block kernel's expert ranking. Launches of few rows per expert
- * (160 on average, 96 for experts of more than 192 output tiles of 256x256)
+ * (144 on average, 96 for experts of more than 192 output tiles of 256x256)
  * keep none. At most 64 weight-gradient
  * launches may be in flight at once across all streams of a device; launches
  * on one stream never overlap, so a single stream has no limit. A launch
@@ -339,7 +339,7 @@ int tt_gmm_gather_supported(int32_t op, int dtype, int64_t src_rows, int64_t m, 
 /* Whether tt_gmm_wgrad runs this shape (bf16 / f16) on its persistent kernel
  * (1) rather than a kernel of one tile per block (0), without launching: short
  * reductions (m <= 512 * num_experts) or at least 512 output tiles of 256x256
- * per expert, unless there are few rows per expert (at most 160 on average, 96
+ * per expert, unless there are few rows per expert (at most 144 on average, 96
  * for more than 192 tiles per expert, 512 for at most 256 tiles in all), which
  * take the small-tile kernel. No counterpart in the reference: it reports the launcher's
  * kernel choice, so that tests and tools can tell which kernel a shape

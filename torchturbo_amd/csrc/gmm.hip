@@ -2554,12 +2554,13 @@ size_t p64_lds_bytes(int E) { return p64_schedule_bytes(E) + 2 * P_STAGE + 4 * P
 // rows 199 + 114 / 162 + 84; 64 of 1024 x 1408 and 704 x 1024 at 144 rows 65 +
 // 47 / 46 + 26; 64 of 7168 x 4096 and 2048 x 7168 (448 and 224 tiles) at 64
 // rows 781 + 376 / 656 + 307, 128 rows 853 + 442 / 852 + 430; 8 of 512 x 1024
-// and 512 x 512 at 500 rows 24 + 35 / 15 + 11. Zipf loads (exponent 0.8, the
-// longest expert about 15 times the mean): the first layer at 62 rows 175 + 96
-// / 152 + 79, 128 rows 203 + 112 / 207 + 106, 256 rows 270 + 154 / 300 + 163
-// (even loads 291 + 161 / 260 + 118): above the line the long experts are
-// bound by their products, which the larger tiles do better.
-constexpr int64_t W_THIN_ROWS = 160, W_WIDE_ROWS = 96;
+// and 512 x 512 at 500 rows 24 + 35 / 15 + 11. Loads skewed by a Zipf(0.8) /
+// Zipf(1.1) prior on the router: 128 of 2048 x 1536 at 64 rows 181 + 186 / 164 +
+// 167, at 144 233 + 234 / 211 + 221, of 768 x 2048 at 128 rows 117 + 118 / 134 +
+// 142, at 144 120 + 123 / 107 + 107; 256 of 1024 x 1024 at 144 rows 179 + 173 /
+// 176 + 188, at 160 184 + 183 / 248 + 254 (even 180 / 130): above the line the
+// long experts are bound by their products, which the larger tiles do better.
+constexpr int64_t W_THIN_ROWS = 144, W_WIDE_ROWS = 96;
 constexpr int W_WIDE_TILES = 192;
 bool wgrad_thin(int64_t M, int64_t E, int ti, int tj) {
   const int64_t rows = (int64_t)ti * tj > W_WIDE_TILES ? W_WIDE_ROWS
@@ -2796,7 +2797,10 @@ int launch_q8_k(const void* p0, const uint8_t* qw, const void* scale, int sdt, v
 // gmm_thin8_kernel (gmm_thin.hip). DeepSeek-V3's fc1 + fc2 (256 experts),
 // gmm_q8_kernel / thin: at 32 rows per expert forward 1718 + 879 / 1418 + 802
 // us, data gradient 1586 + 793 / 1575 + 718; at 64 rows 1806 + 934 / 2001 +
-// 1081 and 1693 + 863 / 2100 + 1047.
+// 1081 and 1693 + 863 / 2100 + 1047. Even loads and ones skewed by a Zipf(0.8) /
+// Zipf(1.1) prior, fc1 forward at 24 rows 1745 + 1476 + 991 / 1368 + 1314 + 891, at
+// 40 1782 + 1864 + 1277 / 1584 + 1724 + 1350, data gradient at 40 1695 + 1675 +
+// 1211 / 1647 + 1735 + 1361; fc2 forward at 40 921 + 939 + 675 / 863 + 936 + 746.
 constexpr int64_t THIN8_ROWS = 40;
 bool thin8_rows(int64_t M, int E) { return M <= (int64_t)E * THIN8_ROWS; }
 bool thin8_takes(int64_t M, int64_t K, int64_t N, int64_t R, int E) {

@@ -256,6 +256,10 @@ static_assert(T8_SMAX == 128, "two registers of one scale per lane");
 // KiB of LDS) rather than 64 (two, 64 KiB): at 16 rows per expert fc1 + fc2
 // forward 1213 + 689 / 1276 + 744 us, data gradient 1353 + 630 / 1414 + 645; at
 // 32 rows 1614 + 887 / 1418 + 802 and 1732 + 816 / 1575 + 718.
+// Even loads and ones skewed by a Zipf(0.8) / Zipf(1.1) prior, 32- / 64-row
+// tiles: fc1 forward at 16 rows 1244 + 1136 + 807 / 1315 + 1110 + 715, at 20 1271 +
+// 1239 + 958 / 1335 + 1202 + 849, at 24 1345 + 1398 + 1033 / 1368 + 1314 + 891,
+// data gradient at 20 1402 + 1310 + 978 / 1449 + 1214 + 866.
 constexpr int64_t T8_ROWS32 = 20;
 
 template <int MODE, bool KMASK, int BM, int S, int OCC>
