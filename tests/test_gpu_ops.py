@@ -173,7 +173,8 @@ GATE_CASES = [
     (129, 192, 64, 4, "softmax", False, None, None, None, False, torch.bfloat16, torch.bfloat16),
     (200, 256, 96, 4, "sigmoid", False, None, None, None, False, torch.float16, torch.float16),
     (0, 256, 128, 8, "softmax", False, None, None, None, False, torch.bfloat16, torch.float32),
-    # 64-token blocks (the grid covers the device); the cases above use 32-token blocks
+    # 64-token blocks of the one-kernel gate (the grid covers the device); the cases above spread
+    # the experts over blocks
     (16448, 128, 128, 8, "softmax", False, None, None, None, False, torch.bfloat16, torch.float32),
 ]
 
@@ -255,6 +256,70 @@ def test_router_gate_topk_hash_routing(hip_ops):
                                                     input_ids=input_ids, **kw)
     assert torch.equal(i.cpu(), ir) and torch.equal(m.cpu(), mr)
     assert rel_errors(p.cpu(), pr)[0] <= 2e-6
+
+
+# the one-kernel gate: T over 256 64-token blocks, ragged
+ONE_KERNEL_GATE = [
+    (16385, 64, 256, 8, "sigmoid", False, 8, 4, 2.5, True, torch.bfloat16, torch.float32),
+    (16401, 64, 160, 6, "softmax", True, None, None, 1.5, True, torch.float16, torch.float32),
+    (16447, 128, 64, 4, "sqrtsoftplus", False, None, None, None, False, torch.bfloat16, torch.float32),
+    (16390, 64, 192, 8, "sigmoid", False, 6, 2, None, True, torch.bfloat16, torch.float32),
+    (16410, 64, 224, 8, "sigmoid", False, None, None, 2.5, True, torch.float16, torch.float32),
+    (16420, 192, 96, 4, "softmax", False, None, None, None, False, torch.float16, torch.float32),
+    (16430, 64, 32, 2, "softmax", False, None, None, None, False, torch.bfloat16, torch.bfloat16),
+    (16399, 128, 64, 4, "hash", True, None, None, 1.7, False, torch.bfloat16, torch.float32),
+]
+
+
+@pytest.mark.parametrize("case", ONE_KERNEL_GATE, ids=lambda c: f"T{c[0]}E{c[2]}k{c[3]}{c[4]}")
+def test_router_gate_one_kernel_batches(hip_ops, case):
+    """Batches that take the one-kernel gate: logits against the exact linear, and the oracle's
+    top-k of the kernel's own logits. Scores of either side lie within 2^-21 of the exact ones
+    (exp, log and the divisions are good to a few units of 2^-24, a group's value sums four), so
+    ids and map must agree where no choice is closer than 2^-18; almost every token is such."""
+    T, H, E, k, score, pre, groups, gtopk, scale, use_bias, idt, rdt = case
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).to(idt)
+    w = (torch.randn(E, H, generator=g) * H ** -0.5).to(idt)
+    bias = (torch.randn(E, generator=g) * 0.05) if use_bias else None
+    kw = dict(use_pre_softmax=pre, num_groups=groups, group_topk=gtopk, scaling_factor=scale,
+              score_function="sigmoid" if score == "hash" else score)
+    hashed = [dict(), dict()]
+    if score == "hash":
+        table = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(10)])
+        tokens = torch.randint(0, 10, (T,), generator=g)
+        hashed = [dict(use_hash_routing=True, hash_table=t.to(d), input_ids=i.to(d))
+                  for t, i, d in ((table, tokens, DEV), (table, tokens, "cpu"))]
+    probs, rmap, ids, logits = hip_ops.router_gate_topk(
+        x.to(DEV), w.to(DEV), rdt, k, expert_bias=None if bias is None else bias.to(DEV), **kw,
+        **hashed[0])
+    lg, exact = logits.cpu(), x.double() @ w.double().T
+    bound = 1e-5 * float(exact.abs().max()) if rdt == torch.float32 else exact.abs() * 2 ** -8 + 1e-6
+    assert torch.all((lg.double() - exact).abs() <= bound)
+    pr, mr, ir = o_route.topk_softmax_with_capacity(lg, k, expert_bias=bias, **kw, **hashed[1])
+    s = lg.double()
+    if score == "sigmoid":
+        s = s.sigmoid()
+    elif score == "sqrtsoftplus":
+        s = F.softplus(s).sqrt()
+    elif pre:
+        s = s.softmax(1)
+    if bias is not None:
+        s = s + bias.double()
+    rows = torch.ones(T, dtype=torch.bool)
+    if score != "hash":
+        if groups:
+            value = s.view(T, groups, -1).topk(k // gtopk, dim=-1).values.sum(-1)
+            best = value.topk(gtopk + 1, dim=1)
+            rows &= best.values[:, -2] - best.values[:, -1] > 2.0 ** -18
+            keep = torch.zeros_like(value).scatter_(1, best.indices[:, :gtopk], 1.0).bool()
+            s = s.view(T, groups, -1).masked_fill(~keep.unsqueeze(-1), -10.0).view(T, E)
+        best = s.topk(k + 1, dim=1).values
+        rows &= (best[:, :-1] - best[:, 1:]).min(dim=1).values > (2.0 ** -18 if rdt == torch.float32 else 0.0)
+    assert float(rows.double().mean()) > (0.98 if rdt == torch.float32 else 0.5)
+    assert torch.equal(ids.cpu()[rows], ir[rows]) and torch.equal(rmap.cpu()[rows], mr[rows])
+    tol = 2e-6 if rdt == torch.float32 else 8e-3
+    assert rel_errors(probs.cpu()[rows], pr[rows])[0] <= tol
 
 
 @pytest.mark.parametrize("H,E", [(64, 32), (192, 96), (320, 256)])
@@ -972,8 +1037,8 @@ def test_grouped_matmul_integer_exact(hip_ops):
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_grouped_matmul_wgrad_writes_every_tile(dtype, E, rows, trans_b):
     """tt_gmm_wgrad into a NaN-filled output: every expert's whole gradient is written
-    (empty experts get zeros), whatever the kernel (fp32, persistent short-reduction,
-    one tile per block on XCD pairs) and whether E is a multiple of 8."""
+    (empty experts get zeros), whatever the kernel (fp32, small tiles of few rows, one
+    tile per block on XCD pairs) and whether E is a multiple of 8."""
     from torchturbo_amd import _lib
 
     torch.backends.cuda.matmul.allow_tf32 = False
@@ -994,6 +1059,35 @@ def test_grouped_matmul_wgrad_writes_every_tile(dtype, E, rows, trans_b):
         ref = xs[e].t() @ ds[e]  # [K, N]; integer sums, exact in fp32
         ref = (ref.t() if trans_b else ref).to(dtype)
         assert torch.equal(dw[e], ref), (e, int(counts[e]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("E,K,N,rows", [(24, 1032, 776, 200), (13, 1544, 1288, 350), (40, 520, 904, 150)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_grouped_matmul_wgrad_persistent_writes_every_tile(dtype, E, K, N, rows, trans_b):
+    """The persistent short-reduction kernel at widths that 256 does not divide, E a multiple
+    of 8 or not, with empty and short experts: exact small-integer sums in a NaN-filled
+    output, operands with NaNs behind their ends."""
+    from torchturbo_amd import _lib
+
+    torch.backends.cuda.matmul.allow_tf32 = False
+    g = torch.Generator().manual_seed(E + rows)
+    counts = torch.randint(rows // 2, 2 * rows, (E,), generator=g)
+    counts[:4] = torch.tensor([0, 1, 63, 65])
+    counts[-1] = 0
+    M = int(counts.sum())
+    assert _lib.load().tt_gmm_wgrad_persistent(_lib.dtype_code(dtype), M, K, N, E, int(trans_b)) == 1
+    full = [torch.full((M + 128, w), float("nan"), dtype=dtype, device=DEV) for w in (K, N)]
+    x, dy = (f[:M].copy_(torch.randint(-2, 3, (M, f.shape[1]), generator=g)) for f in full)
+    dw = torch.full((E + 1, N, K) if trans_b else (E + 1, K, N), float("nan"), dtype=dtype, device=DEV)
+    cnt = counts.to(DEV)
+    _lib.call("tt_gmm_wgrad", _lib.ptr(x), _lib.ptr(dy), _lib.dtype_code(dtype), M, K, N, E,
+              int(trans_b), _lib.ptr(cnt), _lib.ptr(dw), _lib.stream())
+    torch.cuda.synchronize()
+    assert dw[E].isnan().all()
+    for e, (xe, de) in enumerate(zip(x.float().split(counts.tolist()), dy.float().split(counts.tolist()))):
+        ref = xe.t() @ de
+        assert torch.equal(dw[e], (ref.t() if trans_b else ref).to(dtype)), (e, int(counts[e]))
 
 
 @pytest.mark.parametrize("T,H,E", [(1, 64, 32), (31, 192, 64), (129, 320, 96), (700, 2048, 256),
