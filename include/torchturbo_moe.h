@@ -84,7 +84,8 @@ int tt_router_gate_fwd(const void* x, const void* weight, int in_dtype, int64_t 
  * fp32 logits (models/modules/moe/router.py:44-58): with g = grad + grad2
  * (fp32 [T, E], grad2 may be NULL), dx [T, hidden] = bf16(g weight) and dw
  * [E, hidden] = bf16(g^T x), each skipped when NULL. fp32 products and sums: g
- * enters as three bf16 parts that add up to it exactly. Sizes as
+ * enters as three bf16 parts that add up to it (exactly from 2^-110 up, to
+ * 2^-133 below). Sizes as
  * tt_router_gate_fwd with operands under 4 GiB; everything 16-byte aligned.
  * tt_router_gate_bwd_workspace: bytes of scratch, or 0 when the size is not
  * taken. */

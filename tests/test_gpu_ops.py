@@ -1141,6 +1141,26 @@ def test_router_gate_bwd_matches_fp64(T, H, E):
         assert torch.equal(got.isinf(), ref.to(torch.bfloat16).isinf())
 
 
+@pytest.mark.parametrize("exponent", [-90, -108, -112, -118, -124, 100])
+def test_router_gate_bwd_at_the_ends_of_fp32(exponent):
+    """The three bf16 parts of a gradient hold all of it from 2^-110 up; below, the last loses
+    what lies under bf16's smallest subnormal, less than 2^-133 of each gradient. Beside that,
+    fp32 sums and one rounding to bf16 (whose own spacing ends at 2^-133)."""
+    from torchturbo_amd.providers.hip._functions import router_gate_bwd
+
+    T, H, E = 257, 192, 64
+    gen = torch.Generator().manual_seed(7)
+    g = torch.randn(T, E, generator=gen).clamp(-3.9, 3.9) * 2.0 ** exponent
+    x, w = (torch.randn(n, H, generator=gen).to(torch.bfloat16) for n in (T, E))
+    dx, dw = router_gate_bwd(g.to(DEV), None, x.to(DEV), w.to(DEV), True, True)
+    for name, got, a, b in (("dx", dx, g.double(), w), ("dw", dw, g.double().t(), x)):
+        ref, mag = a @ b.double(), a.abs() @ b.double().abs()
+        lost = 2.0 ** -133 * b.double().abs().sum(0) * (exponent < -106)
+        bound = ref.abs() * 2.0 ** -8 + mag * a.shape[1] * 2.0 ** -23 + lost + 2.0 ** -134
+        worst = ((got.cpu().double() - ref).abs() / bound).max()
+        assert worst <= 1.0, (name, float(worst))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("E,K,N,rows", [

@@ -3,12 +3,13 @@
 //
 // As fp32 products these are bound by the fp32 matrix rate (T 4096, H 7168, E
 // 256: 15 GFLOP each, 139 + 136 us in a library GEMM at 110 TFLOP/s, and 62 us
-// more for fp32 copies of x and w and the casts of the results). Every fp32
-// value is the exact sum of three bf16 values of eight significant bits each,
-// so g is split into three bf16 planes and both products run on bf16 matrix
-// instructions with fp32 accumulation: the same products, exact, in three
-// times the operations at sixteen times the rate, and no larger error against
-// float64. Both gradients, composition / here: T 4096, H 7168, E 256 344 / 110
+// more for fp32 copies of x and w and the casts of the results). An fp32 value
+// of 2^-110 or more is the exact sum of three bf16 values of eight significant
+// bits each (below, the third ends at bf16's smallest subnormal and up to 2^-133
+// is lost, the spacing of the smallest bf16 results), so g is split into three
+// bf16 planes and both products run on bf16 matrix instructions with fp32
+// accumulation: the same products, exact, in three times the operations at
+// sixteen times the rate, and no larger error against float64. Both gradients, composition / here: T 4096, H 7168, E 256 344 / 110
 // us (split 6, dx 50, dw 48, the sum of its parts 5), 1024, 7168, 64 64 /
 // 31, 16384, 2048, 128 277 / 85, 128, 1024, 64 24 / 17.
 #include "gemm.h"
@@ -23,9 +24,9 @@ constexpr int GB_STAGE = 3 * GB_PLANE + GB_N * GB_K * 2;  // 32 KiB, two stages
 constexpr int64_t GB_BLOCKS = 512;
 constexpr int GB_RUN = 64, GB_GROUP = 8;  // tile order, as in gmm_wgrad_thin.hip
 
-// v as three bf16 values whose sum it is: the upper eight significant bits by
-// truncation, then those of the exact remainders. Infinities and NaNs stay in
-// the first.
+// v as three bf16 values whose sum it is (from 2^-110 up): the upper eight
+// significant bits by truncation, then those of the exact remainders. Infinities
+// and NaNs stay in the first.
 __device__ __forceinline__ void split3(float v, uint16_t (&p)[3]) {
   const uint32_t b = __builtin_bit_cast(uint32_t, v);
   const bool finite = (b & 0x7f800000u) != 0x7f800000u;
