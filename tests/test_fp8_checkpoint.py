@@ -7,6 +7,7 @@ restated in ``oracle/fp8.py``), assemble ``weight1 = cat(gate, up).T`` /
 from __future__ import annotations
 
 import json
+import math
 
 import pytest
 import torch
@@ -116,3 +117,49 @@ def test_fp8_loader_rejects_bad_tensors():
     bad = {key: v for key, v in tensors.items() if not key.startswith(f"{PREFIX}.0.down_proj")}
     with pytest.raises(KeyError, match="down_proj"):
         load_fp8_experts(mod, bad, PREFIX)
+
+
+def _round_bits(v, bits):
+    """The nearest binary fraction of ``bits`` significant bits to a positive Fraction (ties to even)."""
+    from fractions import Fraction
+
+    num, den = v.numerator, v.denominator
+    e = bits - num.bit_length() + den.bit_length()
+    while True:  # at most twice: the lengths give the exponent up to one
+        n, rest = divmod(num << e, den) if e >= 0 else divmod(num, den << -e)
+        if n < 2 ** bits:
+            break
+        e -= 1
+    if n < 2 ** (bits - 1):
+        e += 1
+        n, rest = divmod(num << e, den) if e >= 0 else divmod(num, den << -e)
+    unit = den if e >= 0 else den << -e
+    n += 2 * rest > unit or (2 * rest == unit and n & 1)
+    return Fraction(n << -e) if e < 0 else Fraction(n, 1 << e)
+
+
+@pytest.mark.parametrize("scale_bits", [24, 8], ids=["f32", "bf16"])
+def test_quantiser_quotient_is_correctly_rounded(scale_bits):
+    """The block quantiser forms w / s as t + r y, with y = 1 / s, t = w y and r = w - t s each
+    rounded to fp32. Scales are a bf16 amax times fp32(1 / 448), so their significands and the
+    weights' are 128 each: the result is the correctly rounded quotient for every pair of them
+    (powers of two change nothing while no step under- or overflows), t being up to 1.5 units
+    in the last place away."""
+    from fractions import Fraction
+
+    inv448 = _round_bits(Fraction(1, 448), 24)
+    farthest = Fraction(0)
+    for a in range(128, 256):
+        s = _round_bits(_round_bits(Fraction(a) * inv448, 24), scale_bits)
+        y = _round_bits(_round_bits(1 / s, 53), 24)  # through fp64, as the kernel forms it
+        for n in range(128, 256):
+            w = Fraction(n)
+            t = _round_bits(w * y, 24)
+            r = w - t * s
+            if r:
+                r = _round_bits(abs(r), 24) * (1 if r > 0 else -1)
+            q = w / s
+            assert _round_bits(t + r * y, 24) == _round_bits(q, 24), (a, n)
+            ulp = Fraction(2) ** (math.frexp(q)[1] - 24)
+            farthest = max(farthest, abs(t - q) / ulp)
+    assert farthest < Fraction(3, 2), float(farthest)

@@ -32,9 +32,11 @@ __device__ __forceinline__ float clamp448(float v) {
 //
 // The quotient is the correctly rounded fp32 w / s without a division per
 // element: y = 1 / s is formed once per block (rounded from fp64), then with
-// t = w y and the exact remainder r = w - t s, t + r y rounds to w / s
-// (Markstein's correction: t is within an ulp of the quotient and y is the
-// rounded reciprocal). That holds while nothing under- or overflows: blocks
+// t = w y (within 1.5 ulp of the quotient) and the remainder r = w - t s, t + r y
+// is Markstein's correction. It rounds to w / s for every pair of a bf16 weight's
+// 128 significands and a scale's 128 (those of amax / 448 in either scale dtype),
+// enumerated in exact arithmetic in tests/test_fp8_checkpoint.py; powers of two
+// change nothing while nothing under- or overflows: blocks
 // whose scale lies outside [2^-60, 2^60] or whose amax is not finite divide.
 template <class ST>
 __global__ __launch_bounds__(Q_THREADS) void fp8_quantize_kernel(
