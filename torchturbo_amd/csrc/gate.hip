@@ -141,7 +141,9 @@ int launch_gate_logits(const void* x, const void* w, int dtype, int64_t T, int H
 int tt_gate_logits(const void* x, const void* w, int dtype, int64_t T, int H, int E, int ldt,
                    void* logits, hipStream_t s) {
   const int64_t tiles = (T + 31) / 32 * (E / 32);
-  if (tiles <= GL_TILES1) return launch_gate_logits<1, 1, 2, 4>(x, w, dtype, T, H, E, ldt, logits, s);
-  if (tiles <= GL_TILES2) return launch_gate_logits<1, 2, 2, 3>(x, w, dtype, T, H, E, ldt, logits, s);
+  if (tiles <= GL_TILES1)
+    return launch_gate_logits<1, 1, 2, 4>(x, w, dtype, T, H, E, ldt, logits, s);
+  if (tiles <= GL_TILES2)
+    return launch_gate_logits<1, 2, 2, 3>(x, w, dtype, T, H, E, ldt, logits, s);
   return launch_gate_logits<2, 2, 2, 2>(x, w, dtype, T, H, E, ldt, logits, s);
 }

@@ -78,11 +78,6 @@ __device__ __forceinline__ i32x4 make_rsrc(const void* base, int64_t bytes) {
   return r;
 }
 
-// One 16-byte buffer load per lane straight into LDS at lds_addr + 16 * lane
-// (lds_addr is wave-uniform and goes to M0). Inline assembly, so that the
-// compiler does not drain outstanding loads before every LDS read:
-// completion of a stage is awaited explicitly (TT_WAIT_VMCNT) before the
-// barrier that publishes it. Nothing else in these kernels uses M0.
 // The resource moved `adv` bytes along (scalar arithmetic): an offset from
 // the new base is in range exactly when the same offset plus adv was before,
 // and nothing is once adv passes the end.
@@ -100,6 +95,11 @@ __device__ __forceinline__ i32x4 advance_rsrc(i32x4 r, uint32_t adv) {
   return o;
 }
 
+// One 16-byte buffer load per lane straight into LDS at lds_addr + 16 * lane
+// (lds_addr is wave-uniform and goes to M0). Inline assembly, so that the
+// compiler does not drain outstanding loads before every LDS read:
+// completion of a stage is awaited explicitly (TT_WAIT_VMCNT) before the
+// barrier that publishes it. Nothing else in these kernels uses M0.
 __device__ __forceinline__ void dma16(uint32_t voff, i32x4 rsrc, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                :

@@ -2680,9 +2680,10 @@ int launch_mfma(const void* p0, const void* p1, void* out, int64_t M, int64_t K,
     }
   } else {
     // The small-tile kernel (see wgrad_thin) or the persistent kernel for short
-    // reductions, the latter also for large tile grids (see wgrad_persistent), the four-stage one-tile-per-block kernel otherwise.
-    // wgrad reduces over each expert's rows (at most M; the loads run up to
-    // two k-tiles past an expert's end).
+    // reductions, the latter also for large tile grids (see wgrad_persistent),
+    // the four-stage one-tile-per-block kernel otherwise. wgrad reduces over
+    // each expert's rows (at most M; the loads run up to two k-tiles past an
+    // expert's end).
     if (wgrad_thin(M, E, ti, tj))
       return tt_gmm_wgrad_thin(TB, ET, p0, p1, out, M, K, N, E, counts, s);
     if (wgrad_persistent(M, K, N, E, ti, tj))

@@ -280,7 +280,10 @@ __global__ __launch_bounds__(LR_NT, RT == 2 && WT ? 3 : 1) void lora_up_kernel(
     const int m = 16 * mi + l16;
     const float* p = h + (row0 + (m < rows ? m : rows - 1)) * r;
 #pragma unroll
-    for (int q = 0; q < 4 * RT; ++q) hv[mi][q] = p[chain16(4 * q + g) < r ? chain16(4 * q + g) : 0];
+    for (int q = 0; q < 4 * RT; ++q) {
+      const int j = chain16(4 * q + g);
+      hv[mi][q] = p[j < r ? j : 0];
+    }
   }
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi)

@@ -1230,42 +1230,43 @@ __device__ __forceinline__ gf32x16 rg_mma<TT_F16>(const uint4& a, const uint4& b
                                                  __builtin_bit_cast(gf16x8, b), c, 0, 0, 0);
 }
 
-// N 32-expert tiles (E = 32 N), TOK tokens per block.
-template <int N, int TOK>
+// Tokens per block, and the block's shape for N 32-expert tiles (E = 32 N).
+constexpr int kGateTok = 64;
+template <int N>
 struct GateShape {
   static constexpr int E = 32 * N;                              // experts
   static constexpr int NT = N;                                  // 32-expert tiles
-  static constexpr int MT = TOK / 32;                           // 32-token tiles
+  static constexpr int MT = kGateTok / 32;                      // 32-token tiles
   static constexpr int WAVES = 16;                              // waves per block
   static constexpr int TPW = (MT * NT + WAVES - 1) / WAVES;     // 32x32 output tiles per wave
-  static constexpr int NI = (TOK + E) / 8;                      // DMA loads per chunk (8 rows)
+  static constexpr int NI = (kGateTok + E) / 8;                 // DMA loads per chunk (8 rows)
   static constexpr int PW = (NI + WAVES - 1) / WAVES;           // ... per wave (rest: dummy)
-  static constexpr int SB = (TOK + E) * kGateRow;               // stage bytes
+  static constexpr int SB = (kGateTok + E) * kGateRow;          // stage bytes
   static constexpr int NS = 4 * SB + 1024 <= 128 * 1024 ? 4 : 3;  // stages in the ring
   static constexpr int LS = E + 4;                              // logits tile row stride (floats)
   static constexpr int EPL = E <= 64 ? 1 : (E <= 128 ? 2 : 4);
   static constexpr int RING = NS * SB + 1024;                   // + a dummy DMA target
-  static constexpr int LDS = RING > TOK * LS * 4 ? RING : TOK * LS * 4;
+  static constexpr int LDS = RING > kGateTok * LS * 4 ? RING : kGateTok * LS * 4;
 };
 
 // 16 waves: the GEMM gives each wave one or two 32x32 (token, expert) tiles;
-// the selection then routes TOK / 16 tokens per wave.
-template <int ET, int N, int TOK>
+// the selection then routes kGateTok / 16 tokens per wave.
+template <int ET, int N>
 __global__ __launch_bounds__(1024) void router_gate_fwd_kernel(
     const char* __restrict__ x, const char* __restrict__ w, int64_t T, int H, int ldt, int K,
     int score_fn, int pre_softmax, const float* __restrict__ bias, int G, int GK, float scaling,
     const int64_t* __restrict__ fixed, void* __restrict__ logits, void* __restrict__ probs,
     uint8_t* __restrict__ rmap, int64_t* __restrict__ top_idx) {
-  typedef GateShape<N, TOK> S;
+  typedef GateShape<N> S;
   constexpr int E = S::E, NS = S::NS, SB = S::SB, EPL = S::EPL, PW = S::PW, MT = S::MT;
   extern __shared__ __align__(16) char gsm[];
   glds_char* const lds = (glds_char*)gsm;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t t0 = (int64_t)blockIdx.x * TOK;
+  const int64_t t0 = (int64_t)blockIdx.x * kGateTok;
   const int nch = H / 64;
-  const int64_t nrow = T - t0 < TOK ? T - t0 : TOK;
+  const int64_t nrow = T - t0 < kGateTok ? T - t0 : kGateTok;
   const gi32x4 rx = rg_rsrc(x + t0 * H * 2, nrow * H * 2);
   const gi32x4 rw = rg_rsrc(w, (int64_t)E * H * 2);
 
@@ -1278,10 +1279,10 @@ __global__ __launch_bounds__(1024) void router_gate_fwd_kernel(
     for (int q = 0; q < PW; ++q) {
       const int g = wave * PW + q;
       const bool real = g < S::NI;
-      const bool isx = 8 * g < TOK;
+      const bool isx = 8 * g < kGateTok;
       const int r = 8 * g + (lane >> 3);
       const int c = (lane & 7) ^ ((r >> 1) & 7);
-      const int orow = isx ? r : r - TOK;
+      const int orow = isx ? r : r - kGateTok;
       const uint32_t off = (uint32_t)(((int64_t)orow * H + (int64_t)kc * 64 + c * 8) * 2);
       const bool live = real && kc < nch;
       gi32x4 rs;
@@ -1318,7 +1319,7 @@ __global__ __launch_bounds__(1024) void router_gate_fwd_kernel(
                                                         st + rg_swz(32 * (tile % MT) + (lane & 31), c)));
           const uint4 b = __builtin_bit_cast(
               uint4, *reinterpret_cast<const glds_u32x4*>(
-                         st + rg_swz(TOK + 32 * (tile / MT) + (lane & 31), c)));
+                         st + rg_swz(kGateTok + 32 * (tile / MT) + (lane & 31), c)));
           acc[i] = rg_mma<ET>(b, a, acc[i]);
         }
       }
@@ -1347,11 +1348,11 @@ __global__ __launch_bounds__(1024) void router_gate_fwd_kernel(
     }
   }
   __syncthreads();
-  for (int idx = tid; idx < TOK * E; idx += 64 * S::WAVES) {
+  for (int idx = tid; idx < kGateTok * E; idx += 64 * S::WAVES) {
     const int row = idx / E, col = idx % E;
     if (row < nrow) store_from_f32(logits, ldt, (t0 + row) * E + col, L[row * S::LS + col]);
   }
-  constexpr int RPW = TOK / S::WAVES;  // tokens routed per wave
+  constexpr int RPW = kGateTok / S::WAVES;  // tokens routed per wave
   for (int rr = 0; rr < RPW; ++rr) {
     const int row = wave * RPW + rr;
     if (row >= nrow) break;  // wave-uniform; no block synchronisation follows
@@ -1368,16 +1369,16 @@ __global__ __launch_bounds__(1024) void router_gate_fwd_kernel(
   }
 }
 
-template <int ET, int N, int TOK>
-int launch_gate_t(const void* x, const void* w, int64_t T, int H, int ldt, int K, int sf, int pre,
-                  const float* bias, int G, int GK, float scale, const int64_t* fixed,
-                  void* logits, void* probs, uint8_t* rmap, int64_t* top, hipStream_t s) {
-  typedef GateShape<N, TOK> S;
+template <int ET, int N>
+int launch_gate(const void* x, const void* w, int64_t T, int H, int ldt, int K, int sf, int pre,
+                const float* bias, int G, int GK, float scale, const int64_t* fixed, void* logits,
+                void* probs, uint8_t* rmap, int64_t* top, hipStream_t s) {
+  typedef GateShape<N> S;
   static_assert(S::LDS <= 160 * 1024, "gate tile exceeds LDS");
   static bool allowed = false;  // the attribute belongs to the kernel, for every device
   if (!allowed) {
     const hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&router_gate_fwd_kernel<ET, N, TOK>),
+        reinterpret_cast<const void*>(&router_gate_fwd_kernel<ET, N>),
         hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
     if (e != hipSuccess) {
       (void)hipGetLastError();
@@ -1387,8 +1388,8 @@ int launch_gate_t(const void* x, const void* w, int64_t T, int H, int ldt, int K
     }
     allowed = true;
   }
-  const dim3 grid((unsigned)((T + TOK - 1) / TOK));
-  hipLaunchKernelGGL((router_gate_fwd_kernel<ET, N, TOK>), grid, dim3(64 * S::WAVES), S::LDS, s,
+  const dim3 grid((unsigned)((T + kGateTok - 1) / kGateTok));
+  hipLaunchKernelGGL((router_gate_fwd_kernel<ET, N>), grid, dim3(64 * S::WAVES), S::LDS, s,
                      static_cast<const char*>(x), static_cast<const char*>(w), T, H, ldt, K, sf,
                      pre, bias, G, GK, scale, fixed, logits, probs, rmap, top);
   return tt_check_launch("router_gate_fwd");
@@ -1651,10 +1652,9 @@ extern "C" int tt_router_loss_fwd(const void* logits, int logits_dtype, int64_t 
 }
 
 static int loss_bwd_run(const void* logits, int logits_dtype, int64_t num_tokens,
-                                  int32_t num_experts, int32_t score_function,
-                                  const uint8_t* padding_mask, const float* grad_prob_sum,
-                                  const float* grad_z_sum, const int64_t* loads, const float* scal,
-                        void* grad_logits, void* stream) {
+                        int32_t num_experts, int32_t score_function, const uint8_t* padding_mask,
+                        const float* grad_prob_sum, const float* grad_z_sum, const int64_t* loads,
+                        const float* scal, void* grad_logits, void* stream) {
   TT_REQUIRE(logits_dtype_ok(logits_dtype), "router_loss_bwd: unsupported logits dtype %d",
              logits_dtype);
   TT_REQUIRE(num_tokens >= 0, "router_loss_bwd: negative token count");
@@ -1668,7 +1668,7 @@ static int loss_bwd_run(const void* logits, int logits_dtype, int64_t num_tokens
   case N:                                                                                        \
     hipLaunchKernelGGL(router_loss_bwd_kernel<N>, grid, dim3(256), 0, S(stream), logits,         \
                        logits_dtype, num_tokens, num_experts, score_function, padding_mask,      \
-                       grad_prob_sum, grad_z_sum, loads, scal, grad_logits);                                \
+                       grad_prob_sum, grad_z_sum, loads, scal, grad_logits);                     \
     break;
     TT_CASE(1) TT_CASE(2) TT_CASE(4) TT_CASE(8) TT_CASE(16)
 #undef TT_CASE
@@ -1779,10 +1779,10 @@ extern "C" int tt_router_gate_fwd(const void* x, const void* weight, int in_dtyp
   }
 #define TT_GATE_N(ET, NN)                                                                       \
   case NN:                                                                                     \
-    return launch_gate_t<ET, NN, 64>(x, weight, num_tokens, H, logits_dtype, topk,             \
-                                     score_function, pre_softmax, expert_bias, num_groups, gk, \
-                                     scaling_factor, fixed_indices, logits, probs,             \
-                                     routing_map, top_indices, S(stream));
+    return launch_gate<ET, NN>(x, weight, num_tokens, H, logits_dtype, topk, score_function,   \
+                               pre_softmax, expert_bias, num_groups, gk, scaling_factor,       \
+                               fixed_indices, logits, probs, routing_map, top_indices,         \
+                               S(stream));
 #define TT_GATE(ET)                                                                            \
   switch (NE) {                                                                                \
     TT_GATE_N(ET, 1) TT_GATE_N(ET, 2) TT_GATE_N(ET, 3) TT_GATE_N(ET, 4)                        \
