@@ -1436,8 +1436,8 @@ def test_grouped_matmul_few_rows_exact(counts, K, N, dtype, trans_b):
 
 # (experts, columns of the output, limit of the few-row kernel): one launch in each class of
 # its rule, by the number of 256-wide column tiles.
-THIN_LIMITS = [(100, 256, 96), (100, 512, 60), (100, 768, 96), (100, 2048, 96), (25, 8192, 40),
-               (130, 2056, 40)]
+THIN_LIMITS = [(100, 256, 96), (100, 512, 96), (32, 2048, 60), (100, 768, 96), (100, 2048, 96),
+               (25, 8192, 40), (130, 2056, 40)]
 
 
 @pytest.mark.parametrize("E,J,limit", THIN_LIMITS, ids=[f"E{c[0]}J{c[1]}" for c in THIN_LIMITS])

@@ -29,6 +29,7 @@ struct BF { static constexpr int code = TT_BF16; };
 struct HF { static constexpr int code = TT_F16; };
 
 constexpr int LR_NT = 256;
+constexpr int64_t LD_BLOCKS = 400;  // see launch_down
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((address_space(3))) float lds_float;
 
@@ -96,22 +97,23 @@ __device__ __forceinline__ float widen1(uint32_t w, bool odd, float s) {
 // ---------------------------------------------------------------------------
 // out[m, j] (fp32 [M, r]) = sum over c of in[m, c] W_e(c, j), in [M, C] 16-bit.
 // W_e: [C, r] (forward), or [r, C] (WT, the backward's B) with in scaled by s
-// and rounded first (SCALE). A block takes 64 rows and every column, wave w
-// rows 16 w .. + 15 over the whole reduction; 64-deep k-tiles of in and W_e
-// stream into a ring of S LDS stages (48 KiB, three blocks per CU), one barrier
-// per k-tile, as in gmm_thin_kernel. LDS of a stage: in 128 bytes per row, chunk c of row r in
+// and rounded first (SCALE). A block takes BM rows and every column, a wave 16
+// rows and the columns of 1 / WC of the 16-wide tiles over the whole reduction;
+// 64-deep k-tiles of in and W_e stream into a ring of S LDS stages (about 48
+// KiB, three blocks per CU), one barrier per k-tile, as in gmm_thin_kernel. LDS of a stage: in 128 bytes per row, chunk c of row r in
 // slot c ^ ((r >> 1) & 7); then W_e's 64 x r elements as they lie in memory,
 // or (WT) 256 bytes per row j, chunk c in slot c ^ (j % 16).
 // ---------------------------------------------------------------------------
-template <class TT, int RT, bool WT, bool SCALE>
+template <class TT, int RT, bool WT, bool SCALE, int WC>
 __global__ __launch_bounds__(LR_NT) void lora_down_kernel(const uint16_t* __restrict__ in,
                                                           const float* __restrict__ W,
                                                           float* __restrict__ out, int C, int r,
                                                           float s, int E,
                                                           const int64_t* __restrict__ counts) {
-  constexpr int BM = 64, BK = 64, S = RT == 1 ? 4 : RT == 2 ? 3 : 2;
+  constexpr int BM = 64 / WC, BK = 64, S = RT == 1 ? 4 : RT == 2 ? 3 : 2;
   constexpr int T_X = BM * BK * 2, T_W = 16 * RT * BK * 4, STAGE = T_X + T_W;
-  constexpr int LD = 2 + RT;  // loads per wave and k-tile
+  constexpr int LX = BM / 32, LD = LX + RT;  // loads per wave and k-tile
+  constexpr int CT = RT / WC;                // column tiles per wave
   __shared__ __align__(16) char lds_raw[S * STAGE];
   RowTile t;
   if (!row_tile<BM, LR_NT>(counts, E, 1, lds_raw, t)) return;
@@ -123,11 +125,11 @@ __global__ __launch_bounds__(LR_NT) void lora_down_kernel(const uint16_t* __rest
   const int nkt = (C + BK - 1) / BK;
   const i32x4 rx = make_rsrc(in + row0 * C, (int64_t)rows * C * 2);
   const i32x4 rw = make_rsrc(W + (int64_t)t.e * C * r, (int64_t)C * r * 4);
-  uint32_t xoff[2], woff[RT];
-  int xk[2], wk[RT];
+  uint32_t xoff[LX], woff[RT];
+  int xk[LX], wk[RT];
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int m = 16 * wave + 8 * q + (lane >> 3), c = (lane & 7) ^ ((m >> 1) & 7);
+  for (int q = 0; q < LX; ++q) {
+    const int m = 8 * (LX * wave + q) + (lane >> 3), c = (lane & 7) ^ ((m >> 1) & 7);
     xk[q] = 8 * c;
     xoff[q] = (uint32_t)(((int64_t)m * C + 8 * c) * 2);
   }
@@ -149,16 +151,17 @@ __global__ __launch_bounds__(LR_NT) void lora_down_kernel(const uint16_t* __rest
     const i32x4 ax = advance_rsrc(rx, (uint32_t)kt * (BK * 2));
     const i32x4 aw = advance_rsrc(rw, (uint32_t)kt * (uint32_t)(BK * 4 * (WT ? 1 : r)));
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-      dma16(kt * BK + xk[q] < C ? xoff[q] : DM_OOB, ax, base + (uint32_t)(2 * wave + q) * 1024u);
+    for (int q = 0; q < LX; ++q)
+      dma16(kt * BK + xk[q] < C ? xoff[q] : DM_OOB, ax, base + (uint32_t)(LX * wave + q) * 1024u);
 #pragma unroll
     for (int q = 0; q < RT; ++q)
       dma16(WT && kt * BK + wk[q] >= C ? DM_OOB : woff[q], aw,
             base + T_X + (uint32_t)(RT * wave + q) * 1024u);
   };
   const bool odd = g >> 1;
-  const int row = 16 * wave + l16;
-  f32x4 acc[RT] = {};
+  const int wr = wave / WC, wc = wave % WC;  // the wave's rows and columns
+  const int row = 16 * wr + l16;
+  f32x4 acc[CT] = {};
 #pragma unroll
   for (int i = 0; i < S - 1; ++i)
     if (i < nkt) issue(i, i);
@@ -175,21 +178,21 @@ __global__ __launch_bounds__(LR_NT) void lora_down_kernel(const uint16_t* __rest
     const lds_float* const wl = reinterpret_cast<const lds_float*>(stg + T_X);
     // The fragments of 16 elements are read while the 16 before are multiplied.
     uint4 xv[2];
-    float wv[2][4][RT];
+    float wv[2][4][CT];
     auto read = [&](int b) {
       xv[b & 1] = read_k(
           stg, (uint32_t)(row * 128 + (((2 * b + (g & 1)) ^ ((row >> 1) & 7)) << 4)));
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int jt = 0; jt < RT; ++jt) {
+        for (int jt = 0; jt < CT; ++jt) {
           const int c = 16 * b + 8 * (g & 1) + 2 * q + (g >> 1);
-          const int j = 16 * jt + l16;  // results of j >= r are not stored
+          const int j = 16 * (CT * wc + jt) + l16;  // results of j >= r are not stored
           wv[b & 1][q][jt] = WT ? wl[j * 64 + (((c >> 2) ^ (j & 15)) << 2) + (c & 3)]
                                 : wl[c * r + (j < r ? j : 0)];
         }
     };
-    if (16 * wave < rows) {
+    if (16 * wr < rows) {
       read(0);
 #pragma unroll
       for (int b = 0; b < BK / 16; ++b) {
@@ -200,19 +203,19 @@ __global__ __launch_bounds__(LR_NT) void lora_down_kernel(const uint16_t* __rest
         for (int q = 0; q < 4; ++q) {
           const float a = widen1<TT, SCALE>(x[q], odd, s);
 #pragma unroll
-          for (int jt = 0; jt < RT; ++jt) acc[jt] = mfma16(a, wv[b & 1][q][jt], acc[jt]);
+          for (int jt = 0; jt < CT; ++jt) acc[jt] = mfma16(a, wv[b & 1][q][jt], acc[jt]);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     slot = slot == S - 1 ? 0 : slot + 1;
   }
-  // Lane l holds rows 16 wave + 4 (l / 16) + 0..3, column 16 jt + l % 16.
+  // Lane l holds rows 16 wr + 4 (l / 16) + 0..3, column 16 (CT wc + jt) + l % 16.
 #pragma unroll
-  for (int jt = 0; jt < RT; ++jt)
+  for (int jt = 0; jt < CT; ++jt)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int m = 16 * wave + 4 * g + e, j = 16 * jt + l16;
+      const int m = 16 * wr + 4 * g + e, j = 16 * (CT * wc + jt) + l16;
       if (m < rows && j < r) out[(row0 + m) * r + j] = acc[jt][e];
     }
 }
@@ -452,14 +455,30 @@ struct LoraArgs {
   const int64_t* counts;
 };
 
-int64_t row_blocks(int64_t M, int E) { return M / 64 + (M < E ? M : E); }
+int64_t row_blocks(int64_t M, int E, int bm = 64) { return M / bm + (M < E ? M : E); }
 
+template <class TT, int RT, bool WT, bool SCALE, int WC>
+int launch_down_wc(const LoraArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((lora_down_kernel<TT, RT, WT, SCALE, WC>),
+                     dim3((unsigned)row_blocks(a.M, a.E, 64 / WC)), dim3(LR_NT), 0, s, a.in, a.w,
+                     static_cast<float*>(a.out), a.C, a.r, a.s, a.E, a.counts);
+  return tt_check_launch("lora_down");
+}
+// Ranks above 32 in blocks of 32 rows, two waves to the columns, ranks above 16
+// while 64-row blocks make at most LD_BLOCKS. 64- / 32-row blocks, 2432 columns,
+// forward and transposed: r 64, 32 experts of 55 rows 70.9 + 80.2 / 42.2 + 49.3 us,
+// 128 of 130 108.6 + 119.5 / 85.4 + 97.9, of 256 149.4 + 162.8 / 136.9 + 155.0; r
+// 32, 32 of 55 43.9 + 47.3 / 29.2 + 34.3, 128 of 130 (388 blocks) 65.4 + 70.4 /
+// 52.1 + 65.1, of 200 (528) 65.6 + 71.0 / 65.7 + 80.6.
 template <class TT, int RT, bool WT, bool SCALE>
 int launch_down(const LoraArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((lora_down_kernel<TT, RT, WT, SCALE>), dim3((unsigned)row_blocks(a.M, a.E)),
-                     dim3(LR_NT), 0, s, a.in, a.w, static_cast<float*>(a.out), a.C, a.r, a.s, a.E,
-                     a.counts);
-  return tt_check_launch("lora_down");
+  if constexpr (RT == 4) {
+    return launch_down_wc<TT, RT, WT, SCALE, 2>(a, s);
+  } else {
+    if constexpr (RT == 2)
+      if (row_blocks(a.M, a.E) <= LD_BLOCKS) return launch_down_wc<TT, RT, WT, SCALE, 2>(a, s);
+    return launch_down_wc<TT, RT, WT, SCALE, 1>(a, s);
+  }
 }
 template <class TT, int RT, bool WT, bool BASE>
 int launch_up(const LoraArgs& a, const float* h, hipStream_t s) {
