@@ -110,9 +110,9 @@ class MoELayer(BaseMoELayer):
         """The experts' output for a small batch without gradients, in one native call where
         the HIP providers serve the ops it stands for (the conditions are in
         ``providers.hip.fused_experts.inference_eligible``); None otherwise."""
-        tokens = hidden_states.view(-1, hidden_states.shape[-1])
-        if torch.is_grad_enabled() or not tokens.is_cuda:
+        if torch.is_grad_enabled() or not hidden_states.is_cuda:
             return None
+        tokens = hidden_states.view(-1, hidden_states.shape[-1])
         e = self.experts
         fp8 = type(e) is Fp8GroupedMLP
         if not fp8 and type(e) is not GroupedMLP:

@@ -52,16 +52,17 @@ class MoEAuxLossAutoScaler(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, output, aux_loss):
-        ctx.save_for_backward(aux_loss)
+        # Not saved as a tensor: only its form is needed, and a metric that shares its memory
+        # may be changed in place before the backward.
+        ctx.form = dict(size=aux_loss.shape, dtype=aux_loss.dtype, device=aux_loss.device)
         return output
 
     @staticmethod
     def backward(ctx, grad_output):
-        (aux_loss,) = ctx.saved_tensors
         scale = MoEAuxLossAutoScaler.loss_scale
         if isinstance(scale, (int, float)):
-            return grad_output, torch.full_like(aux_loss, scale)
-        return grad_output, torch.ones_like(aux_loss) * scale
+            return grad_output, torch.full(fill_value=scale, **ctx.form)
+        return grad_output, torch.ones(**ctx.form) * scale
 
     @classmethod
     def set_loss_scale(cls, scale: float) -> None:

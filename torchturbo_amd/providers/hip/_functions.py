@@ -269,10 +269,10 @@ class RouterLosses(torch.autograd.Function):
         ctx.save_for_backward(logits, counts, losses)
         ctx.sf = sf
         ctx.set_materialize_grads(False)
-        # Tensors with version counters of their own, not views of what is saved here: a metric
-        # changed in place (an all-reduce of it) leaves the backward valid. The backward reads
-        # the factors behind the four.
-        aux, aux_raw, z, z_raw = (v.view(()) for v in losses.unsafe_split(1)[:4])
+        # Views with a version counter of their own (``data``): metrics changed in place (an
+        # all-reduce of them) leave what is saved here valid, of which the backward reads the
+        # factors behind the four.
+        aux, aux_raw, z, z_raw = losses.data[:4].unbind()
         ctx.mark_non_differentiable(aux_raw, z_raw)
         return aux, z, aux_raw, z_raw
 

@@ -248,18 +248,20 @@ def _sizes_agree(experts, weights, scales, tokens, probs, num_experts, ffn) -> b
     or from the config: it gets addresses and cannot check. The separate ops refuse the rest,
     or serve it from the weights' own widths."""
     T, H = tokens.shape
-    E, cfg = num_experts, experts.config
-    if not ffn or experts.num_local_experts != E or cfg.hidden_size != H:
+    E = num_experts
+    if not ffn or experts.num_local_experts != E or experts.config.hidden_size != H:
         return False
-    if tuple(probs.shape) != (T, E):
+    if probs.shape != (T, E):
         return False
+    w1, w2 = weights
     if scales is None:
-        return [tuple(w.shape) for w in weights] == [(E * H, 2 * ffn), (E * ffn, H)]
-    want = [(E, 2 * ffn, H), (E, H, ffn)]
-    blocks = [(E, -(-n // 128), -(-k // 128)) for _, n, k in want]
-    masters = (experts.master1, experts.master2)
-    return ([tuple(w.shape) for w in weights] == want and [tuple(s.shape) for s in scales] == blocks
-            and all(m is None or tuple(m.shape) == n for m, n in zip(masters, want)))
+        return w1.shape == (E * H, 2 * ffn) and w2.shape == (E * ffn, H)
+    for w, s, m, N, K in ((w1, scales[0], experts.master1, 2 * ffn, H),
+                          (w2, scales[1], experts.master2, H, ffn)):
+        if (w.shape != (E, N, K) or s.shape != (E, -(-N // 128), -(-K // 128))
+                or m is not None and m.shape != (E, N, K)):
+            return False
+    return True
 
 
 def inference_eligible(experts, weights, scales, tokens, probs, expert_indices, num_experts,
