@@ -40,7 +40,8 @@ __global__ __launch_bounds__(GL_NT) void gate_logits_kernel(const char* __restri
     const int g = LD * wave + q;
     const int r = 8 * g + (lane >> 3);
     isx[q] = 8 * g < 32 * MT;
-    off[q] = (uint32_t)(((isx[q] ? r : r - 32 * MT) * (int64_t)H + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2);
+    off[q] = (uint32_t)(((isx[q] ? r : r - 32 * MT) * (int64_t)H +
+                         8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2);
   }
   lds_char* const lds = (lds_char*)lds_raw;
   const uint32_t lds0 = lds_addr_of(lds);

@@ -9,9 +9,10 @@
 // is lost, the spacing of the smallest bf16 results), so g is split into three
 // bf16 planes and both products run on bf16 matrix instructions with fp32
 // accumulation: the same products, exact, in three times the operations at
-// sixteen times the rate, and no larger error against float64. Both gradients, composition / here: T 4096, H 7168, E 256 344 / 110
-// us (split 6, dx 50, dw 48, the sum of its parts 5), 1024, 7168, 64 64 /
-// 31, 16384, 2048, 128 277 / 85, 128, 1024, 64 24 / 17.
+// sixteen times the rate, and no larger error against float64. Both gradients,
+// composition / here: T 4096, H 7168, E 256 344 / 110 us (split 6, dx 50, dw 48,
+// the sum of its parts 5), 1024, 7168, 64 64 / 31, 16384, 2048, 128 277 / 85,
+// 128, 1024, 64 24 / 17.
 #include "gemm.h"
 
 namespace {

@@ -2616,25 +2616,26 @@ int launch_p64_k(const void* p0, const void* p1, void* out, int64_t M, int64_t K
 
 // fwd / dgrad (J columns) with at most this many rows per expert on average run
 // on the kernel of gmm_thin.hip (its loads run up to a k-tile past the reduction
-// end, in 32-bit offsets). The line depends on how many 256-wide column tiles
-// the launch has: up to 192 of them leave CUs of the persistent kernel idle,
-// about 256 give each CU one (which few experts over many columns fill well when
-// loads are skewed), more need a second round; above 1024, and for few experts
-// over many columns, the persistent kernel's rounds are full. Loads even
-// and skewed as a router with a Zipf(0.8) / Zipf(1.1) prior makes them,
-// persistent / thin in us: 8 experts of 512 x 1024 fwd (32 tiles) at 80 rows 12 +
-// 16 + 17 / 8 + 9 + 9; 16 of 1536 x 4096 fwd (256) at 48 rows 59 + 48 + 49 / 35 +
-// 45 + 45, at 66 43 + 51 + 51 / 35 + 57 + 55; 64 of 704 x 1024 fwd (256) at 66 27
-// + 29 + 30 / 19 + 25 + 26; 128 of 2048 x 1536 fwd (768) at 32 rows 169 + 152 + 138 / 147 + 145 + 122, at 48 173 + 152 + 133 / 157 + 161 +
-// 133, at 66 192 + 193 + 139 / 162 + 170 + 156, at 96 173 + 191 + 180 / 165 + 194
-// + 182, at 128 (even) 188 / 218; its 768 x 2048 fwd (1024) at 66 106 + 91 + 85 /
-// 89 + 98 + 84, dgrad (384) 135 / 108 (even, 62); 128 of 512 x 4096 fwd (2048) at
-// 32 109 + 111 + 88 / 107 + 103 + 87, at 80 134 + 133 + 119 / 134 + 145 + 131; 32
-// of 2048 x 5632 fwd (704, 22 per expert) at 48 153 + 149 + 143 / 140 + 146 +
-// 142, at 66 180 + 144 + 142 / 154 + 170 + 162. Over 26 layers, 14 row counts and
-// these loads the launches take 0.74 of the persistent kernel's time on average;
-// 3 % of them are slower by more than 5 % (at most 1.3). Over 130 random layers
-// at 30 to 97 rows 0.76, and 5 % of them.
+// end, in 32-bit offsets). The line depends on how many 256-wide column tiles the
+// launch has: up to 192 of them leave CUs of the persistent kernel idle, about
+// 256 give each CU one (which few experts over many columns fill well when loads
+// are skewed), more need a second round; above 1024, and for few experts over
+// many columns, the persistent kernel's rounds are full. Loads even and skewed as
+// a router with a Zipf(0.8) / Zipf(1.1) prior makes them, persistent / thin in
+// us: 8 experts of 512 x 1024 fwd (32 tiles) at 80 rows 12 + 16 + 17 / 8 + 9 + 9;
+// 16 of 1536 x 4096 fwd (256) at 48 rows 59 + 48 + 49 / 35 + 45 + 45, at 66 43 +
+// 51 + 51 / 35 + 57 + 55; 64 of 704 x 1024 fwd (256) at 66 27 + 29 + 30 / 19 + 25
+// + 26; 128 of 2048 x 1536 fwd (768) at 32 rows 169 + 152 + 138 / 147 + 145 +
+// 122, at 48 173 + 152 + 133 / 157 + 161 + 133, at 66 192 + 193 + 139 / 162 + 170
+// + 156, at 96 173 + 191 + 180 / 165 + 194 + 182, at 128 (even) 188 / 218; its
+// 768 x 2048 fwd (1024) at 66 106 + 91 + 85 / 89 + 98 + 84, dgrad (384) 135 / 108
+// (even, 62); 128 of 512 x 4096 fwd (2048) at 32 109 + 111 + 88 / 107 + 103 + 87,
+// at 80 134 + 133 + 119 / 134 + 145 + 131; 32 of 2048 x 5632 fwd (704, 22 per
+// expert) at 48 153 + 149 + 143 / 140 + 146 + 142, at 66 180 + 144 + 142 / 154 +
+// 170 + 162. Over 26 layers, 14 row counts and these loads the launches take 0.74
+// of the persistent kernel's time on average; 3 % of them are slower by more than
+// 5 % (at most 1.3). Over 130 random layers at 30 to 97 rows 0.76, and 5 % of
+// them.
 int64_t thin_row_limit(int64_t E, int64_t J) {
   const int64_t tiles = E * ((J + DM_BN - 1) / DM_BN);
   if (tiles <= 192) return 96;
