@@ -52,17 +52,17 @@ class MoEAuxLossAutoScaler(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, output, aux_loss):
-        # Not saved as a tensor: only its form is needed, and a metric that shares its memory
-        # may be changed in place before the backward.
-        ctx.form = dict(size=aux_loss.shape, dtype=aux_loss.dtype, device=aux_loss.device)
+        # Not saved for the backward, which needs its form and not its value: a metric that
+        # shares its memory may be changed in place in between.
+        ctx.like = aux_loss.detach()
         return output
 
     @staticmethod
     def backward(ctx, grad_output):
         scale = MoEAuxLossAutoScaler.loss_scale
         if isinstance(scale, (int, float)):
-            return grad_output, torch.full(fill_value=scale, **ctx.form)
-        return grad_output, torch.ones(**ctx.form) * scale
+            return grad_output, torch.full_like(ctx.like, scale)
+        return grad_output, torch.ones_like(ctx.like) * scale
 
     @classmethod
     def set_loss_scale(cls, scale: float) -> None:
